@@ -13,6 +13,11 @@ HIPCC_FLAGS = [
     # packed FP32 (v_pk_*_f32) stays off for every HIP translation unit
     '-Xclang', '-target-feature', '-Xclang', '-packed-fp32-ops',
     '-Wno-unused-result',
+    # branches that are uniform over a wave stay scalar branches instead of
+    # being structurised: without it every path of the tile kernels' member
+    # dispatch ends in vector register copies (a stage member's 12-30, the
+    # whole tile in a register-resident one)
+    '-mllvm', '-structurizecfg-skip-uniform-regions',
     # no FMA contraction in host code: the planner's scores and the host MLP
     # forward round the same way wherever they are evaluated
     '-ffp-contract=off',
