@@ -1294,6 +1294,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(sizeof(T) ==
   }
 }
 
+#include "tile_reg.h"
+
 // ---------------------------------------------------------------------------
 // K6: reductions (FP64 accumulation).
 // ---------------------------------------------------------------------------
@@ -1845,6 +1847,18 @@ struct FusedPass {
   TileGeom geo;
   std::vector<TileOp> ops;     // param offsets relative to this pass's values
   std::vector<double> vals;    // values in kernel layout (FP64; converted at upload)
+  bool reg = false;            // register-resident form (reg_geo, recs) instead of geo and ops
+  RegGeom reg_geo;
+  int reg_stages = 0;
+  std::vector<uint32_t> recs;  // its device records: the stages, then the members' kinds
+  // device records as 32-bit words
+  size_t rec_words() const { return reg ? recs.size() : ops.size() * (sizeof(TileOp) / 4); }
+  void put_recs(std::vector<uint32_t> *out) const {
+    const size_t at = out->size();
+    out->resize(at + rec_words());
+    if (rec_words())
+      memcpy(out->data() + at, reg ? (const void *)recs.data() : (const void *)ops.data(), rec_words() * 4);
+  }
 };
 
 struct dm_state {
@@ -2590,7 +2604,75 @@ void group_stages(FusedPass *fp) {
   fp->ops.swap(out);
 }
 
-int parse_fused(const dm_state *h, const double *p, int64_t avail, int opi, FusedPass *fp) {
+// The register-resident form (k_tile_reg) of a parsed pass, its tile
+// completed to 7 digits with the lowest other positions, where that is the
+// faster one; false leaves the pass as it is.  It takes single-qubit and CX
+// operations in a tile that holds the positions 0-2 (64 consecutive
+// coefficients per access).  The grid is one workgroup of 256 threads per
+// tile, so 18 qubits are the most that fit the 2^32 work items of a launch.
+// From 12 qubits on it is faster for any pass (16 qubits, one / 8 / 16 pairs
+// of a single-qubit map and a CX on three digits: FP32 6.0 / 6.5 / 7.1 ms
+// against 6.7 / 7.7 / 14.3 with the tile in LDS, FP64 12.0 / 12.6 / 16.4
+// against 13.1 / 15.5 / 24.8).  Below, a launch is a few workgroups per CU
+// and its latency counts: the tile-in-LDS kernel's 6-digit tiles fill more
+// CUs, and only passes with many operations per redistribution gain (9
+// qubits, FP64: one pair 9.5 against 6.2 us, 8 pairs 18.8 against 20.3).
+bool plan_reg(const dm_state *h, FusedPass *fp) {
+  if (h->n < kRegTile || h->n > 18) return false;
+  if (h->n < 12 && fp->ops.size() < 12) return false;
+  for (const TileOp &op : fp->ops)
+    if (op.kind != TOP_1Q && op.kind != TOP_CX) return false;
+  bool in[kMaxQubits] = {false};
+  for (int j = 0; j < fp->m; ++j) in[fp->geo.tpos[j]] = true;
+  int count = fp->m;
+  for (int pos = 0; pos < h->n && count < kRegTile; ++pos)
+    if (!in[pos]) {
+      in[pos] = true;
+      ++count;
+    }
+  if (!in[0] || !in[1] || !in[2]) return false;
+  int tpos[kRegTile], rpos[kMaxQubits], digit[kMaxQubits], nt = 0, nr = 0;
+  for (int pos = 0; pos < h->n; ++pos) {
+    if (in[pos]) {
+      digit[pos] = nt;
+      tpos[nt++] = pos;
+    } else {
+      rpos[nr++] = pos;
+    }
+  }
+  // FP32 keeps the order of operations of the tile-in-LDS form, and with it
+  // every rounding: a state does not depend on which form ran.  FP64 may
+  // reorder what commutes (differences of 1e-15).
+  const bool ordered = h->dtype == DM_FP32;
+  std::vector<TileOp> ops;
+  std::vector<double> vals;
+  if (ordered) {
+    FusedPass staged;
+    staged.ops = fp->ops;
+    staged.vals = fp->vals;
+    group_stages(&staged);
+    for (const TileOp &op : staged.ops)
+      if (op.kind != TOP_STAGE) ops.push_back(op);
+    vals = std::move(staged.vals);
+  } else {
+    ops = fp->ops;
+    vals = fp->vals;
+  }
+  for (TileOp &op : ops)
+    for (int x = 0; x < (op.kind == TOP_CX ? 2 : 1); ++x) op.d[x] = digit[fp->geo.tpos[op.d[x]]];
+  RegPlan rp;
+  reg_plan(ops, vals, tpos, rpos, nr, ordered, &rp);
+  if (h->n < 12 && ops.size() < 4 * (size_t)rp.ns) return false;
+  fp->reg = true;
+  fp->reg_geo = rp.geo;
+  fp->reg_stages = rp.ns;
+  fp->recs = std::move(rp.words);
+  fp->vals = std::move(rp.vals);
+  fp->ops.clear();
+  return true;
+}
+
+int parse_fused(const dm_state *h, const double *p, int64_t avail, int opi, FusedPass *fp, bool allow_reg = false) {
   int64_t at = 0;
   auto next = [&](double *out) -> bool {
     if (at >= avail) return false;
@@ -2686,6 +2768,7 @@ int parse_fused(const dm_state *h, const double *p, int64_t avail, int opi, Fuse
     at += nv;
     fp->ops.push_back(op);
   }
+  if (allow_reg && plan_reg(h, fp)) return DM_OK;
   // LDS layout.  The 64 banks (4 bytes each) are LDS index bits 0-5, tile
   // digits 0-2.  Stages on digits 3 and up, and stages on digit 0 and a
   // digit >= 3 (one quad access per component), fall on distinct banks in
@@ -2797,8 +2880,25 @@ int stage_io_flags(const FusedPass &fp, int *last) {
 }
 
 template <typename T>
-int launch_fused(dm_state *h, const FusedPass &fp, const TileOp *d_ops, const T *d_vals) {
+int launch_fused(dm_state *h, const FusedPass &fp, const uint32_t *d_recs, const T *d_vals) {
   ProfScope ps(h, 9);
+  if (fp.reg) {
+    const RegStage *st = reinterpret_cast<const RegStage *>(d_recs);
+    const uint32_t *mem = reinterpret_cast<const uint32_t *>(st + fp.reg_stages);
+    // states above the 256 MB of the last-level cache stream with
+    // nontemporal accesses (16 qubits, FP32: 6.0 against 6.4 ms a pass), the
+    // others stay in it from pass to pass with plain ones (13 qubits, FP32,
+    // 256 MB: 71 against 93 us)
+    const bool nt = h->N * sizeof(T) > (256ull << 20);
+    if (nt)
+      hipLaunchKernelGGL((k_tile_reg<T, true>), dim3(fp.reg_geo.tiles), dim3(kRegThreads), 0, h->stream,
+                         static_cast<T *>(h->d_a), fp.reg_geo, st, fp.reg_stages, mem, d_vals);
+    else
+      hipLaunchKernelGGL((k_tile_reg<T, false>), dim3(fp.reg_geo.tiles), dim3(kRegThreads), 0, h->stream,
+                         static_cast<T *>(h->d_a), fp.reg_geo, st, fp.reg_stages, mem, d_vals);
+    return last_launch("k_tile_reg");
+  }
+  const TileOp *d_ops = reinterpret_cast<const TileOp *>(d_recs);
   const int nops = (int)fp.ops.size();
   bool dense = false, gen = false;
   for (const TileOp &op : fp.ops) {
@@ -2915,7 +3015,7 @@ int launch_memory_noise_tiles(dm_state *h, double f, double p, double g) {
         rec.insert(rec.end(), R, R + 12);
       }
       FusedPass fp;
-      if (int rc = parse_fused(h, rec.data(), (int64_t)rec.size(), 0, &fp)) return rc;
+      if (int rc = parse_fused(h, rec.data(), (int64_t)rec.size(), 0, &fp, true)) return rc;
       passes.push_back(std::move(fp));
       return DM_OK;
     };
@@ -2923,20 +3023,20 @@ int launch_memory_noise_tiles(dm_state *h, double f, double p, double g) {
     for (int lo = m; lo < n; lo += m - 3)
       if (int rc = add_pass(lo, std::min(n, lo + m - 3))) return rc;
     // device image: [records of every pass | values (T)], values 256-byte aligned
-    std::vector<TileOp> tops;
+    std::vector<uint32_t> tops;
     std::vector<T> vals;
     std::vector<size_t> top_off, val_off;
     for (const FusedPass &fp : passes) {
       top_off.push_back(tops.size());
       val_off.push_back(vals.size());
-      tops.insert(tops.end(), fp.ops.begin(), fp.ops.end());
+      fp.put_recs(&tops);
       for (double v : fp.vals) vals.push_back((T)v);
     }
-    const size_t vals_at = (tops.size() * sizeof(TileOp) + 255) & ~(size_t)255;
+    const size_t vals_at = (tops.size() * 4 + 255) & ~(size_t)255;
     const size_t bytes = vals_at + vals.size() * sizeof(T);
     HIP_TRY(hipStreamSynchronize(h->stream));  // earlier passes may still read the old image
     if (int rc = ensure(&h->d_mn, &h->mn_cap, bytes)) return rc;
-    HIP_TRY(hipMemcpy(h->d_mn, tops.data(), tops.size() * sizeof(TileOp), hipMemcpyHostToDevice));
+    HIP_TRY(hipMemcpy(h->d_mn, tops.data(), tops.size() * 4, hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(static_cast<char *>(h->d_mn) + vals_at, vals.data(), vals.size() * sizeof(T),
                       hipMemcpyHostToDevice));
     for (size_t &o : val_off) o = vals_at + o * sizeof(T);
@@ -2948,7 +3048,7 @@ int launch_memory_noise_tiles(dm_state *h, double f, double p, double g) {
     h->mn_key[2] = g;
   }
   for (size_t i = 0; i < h->mn_passes.size(); ++i) {
-    const TileOp *d_ops = static_cast<const TileOp *>(h->d_mn) + h->mn_top_off[i];
+    const uint32_t *d_ops = static_cast<const uint32_t *>(h->d_mn) + h->mn_top_off[i];
     const T *d_vals = reinterpret_cast<const T *>(static_cast<const char *>(h->d_mn) + h->mn_val_off[i]);
     if (int rc = launch_fused<T>(h, h->mn_passes[i], d_ops, d_vals)) return rc;
   }
@@ -2968,7 +3068,7 @@ struct Prepared {
   std::vector<int> fused_of;
   std::vector<size_t> offs, top_off;
   std::vector<int> pos;
-  std::vector<TileOp> tops;            // host image: records
+  std::vector<uint32_t> tops;          // host image: records (32-bit words)
   std::vector<unsigned char> values;   // host image: values, storage type
   size_t vals_at = 0;                  // byte offset of the values in the image
   const void *d_mat = nullptr;         // device values (after upload)
@@ -2989,7 +3089,7 @@ int stage_program(dm_state *h, const dm_op *ops, int nops, const double *params,
     if (ops[i].kind == DM_OP_FUSED) {
       if (ops[i].param < 0 || ops[i].param >= nparams) return fail(DM_ERR_ARG, "op %d: bad parameter offset", i);
       FusedPass fp;
-      if (int rc = parse_fused(h, params + ops[i].param, nparams - ops[i].param, i, &fp)) return rc;
+      if (int rc = parse_fused(h, params + ops[i].param, nparams - ops[i].param, i, &fp, true)) return rc;
       pp->fused_of[i] = (int)pp->fused.size();
       pool += fp.vals.size();
       pp->fused.push_back(std::move(fp));
@@ -3015,10 +3115,10 @@ int stage_program(dm_state *h, const dm_op *ops, int nops, const double *params,
       pp->offs[i] = off;
       for (double v : fp.vals) staging[off++] = (T)v;
       pp->top_off[pp->fused_of[i]] = pp->tops.size();
-      pp->tops.insert(pp->tops.end(), fp.ops.begin(), fp.ops.end());
+      fp.put_recs(&pp->tops);
     }
   }
-  pp->vals_at = (pp->tops.size() * sizeof(TileOp) + 255) & ~(size_t)255;
+  pp->vals_at = (pp->tops.size() * 4 + 255) & ~(size_t)255;
   pp->values.resize(staging.size() * sizeof(T));
   if (!staging.empty()) memcpy(pp->values.data(), staging.data(), pp->values.size());
   return DM_OK;
@@ -3031,7 +3131,7 @@ int upload_image(dm_state *h, Prepared *pp, void *dev) {
   if (pp->tops.empty() && pp->values.empty()) return DM_OK;
   HIP_TRY(hipStreamSynchronize(h->stream));
   if (!pp->tops.empty())
-    HIP_TRY(hipMemcpy(dev, pp->tops.data(), pp->tops.size() * sizeof(TileOp), hipMemcpyHostToDevice));
+    HIP_TRY(hipMemcpy(dev, pp->tops.data(), pp->tops.size() * 4, hipMemcpyHostToDevice));
   if (!pp->values.empty())
     HIP_TRY(hipMemcpy(static_cast<char *>(dev) + pp->vals_at, pp->values.data(), pp->values.size(),
                       hipMemcpyHostToDevice));
@@ -3066,7 +3166,7 @@ int launch_program(dm_state *h, const Prepared &pp) {
       case DM_OP_BLOCK: rc = launch_block_dev<T>(h, op.k, &pp.pos[4 * i], dmat + pp.offs[i]); break;
       case DM_OP_FUSED: {
         const int f = pp.fused_of[i];
-        rc = launch_fused<T>(h, pp.fused[f], static_cast<const TileOp *>(pp.d_ops) + pp.top_off[f],
+        rc = launch_fused<T>(h, pp.fused[f], static_cast<const uint32_t *>(pp.d_ops) + pp.top_off[f],
                              dmat + pp.offs[i]);
         break;
       }

@@ -1,0 +1,699 @@
+// tile_reg.h -- fused tile passes with the tile held in registers (gfx950).
+// Included by dmsim.hip.
+//
+// A workgroup of 256 threads owns a tile of 4^7 coefficients, 64 per thread:
+// three tile digits ("register digits") index a thread's 64 values, the four
+// others ("lane digits", three, and one "wave digit") say which thread holds
+// them.  A stage applies single-qubit maps and CX gates on its three register
+// digits without touching LDS; between stages the tile is redistributed
+// through LDS once so that the next three digits are in registers.
+
+constexpr int kRegTile = 7;
+constexpr int kRegThreads = 256;
+constexpr int kRegVals = 16;  // values of one member (unused ones zero)
+
+// Members of a stage.  A slot is a register digit (0, 1, 2).
+enum {
+  RM_U1 = 0,    // + slot: unital single-qubit map, 9 values (3x3, rows X Y Z)
+  RM_A1 = 3,    // + slot: general single-qubit map, 12 values (rows X Y Z, columns I X Y Z)
+  RM_CX = 6,    // + pair: CX, no values; pairs (control, target) (0,1) (1,0) (0,2) (2,0) (1,2) (2,1)
+  RM_D1 = 12,   // + slot: scale components X, Y, Z by 3 values
+  RM_D2 = 15,   // + pair of slots (0,1) (0,2) (1,2): 16 scales, index 4 i_first + i_second
+};
+
+struct RegStage {
+  uint32_t nm, mem;       // members: count, first one
+  // redistribution into this stage (unused in the first): the slot whose
+  // digit is a register digit before and after (it orders the phases), and
+  // the LDS offset (coefficients) of one unit of each other digit, for the
+  // writer's layout (the previous stage) and the reader's (this stage); a
+  // coefficient's offset is the XOR of its digits times their offsets
+  uint32_t slot;
+  uint32_t wr[3], wl[3], ww;
+  uint32_t rr[3], rl[3], rw;
+  uint32_t pad[3];
+};
+
+struct RegGeom {
+  int nr;
+  int rpos[kMaxQubits];   // positions enumerating the tiles, ascending
+  uint32_t tiles;
+  // HBM strides (coefficients) of the register digits and the wave digit in
+  // the layouts that load and store the tile; the lane digits are digits 0-2,
+  // 64 consecutive coefficients
+  uint64_t is[3], iw, os[3], ow;
+};
+
+// a * x + c into a register of its own choice: the compiler's two-address
+// form would accumulate into c and then copy the result into its place.
+__device__ __forceinline__ float reg_fma(float a, float x, float c) {
+  float r;
+  asm("v_fma_f32 %0, %1, %2, %3" : "=v"(r) : "s"(a), "v"(x), "v"(c));
+  return r;
+}
+__device__ __forceinline__ double reg_fma(double a, double x, double c) {
+  double r;
+  asm("v_fma_f64 %0, %1, %2, %3" : "=v"(r) : "s"(a), "v"(x), "v"(c));
+  return r;
+}
+
+template <typename T, int SLOT, bool AFF>
+__device__ __forceinline__ void reg_1q(T (&v)[64], const T (&pv)[kRegVals]) {
+  constexpr int S = 1 << (2 * SLOT);
+  constexpr int C = AFF ? 4 : 3;
+  T r[3][C];
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int j = 0; j < C; ++j) r[i][j] = pv[C * i + j];
+#pragma unroll
+  for (int o = 0; o < 16; ++o) {
+    const int b = SLOT == 0 ? 4 * o : SLOT == 1 ? (o & 3) + 16 * (o >> 2) : o;
+    const T x0 = v[b], x1 = v[b + S], x2 = v[b + 2 * S], x3 = v[b + 3 * S];
+    T t[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const T *q = &r[i][AFF ? 1 : 0];
+      const T first = AFF ? fmad(q[0], x1, r[i][0] * x0) : q[0] * x1;
+      t[i] = fmad(q[1], x2, first);
+    }
+#pragma unroll
+    for (int i = 0; i < 3; ++i) v[b + (i + 1) * S] = reg_fma(r[i][AFF ? 3 : 2], x3, t[i]);
+  }
+}
+
+template <typename T>
+__device__ __forceinline__ void reg_swap(T &a, T &b) {
+  if constexpr (sizeof(T) == 4) {
+    asm("v_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+  } else {
+    const T t = a;
+    a = b;
+    b = t;
+  }
+}
+
+// CX with control digit slot C and target slot T_ (pairs as cx_map).
+template <typename T, int C, int TG>
+__device__ __forceinline__ void reg_cx(T (&v)[64]) {
+  constexpr int SC = 1 << (2 * C), ST = 1 << (2 * TG), SO = 1 << (2 * (3 - C - TG));
+#pragma unroll
+  for (int o = 0; o < 4; ++o) {
+    auto X = [&](int c, int t) -> T & { return v[o * SO + c * SC + t * ST]; };
+    reg_swap(X(0, 2), X(3, 2));
+    reg_swap(X(0, 3), X(3, 3));
+    reg_swap(X(1, 0), X(1, 1));
+    reg_swap(X(1, 2), X(2, 3));
+    reg_swap(X(2, 0), X(2, 1));
+    reg_swap(X(1, 3), X(2, 2));
+    X(1, 3) = -X(1, 3);
+    X(2, 2) = -X(2, 2);
+  }
+}
+
+template <typename T, int SLOT>
+__device__ __forceinline__ void reg_d1(T (&v)[64], const T (&pv)[kRegVals]) {
+  constexpr int S = 1 << (2 * SLOT);
+  const T d[3] = {pv[0], pv[1], pv[2]};
+#pragma unroll
+  for (int i = 0; i < 64; ++i) {
+    const int c = (i / S) & 3;
+    if (c) v[i] *= d[c - 1];
+  }
+}
+
+template <typename T, int A, int B>
+__device__ __forceinline__ void reg_d2(T (&v)[64], const T (&pv)[kRegVals]) {
+  constexpr int SA = 1 << (2 * A), SB = 1 << (2 * B);
+  T d[16];
+#pragma unroll
+  for (int i = 1; i < 16; ++i) d[i] = pv[i];
+#pragma unroll
+  for (int i = 0; i < 64; ++i) {
+    const int c = 4 * ((i / SA) & 3) + ((i / SB) & 3);
+    if (c) v[i] *= d[c];
+  }
+}
+
+// The members of a stage in order.  The next member's kind and values are
+// loaded (scalar loads) while the current one computes.
+template <typename T>
+__device__ __forceinline__ void reg_members(T (&v)[64], const uint32_t *__restrict__ kinds, uint32_t nm,
+                                            const T *__restrict__ prm) {
+  if (nm == 0) return;
+  uint32_t next_kind = kinds[0];
+  T next[kRegVals];
+#pragma unroll
+  for (int i = 0; i < kRegVals; ++i) next[i] = prm[i];
+  for (uint32_t q = 0; q < nm; ++q) {
+    const uint32_t kind = __builtin_amdgcn_readfirstlane(next_kind);
+    T pv[kRegVals];
+#pragma unroll
+    for (int i = 0; i < kRegVals; ++i) pv[i] = next[i];
+    // scalar loads return out of order: wait for this member's values, then
+    // start the next one's (the arrays end with one spare member)
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+    __builtin_amdgcn_sched_barrier(0);
+    next_kind = kinds[q + 1];
+    prm += kRegVals;
+#pragma unroll
+    for (int i = 0; i < kRegVals; ++i) next[i] = prm[i];
+    __builtin_amdgcn_sched_barrier(0);
+    switch (kind) {
+      case RM_U1 + 0: reg_1q<T, 0, false>(v, pv); break;
+      case RM_U1 + 1: reg_1q<T, 1, false>(v, pv); break;
+      case RM_U1 + 2: reg_1q<T, 2, false>(v, pv); break;
+      case RM_A1 + 0: reg_1q<T, 0, true>(v, pv); break;
+      case RM_A1 + 1: reg_1q<T, 1, true>(v, pv); break;
+      case RM_A1 + 2: reg_1q<T, 2, true>(v, pv); break;
+      case RM_CX + 0: reg_cx<T, 0, 1>(v); break;
+      case RM_CX + 1: reg_cx<T, 1, 0>(v); break;
+      case RM_CX + 2: reg_cx<T, 0, 2>(v); break;
+      case RM_CX + 3: reg_cx<T, 2, 0>(v); break;
+      case RM_CX + 4: reg_cx<T, 1, 2>(v); break;
+      case RM_CX + 5: reg_cx<T, 2, 1>(v); break;
+      case RM_D1 + 0: reg_d1<T, 0>(v, pv); break;
+      case RM_D1 + 1: reg_d1<T, 1>(v, pv); break;
+      case RM_D1 + 2: reg_d1<T, 2>(v, pv); break;
+      case RM_D2 + 0: reg_d2<T, 0, 1>(v, pv); break;
+      case RM_D2 + 1: reg_d2<T, 0, 2>(v, pv); break;
+      default: reg_d2<T, 1, 2>(v, pv); break;
+    }
+  }
+}
+
+// Redistribution through LDS in phases: phase h moves the coefficients whose
+// digit in SLOT (a register digit before and after) lies in the h-th part of
+// its range, from and into the same registers, so that a phase needs only
+// 1/PH of the tile's bytes of LDS and several workgroups fit a CU.
+template <typename T, int SLOT, int PH>
+__device__ __forceinline__ void reg_exchange(T (&v)[64], T *s, const RegStage &st, int lane, int wave) {
+  constexpr int S = 1 << (2 * SLOT);
+  constexpr int IN = 4 / PH;  // digit values per phase
+  const uint32_t l0 = lane & 3, l1 = (lane >> 2) & 3, l2 = lane >> 4;
+  constexpr uint32_t B = sizeof(T);
+  const uint32_t tw = ((l0 * st.wl[0]) ^ (l1 * st.wl[1]) ^ (l2 * st.wl[2]) ^ ((uint32_t)wave * st.ww)) * B;
+  const uint32_t tr = ((l0 * st.rl[0]) ^ (l1 * st.rl[1]) ^ (l2 * st.rl[2]) ^ ((uint32_t)wave * st.rw)) * B;
+  constexpr int SA = SLOT == 0 ? 1 : 0, SB = SLOT == 2 ? 1 : 2;  // the other slots
+  char *c = reinterpret_cast<char *>(s);
+#pragma unroll
+  for (int h = 0; h < PH; ++h) {
+    __syncthreads();  // the previous phase has been read
+#pragma unroll
+    for (int i = 0; i < 64; ++i) {
+      const int d = (i / S) & 3;
+      if (d / IN != h) continue;
+      const uint32_t o = ((((i >> (2 * SA)) & 3) * st.wr[SA]) ^ (((i >> (2 * SB)) & 3) * st.wr[SB])) * B;
+      *reinterpret_cast<T *>(c + (tw ^ o) + (d % IN) * 4096 * B) = v[i];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 64; ++i) {
+      const int d = (i / S) & 3;
+      if (d / IN != h) continue;
+      const uint32_t o = ((((i >> (2 * SA)) & 3) * st.rr[SA]) ^ (((i >> (2 * SB)) & 3) * st.rr[SB])) * B;
+      v[i] = *reinterpret_cast<const T *>(c + (tr ^ o) + (d % IN) * 4096 * B);
+    }
+  }
+}
+
+template <typename T, bool NTM>
+__device__ __forceinline__ T reg_load(const T *p, uint32_t off) {
+  const T *q = reinterpret_cast<const T *>(reinterpret_cast<const char *>(p) + off);
+  return NTM ? __builtin_nontemporal_load(q) : *q;
+}
+template <typename T, bool NTM>
+__device__ __forceinline__ void reg_store(T *p, uint32_t off, T x) {
+  T *q = reinterpret_cast<T *>(reinterpret_cast<char *>(p) + off);
+  if (NTM) __builtin_nontemporal_store(x, q);
+  else *q = x;
+}
+
+// Phases of a redistribution: 32 KB of LDS (FP32 two phases, FP64 four).
+template <typename T>
+struct RegShape {
+  static constexpr int phases = sizeof(T) == 4 ? 2 : 4;
+  static constexpr int lds = (1 << (2 * kRegTile)) / phases;  // coefficients
+};
+
+template <typename T, bool NTM>
+__device__ __forceinline__ void reg_tile(T *__restrict__ a, T *s, const RegGeom &geo, uint32_t tile,
+                                         const RegStage *__restrict__ st, int ns, const uint32_t *__restrict__ kinds,
+                                         const T *__restrict__ prm) {
+  constexpr int PH = RegShape<T>::phases;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  uint64_t base = 0;
+  {
+    uint32_t r = tile;
+    for (int j = 0; j < geo.nr; ++j) {
+      base |= (uint64_t)(r & 3u) << (2 * geo.rpos[j]);
+      r >>= 2;
+    }
+  }
+  const uint32_t loff = lane * (uint32_t)sizeof(T);
+  T v[64];
+  {
+    const T *p = a + base + wave * geo.iw;
+#pragma unroll
+    for (int i = 0; i < 64; ++i)
+      v[i] = reg_load<T, NTM>(p + (i & 3) * geo.is[0] + ((i >> 2) & 3) * geo.is[1] + (i >> 4) * geo.is[2], loff);
+  }
+  for (int k = 0; k < ns; ++k) {
+    const RegStage sg = st[k];
+    if (k) {
+      if (sg.slot == 0) reg_exchange<T, 0, PH>(v, s, sg, lane, wave);
+      else if (sg.slot == 1) reg_exchange<T, 1, PH>(v, s, sg, lane, wave);
+      else reg_exchange<T, 2, PH>(v, s, sg, lane, wave);
+    }
+    reg_members<T>(v, kinds + sg.mem, sg.nm, prm + (size_t)sg.mem * kRegVals);
+  }
+  {
+    T *p = a + base + wave * geo.ow;
+#pragma unroll
+    for (int i = 0; i < 64; ++i)
+      reg_store<T, NTM>(p + (i & 3) * geo.os[0] + ((i >> 2) & 3) * geo.os[1] + (i >> 4) * geo.os[2], loff, v[i]);
+  }
+}
+
+template <typename T, bool NTM>
+__global__ __launch_bounds__(kRegThreads, sizeof(T) == 4 ? 4 : 2) void k_tile_reg(T *__restrict__ a, RegGeom geo,
+                                                             const RegStage *__restrict__ st, int ns,
+                                                             const uint32_t *__restrict__ kinds,
+                                                             const T *__restrict__ prm) {
+  __shared__ __align__(16) T s[RegShape<T>::lds];
+  if (blockIdx.x >= geo.tiles) return;  // uniform over the workgroup
+  reg_tile<T, NTM>(a, s, geo, blockIdx.x, st, ns, kinds, prm);
+}
+
+// ---------------------------------------------------------------------------
+// Host: the register program of a fused pass.
+// ---------------------------------------------------------------------------
+
+struct RegItem {
+  uint32_t mask;       // tile digits
+  int kind;            // 0: single-qubit map, 1: CX, 2: pair scale
+  bool scaled;         // CX with 16 pair scales
+  bool exact;          // rounds nothing (a CX permutation)
+  int d0, d1;
+  double v[16];        // rows X, Y, Z (12 values), or 16 pair scales
+};
+
+// Kind and values of a single-qubit map: identity (no member), diagonal,
+// unital or general.
+inline int reg_1q_kind(const double *r) {
+  bool unital = true, diag = true, ident = true;
+  for (int i = 0; i < 3; ++i) {
+    if (r[4 * i] != 0.0) unital = false;
+    for (int j = 0; j < 3; ++j) {
+      const double x = r[4 * i + 1 + j];
+      if (i != j && x != 0.0) diag = false;
+      if (x != (i == j ? 1.0 : 0.0)) ident = false;
+    }
+  }
+  if (!unital) return RM_A1;
+  return ident ? -1 : diag ? RM_D1 : RM_U1;
+}
+
+// The operations of a pass in their given order, one item each (two for a
+// scaled CX: the permutation and the scale).
+inline std::vector<RegItem> reg_items_in_order(const std::vector<TileOp> &ops, const std::vector<double> &vals) {
+  std::vector<RegItem> out;
+  out.reserve(2 * ops.size());
+  for (const TileOp &op : ops) {
+    const double *v = vals.data() + op.param;
+    RegItem it;
+    it.scaled = false;
+    it.d0 = op.d[0];
+    if (op.kind == TOP_1Q || op.kind == TOP_1QU) {
+      it.kind = 0;
+      it.d1 = op.d[0];
+      it.mask = 1u << op.d[0];
+      it.exact = false;
+      memcpy(it.v, v, 12 * sizeof(double));
+      out.push_back(it);
+      continue;
+    }
+    it.kind = 1;
+    it.d1 = op.d[1];
+    it.mask = (1u << it.d0) | (1u << it.d1);
+    it.exact = true;
+    out.push_back(it);
+    bool scaled = false;
+    for (int i = 1; op.k && i < 16; ++i) scaled = scaled || v[i] != 1.0;
+    if (scaled) {
+      it.kind = 2;
+      it.exact = false;
+      memcpy(it.v, v, 16 * sizeof(double));
+      out.push_back(it);
+    }
+  }
+  return out;
+}
+
+// The pass's operations as register-stage items, free to be reordered where
+// they commute: runs of single-qubit maps on one digit become one map, and
+// the separable scale of a CX (a depolarising channel on each of its qubits)
+// goes into the next map on either digit where one follows before another
+// CX, so that the CX itself only permutes registers; what is left stays as a
+// scale of its own.
+inline std::vector<RegItem> reg_items(const std::vector<TileOp> &ops, const std::vector<double> &vals, int m) {
+  std::vector<RegItem> out;
+  out.reserve(2 * ops.size());
+  int pend[8];  // item index of the single-qubit map a digit's next one joins, or -1
+  for (int d = 0; d < m; ++d) pend[d] = -1;
+  for (const TileOp &op : ops) {
+    const double *v = vals.data() + op.param;
+    if (op.kind == TOP_1Q) {
+      const int d = op.d[0];
+      if (pend[d] < 0) {
+        RegItem it;
+        it.mask = 1u << d;
+        it.kind = 0;
+        it.scaled = it.exact = false;
+        it.d0 = it.d1 = d;
+        memcpy(it.v, v, 12 * sizeof(double));
+        pend[d] = (int)out.size();
+        out.push_back(it);
+      } else {
+        // (I, X, Y, Z) -> rows of the later map applied to the earlier one
+        double *e = out[pend[d]].v, w[12];
+        for (int i = 0; i < 3; ++i)
+          for (int j = 0; j < 4; ++j) {
+            double acc = j == 0 ? v[4 * i] : 0.0;
+            for (int k = 0; k < 3; ++k) acc += v[4 * i + 1 + k] * e[4 * k + j];
+            w[4 * i + j] = acc;
+          }
+        memcpy(e, w, sizeof(w));
+      }
+    } else {
+      RegItem it;
+      it.d0 = op.d[0];
+      it.d1 = op.d[1];
+      it.mask = (1u << it.d0) | (1u << it.d1);
+      it.kind = 1;
+      it.scaled = op.k != 0;
+      it.exact = false;
+      if (op.k) memcpy(it.v, v, 16 * sizeof(double));
+      out.push_back(it);
+      pend[it.d0] = pend[it.d1] = -1;
+    }
+  }
+  // scales
+  std::vector<RegItem> res;
+  res.reserve(out.size() + 8);
+  for (size_t i = 0; i < out.size(); ++i) {
+    const RegItem it = out[i];
+    if (it.kind != 1 || !it.scaled) {
+      res.push_back(it);
+      continue;
+    }
+    bool scaled = false, separable = it.v[0] == 1.0;
+    for (int c = 0; c < 4; ++c)
+      for (int t = 0; t < 4; ++t) {
+        const double s = it.v[4 * c + t];
+        if (s != 1.0 && (c | t)) scaled = true;
+        if (!(fabs(s - it.v[4 * c] * it.v[t]) <= 4e-16 * fabs(s))) separable = false;
+      }
+    RegItem cx = it;
+    cx.scaled = false;
+    res.push_back(cx);
+    if (!scaled) continue;
+    RegItem *next[2] = {nullptr, nullptr};
+    if (separable)
+      for (int s = 0; s < 2; ++s) {
+        const uint32_t bit = 1u << (s ? it.d1 : it.d0);
+        for (size_t j = i + 1; j < out.size(); ++j)
+          if (out[j].mask & bit) {
+            if (out[j].kind == 0) next[s] = &out[j];
+            break;
+          }
+      }
+    for (int s = 0; s < 2; ++s)
+      if (next[s])
+        for (int r = 0; r < 3; ++r)
+          for (int c = 1; c < 4; ++c) next[s]->v[4 * r + c] *= s ? it.v[c] : it.v[4 * c];
+    if (next[0] && next[1]) continue;
+    RegItem d = it;
+    if (!next[0] && !next[1]) {
+      d.kind = 2;
+    } else {
+      const int s = next[0] ? 1 : 0;
+      d.kind = 0;
+      d.d0 = d.d1 = s ? it.d1 : it.d0;
+      d.mask = 1u << d.d0;
+      for (int r = 0; r < 3; ++r)
+        for (int c = 0; c < 4; ++c) d.v[4 * r + c] = c == r + 1 ? (s ? it.v[c] : it.v[4 * c]) : 0.0;
+    }
+    res.push_back(d);
+  }
+  return res;
+}
+
+// Items (of those with done[i] == 0) that a stage on the digits of `triple`
+// takes: an item joins unless it, or an earlier one left out that it does
+// not commute with, reaches outside the triple.  Items on different digits
+// commute; with `ordered` (results bit for bit those of the given order)
+// only if one of them rounds nothing.
+inline int reg_absorb(const std::vector<RegItem> &items, const std::vector<char> &done, size_t first, uint32_t triple,
+                      bool ordered, std::vector<int> *take) {
+  uint32_t blocked = 0;
+  bool rounded = false;  // an item that rounds was left out
+  int n = 0;
+  for (size_t i = first; i < items.size(); ++i) {
+    if (done[i]) continue;
+    const uint32_t m = items[i].mask;
+    if ((m & blocked) || (m & ~triple) || (ordered && rounded && !items[i].exact)) {
+      blocked |= m;
+      rounded = rounded || !items[i].exact;
+      if (!(triple & ~blocked)) break;
+    } else {
+      ++n;
+      if (take) take->push_back((int)i);
+    }
+  }
+  return n;
+}
+
+struct RegPlan {
+  RegGeom geo;
+  int ns = 0;
+  std::vector<uint32_t> words;  // RegStage records, then the members' kinds and one spare
+  std::vector<double> vals;     // kRegVals values a member, and one spare block
+};
+
+// Stages: the first one on a layout that loads HBM directly (register digits
+// among 3-6, lanes on digits 0-2: 64 consecutive coefficients per access),
+// each further one on the three digits that take the most pending items, and
+// a last, possibly empty one on a layout that stores directly.  With
+// `ordered` the operations keep their order (see reg_absorb).
+inline void reg_plan(const std::vector<TileOp> &ops, const std::vector<double> &vals, const int *tpos, const int *rpos,
+                     int nr, bool ordered, RegPlan *out) {
+  constexpr int m = kRegTile;
+  const std::vector<RegItem> items = ordered ? reg_items_in_order(ops, vals) : reg_items(ops, vals, m);
+  uint32_t triples[35], nt = 0;
+  for (int a = 3; a < m; ++a)  // the 4 load / store layouts first
+    for (int b = a + 1; b < m; ++b)
+      for (int c = b + 1; c < m; ++c) triples[nt++] = (1u << a) | (1u << b) | (1u << c);
+  const uint32_t nio = nt;
+  for (int a = 0; a < 3; ++a)
+    for (int b = a + 1; b < m; ++b)
+      for (int c = b + 1; c < m; ++c) triples[nt++] = (1u << a) | (1u << b) | (1u << c);
+  std::vector<char> done(items.size(), 0);
+  std::vector<uint32_t> stage;
+  std::vector<std::vector<int>> members;
+  size_t first = 0, left = items.size();
+  while (left || stage.empty()) {
+    uint32_t best = 0;
+    int most = -1;
+    for (uint32_t t = 0; t < (stage.empty() ? nio : nt); ++t) {
+      if (!stage.empty() && !(triples[t] & stage.back())) continue;  // a redistribution keeps one digit
+      const int n = reg_absorb(items, done, first, triples[t], ordered, nullptr);
+      if (n > most) {
+        most = n;
+        best = t;
+      }
+    }
+    std::vector<int> take;
+    reg_absorb(items, done, first, triples[best], ordered, &take);
+    for (int i : take) done[i] = 1;
+    if (take.empty() && !stage.empty()) {
+      // the pending items' digits are all outside the triples that share a
+      // digit with this one: step through a triple that holds one of each
+      for (size_t i = first; i < items.size(); ++i)
+        if (!done[i]) {
+          best = nt;
+          for (uint32_t t = 0; t < nt && best == nt; ++t)
+            if ((triples[t] & stage.back()) && (triples[t] & items[i].mask)) best = t;
+          break;
+        }
+    }
+    left -= take.size();
+    while (first < items.size() && done[first]) ++first;
+    stage.push_back(triples[best]);
+    members.push_back(std::move(take));
+  }
+  if (stage.back() & 7u) {  // an empty stage that stores directly
+    const uint32_t last = stage.back();
+    uint32_t best = nio;
+    for (uint32_t t = 0; t < nio; ++t)
+      if ((triples[t] & last) && (best == nio || __builtin_popcount(triples[t] & last) >
+                                                     __builtin_popcount(triples[best] & last)))
+        best = t;
+    if (best == nio) {  // digits 0-2 in registers: one stage in between
+      stage.push_back((1u << 2) | (1u << 3) | (1u << 4));
+      members.emplace_back();
+      best = 0;  // digits 3, 4, 5
+    }
+    stage.push_back(triples[best]);
+    members.emplace_back();
+  }
+  const int ns = (int)stage.size();
+  struct Lay {
+    int r[3], l[3], w, slot;
+  };
+  std::vector<Lay> lay(ns);
+  for (int k = 0; k < ns; ++k) {
+    Lay &y = lay[k];
+    int reg[3], nreg = 0, rest[4], nrest = 0;
+    for (int d = 0; d < m; ++d) {
+      if ((stage[k] >> d) & 1) reg[nreg++] = d;
+      else rest[nrest++] = d;
+    }
+    // register digits: those kept from the previous stage stay in their
+    // slots, the first such slot orders the phases
+    for (int j = 0; j < 3; ++j) y.r[j] = -1;
+    y.slot = 0;
+    if (k) {
+      y.slot = -1;
+      for (int j = 0; j < 3; ++j)
+        if ((stage[k] >> lay[k - 1].r[j]) & 1) {
+          y.r[j] = lay[k - 1].r[j];
+          y.slot = j;  // the last one
+        }
+    }
+    for (int x = 0; x < 3; ++x) {
+      bool held = false;
+      for (int j = 0; j < 3; ++j) held = held || y.r[j] == reg[x];
+      for (int j = 0; j < 3 && !held; ++j)
+        if (y.r[j] < 0) {
+          y.r[j] = reg[x];
+          held = true;
+        }
+    }
+    // lane digits: digits 0-2 at the lane index of the load / store layouts,
+    // digits that were lanes before at their index; the wave digit is the
+    // highest of the others
+    for (int j = 0; j < 3; ++j) y.l[j] = -1;
+    bool used[8] = {false};
+    for (int x = 0; x < 4; ++x)
+      if (rest[x] < 3) {
+        y.l[rest[x]] = rest[x];
+        used[rest[x]] = true;
+      }
+    if (k)
+      for (int j = 0; j < 3; ++j) {
+        const int d = lay[k - 1].l[j];
+        if (d >= 3 && y.l[j] < 0 && !((stage[k] >> d) & 1)) {
+          y.l[j] = d;
+          used[d] = true;
+        }
+      }
+    int x = 0;
+    for (int j = 0; j < 3; ++j)
+      if (y.l[j] < 0) {
+        while (used[rest[x]]) ++x;
+        y.l[j] = rest[x];
+        used[rest[x]] = true;
+      }
+    for (int q = 0; q < 4; ++q)
+      if (!used[rest[q]]) y.w = rest[q];
+  }
+  memset(&out->geo, 0, sizeof(out->geo));
+  out->geo.nr = nr;
+  for (int j = 0; j < nr; ++j) out->geo.rpos[j] = rpos[j];
+  out->geo.tiles = 1u << (2 * nr);
+  for (int j = 0; j < 3; ++j) {
+    out->geo.is[j] = pow4(tpos[lay[0].r[j]]);
+    out->geo.os[j] = pow4(tpos[lay[ns - 1].r[j]]);
+  }
+  out->geo.iw = pow4(tpos[lay[0].w]);
+  out->geo.ow = pow4(tpos[lay[ns - 1].w]);
+  out->ns = ns;
+  out->words.clear();
+  out->vals.clear();
+  std::vector<uint32_t> kinds;
+  for (int k = 0; k < ns; ++k) {
+    RegStage sg;
+    memset(&sg, 0, sizeof(sg));
+    sg.mem = (uint32_t)kinds.size();
+    auto slot = [&](int d) { return lay[k].r[0] == d ? 0 : lay[k].r[1] == d ? 1 : 2; };
+    for (int i : members[k]) {
+      const RegItem &it = items[i];
+      double v[kRegVals] = {0.0};
+      uint32_t kind;
+      if (it.kind == 0) {
+        const int k1 = reg_1q_kind(it.v);
+        if (k1 < 0) continue;
+        kind = k1 + slot(it.d0);
+        int at = 0;
+        for (int r = 0; r < 3; ++r)
+          for (int c = 0; c < 4; ++c)
+            if (k1 == RM_A1 || (k1 == RM_U1 && c > 0) || (k1 == RM_D1 && c == r + 1)) v[at++] = it.v[4 * r + c];
+      } else {
+        const int s0 = slot(it.d0), s1 = slot(it.d1);
+        const int lo = std::min(s0, s1), hi = std::max(s0, s1);
+        const int pair = lo == 0 ? hi - 1 : 2;  // (0,1) (0,2) (1,2)
+        if (it.kind == 1) {
+          kind = RM_CX + 2 * pair + (s0 > s1 ? 1 : 0);
+        } else {
+          kind = RM_D2 + pair;
+          for (int a = 0; a < 4; ++a)
+            for (int b = 0; b < 4; ++b) v[4 * a + b] = it.v[s0 < s1 ? 4 * a + b : 4 * b + a];
+        }
+      }
+      kinds.push_back(kind);
+      out->vals.insert(out->vals.end(), v, v + kRegVals);
+    }
+    sg.nm = (uint32_t)kinds.size() - sg.mem;
+    if (k) {
+      // LDS offsets of the digits.  The banks are the lowest three base-4
+      // digits of the coefficient index: the writer's lane digits sit there,
+      // and a lane digit of the reader that is none of them is added (XOR)
+      // to the place of one that is no lane of the reader, so that the lanes of a wave fall on
+      // distinct banks on both sides.  Every digit but the writer's lanes
+      // and the phase digit also has a place of its own above them.
+      const Lay &w = lay[k - 1], &y = lay[k];
+      uint32_t co[8] = {0};
+      for (int j = 0; j < 3; ++j) co[w.l[j]] = 1u << (2 * j);
+      int high = 3;
+      for (int d = 0; d < m; ++d)
+        if (!co[d] && d != y.r[y.slot]) co[d] = 1u << (2 * high++);
+      bool place[3];  // places of writer lanes that are no reader lanes
+      for (int j = 0; j < 3; ++j) place[j] = w.l[j] != y.l[0] && w.l[j] != y.l[1] && w.l[j] != y.l[2];
+      for (int j = 0; j < 3; ++j) {
+        if (y.l[j] == w.l[0] || y.l[j] == w.l[1] || y.l[j] == w.l[2]) continue;
+        int at = j;
+        while (!place[at]) at = (at + 1) % 3;
+        place[at] = false;
+        co[y.l[j]] |= 1u << (2 * at);
+      }
+      sg.slot = (uint32_t)y.slot;
+      for (int j = 0; j < 3; ++j) {
+        sg.wr[j] = co[w.r[j]];
+        sg.wl[j] = co[w.l[j]];
+        sg.rr[j] = co[y.r[j]];
+        sg.rl[j] = co[y.l[j]];
+      }
+      sg.ww = co[w.w];
+      sg.rw = co[y.w];
+    }
+    uint32_t w[sizeof(RegStage) / 4];
+    memcpy(w, &sg, sizeof(sg));
+    out->words.insert(out->words.end(), w, w + sizeof(RegStage) / 4);
+  }
+  // the spare member that the last one's prefetch reads
+  kinds.push_back(0);
+  out->words.insert(out->words.end(), kinds.begin(), kinds.end());
+  out->vals.resize(out->vals.size() + kRegVals, 0.0);
+}

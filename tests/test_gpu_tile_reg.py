@@ -1,0 +1,127 @@
+"""Register-resident fused passes against the oracle.
+
+Passes of many single-qubit maps and CX gates on a few qubits take the
+register-resident kernel from 7 qubits up (always from 12).  The cases cover
+every place of the operands in the tile (load and store layouts, the digits
+that lie across lanes, tiles of 5-7 digits completed to 7), unital, general
+and diagonal maps, plain CX and CX with separable and general pair scales,
+and the first and last digits of the register.
+Tolerance: an output coefficient passes through at most one operation per
+member, each a sum of at most 4 products of magnitude <= the state's largest
+coefficient times the map's row norm (<= 2 here, kept below 1 on average by
+the maps' contraction), so max|da| <= members * 8 eps * max over time of
+max|a|, taken from the oracle's own states.
+"""
+import numpy as np
+import pytest
+
+from dmsim import native, ptm
+from dmsim.program import Program
+from oracle import refsim
+
+pytestmark = pytest.mark.gpu
+
+EPS = {'fp64': 2.0 ** -53, 'fp32': 2.0 ** -24}
+
+
+def oracle_1q(a, n, q, R4):
+    x = a.reshape(4 ** q, 4, 4 ** (n - q - 1))
+    return np.einsum('ij,ajb->aib', R4, x).reshape(-1)
+
+
+def oracle_cx(a, n, c, t, scale):
+    x = refsim.apply_cx(a.copy().reshape(n * [4]), c, t, [1.0, 0.0], n)  # updates its argument
+    if scale is not None:
+        x = np.moveaxis(x, (c, t), (0, 1))
+        x = np.asarray(scale).reshape(4, 4)[(...,) + (None,) * (n - 2)] * x
+        x = np.moveaxis(x, (0, 1), (c, t))
+    return np.ascontiguousarray(x).reshape(-1)
+
+
+def random_map(rng, kind):
+    R = np.eye(4)
+    th, ph, la = rng.uniform(0, 2 * np.pi, 3)
+    if kind != 'diag':
+        R = ptm.gate_ptm('u3', [th, ph, la])
+    R = ptm.depolarizing1(rng.uniform(0, 0.1)) @ R
+    if kind == 'general':
+        R = ptm.memory_noise(0.9, 0.8, 0.7) @ R
+    return R
+
+
+def random_scale(rng, kind):
+    if kind == 'none':
+        return None
+    a, b = (np.concatenate([[1.0], rng.uniform(0.5, 1.0, 3)]) for _ in range(2))
+    s = np.outer(a, b).reshape(16)
+    if kind == 'general':
+        s = rng.uniform(0.5, 1.0, 16)
+        s[0] = 1.0
+    return s
+
+
+def check(n, m, qubits, members, precision, seed):
+    rng = np.random.default_rng(seed)
+    a = rng.normal(size=4 ** n) * 2.0 ** -n
+    a[0] = 2.0 ** -n
+    if precision == 'fp32':
+        a = a.astype(np.float32).astype(np.float64)
+    want, top, sub = a, np.abs(a).max(), []
+    for _ in range(members):
+        if rng.random() < 0.5:
+            q = int(rng.choice(qubits))
+            R = random_map(rng, rng.choice(['unital', 'general', 'diag']))
+            sub.append((native.SUB_1Q, [q], ptm.rows3(R)))
+            want = oracle_1q(want, n, q, R)
+        else:
+            c, t = (int(x) for x in rng.choice(qubits, 2, replace=False))
+            s = random_scale(rng, rng.choice(['none', 'separable', 'general']))
+            sub.append((native.SUB_CX, [c, t], s))
+            want = oracle_cx(want, n, c, t, s)
+        top = max(top, np.abs(want).max())
+    prog = Program(n)
+    prog.fused(m, qubits, sub)
+    st = native.DeviceState(n, precision)
+    st.upload(a)
+    prog.run(st)
+    got = st.download()
+    st.close()
+    assert got[0] == 2.0 ** -n
+    err = np.abs(got - want).max()
+    assert err <= members * 8 * EPS[precision] * top, (n, m, qubits, seed, err, top)
+
+
+@pytest.mark.parametrize('precision', ['fp64', 'fp32'])
+@pytest.mark.parametrize('n,m,qubits', [
+    (7, 7, [0, 1, 2]), (7, 7, [4, 5, 6]), (7, 6, [0, 6]), (8, 7, [0, 1, 2, 3]), (8, 5, [6, 7]), (8, 6, [1, 4, 7]),
+    (9, 7, [0, 2, 4, 5]), (9, 6, [0, 1, 2]), (9, 7, [0, 1, 7, 8]),
+])
+def test_many_members_on_few_qubits(n, m, qubits, precision):
+    for seed in range(4):
+        check(n, m, qubits, 24 + 8 * seed, precision, 100 * n + seed)
+
+
+@pytest.mark.parametrize('precision', ['fp64', 'fp32'])
+@pytest.mark.parametrize('qubits,members', [([0, 1, 2, 3], 1), ([11], 3), ([0, 5, 10, 11], 9), ([8, 9, 10, 11], 14),
+                                            ([0, 3, 6], 0)])
+def test_every_pass_from_12_qubits(qubits, members, precision):
+    if len(qubits) == 1:
+        n = 12
+        rng = np.random.default_rng(5)
+        a = rng.normal(size=4 ** n) * 2.0 ** -n
+        a[0] = 2.0 ** -n
+        a = a.astype(np.float32).astype(np.float64)
+        R = random_map(rng, 'general')
+        prog = Program(n)
+        prog.fused(6, qubits, [(native.SUB_1Q, qubits, ptm.rows3(R))] * members)
+        st = native.DeviceState(n, precision)
+        st.upload(a)
+        prog.run(st)
+        got = st.download()
+        st.close()
+        want = a
+        for _ in range(members):
+            want = oracle_1q(want, n, qubits[0], R)
+        assert np.abs(got - want).max() <= members * 8 * EPS[precision] * np.abs(a).max()
+        return
+    check(12, 7, qubits, members, precision, 7)
