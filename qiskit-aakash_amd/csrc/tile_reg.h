@@ -484,7 +484,8 @@ struct RegPlan {
 
 // Stages: the first one on a layout that loads HBM directly (register digits
 // among 3-6, lanes on digits 0-2: 64 consecutive coefficients per access),
-// each further one on the three digits that take the most pending items, and
+// each further one on the three digits that take the most pending items (at
+// least one: an item's digits and one kept from the stage before), and
 // a last, possibly empty one on a layout that stores directly.  With
 // `ordered` the operations keep their order (see reg_absorb).
 inline void reg_plan(const std::vector<TileOp> &ops, const std::vector<double> &vals, const int *tpos, const int *rpos,
@@ -517,17 +518,6 @@ inline void reg_plan(const std::vector<TileOp> &ops, const std::vector<double> &
     std::vector<int> take;
     reg_absorb(items, done, first, triples[best], ordered, &take);
     for (int i : take) done[i] = 1;
-    if (take.empty() && !stage.empty()) {
-      // the pending items' digits are all outside the triples that share a
-      // digit with this one: step through a triple that holds one of each
-      for (size_t i = first; i < items.size(); ++i)
-        if (!done[i]) {
-          best = nt;
-          for (uint32_t t = 0; t < nt && best == nt; ++t)
-            if ((triples[t] & stage.back()) && (triples[t] & items[i].mask)) best = t;
-          break;
-        }
-    }
     left -= take.size();
     while (first < items.size() && done[first]) ++first;
     stage.push_back(triples[best]);

@@ -7,11 +7,12 @@ all qubits with polarisation retention ``depolarization_factor``.  Small
 registers (<= ``lds_max_qubits``) run whole inside one workgroup's LDS; the
 others keep their state in one HBM arena and run as fused 6-digit tile
 passes (7-digit in FP32 where 6 digits would leave contiguous runs of 4^2
-or 4^3 coefficients that 7 digits lengthen); round r (pass r of every
-circuit) is up to three launches side by side: the initialisation and
-probability work, split into at most ``items_per_pass`` work items per
-pass, and one launch per tile size with a workgroup per tile; the batch is
-captured once into a hipGraph and replayed (``dm_batch_*`` in dmsim.h).
+or 4^3 coefficients that 7 digits lengthen), in groups whose states stay
+in the last-level cache; round r of a group (pass r of its circuits) is up
+to three launches: the initialisation and probability work, split into at
+most ``items_per_pass`` work items per pass, and one launch per tile size
+with a workgroup per tile; the batch is captured once into a hipGraph and
+replayed (``dm_batch_*`` in dmsim.h).
 
 ``autotune`` picks the LDS cutoff width, the LDS workgroup size and the
 HBM tier's items per pass by timing the candidates on the batch itself; the
