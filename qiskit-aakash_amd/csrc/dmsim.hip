@@ -2680,10 +2680,10 @@ bool plan_reg(const dm_state *h, FusedPass *fp) {
   for (TileOp &op : ops)
     for (int x = 0; x < (op.kind == TOP_CX ? 2 : 1); ++x) op.d[x] = digit[fp->geo.tpos[op.d[x]]];
   RegPlan rp;
-  reg_plan(ops, vals, tpos, rpos, nr, ordered, &rp);
+  reg_plan(ordered ? reg_items_in_order(ops, vals) : reg_items(ops, vals, kRegTile), kRegTile, true, ordered, &rp);
   if (few && ops.size() < 4 * (size_t)rp.ns) return false;
   fp->reg = true;
-  fp->reg_geo = rp.geo;
+  fp->reg_geo = reg_geom(rp, tpos, rpos, nr);
   fp->reg_stages = rp.ns;
   fp->recs = std::move(rp.words);
   fp->vals = std::move(rp.vals);
@@ -3280,8 +3280,14 @@ struct dm_batch {
   // LDS tier: circuits held entirely in one workgroup's LDS, grouped by width
   std::vector<int> small;
   std::vector<int> small_width_start;  // per width 1..7: first index into small-ordered arrays
+  // in the order: register-resident circuits of up to 6 qubits, of 7 qubits,
+  // then the others by width (small_width_start)
+  int nreg6 = 0, nreg7 = 0;
+  void *d_rcircs = nullptr, *d_rrecs = nullptr, *d_rvals = nullptr;
   void *d_circs = nullptr, *d_tops = nullptr, *d_vals = nullptr;
   int lds_threads = 256;
+  hipStream_t side2 = nullptr;
+  hipEvent_t join2 = nullptr;
   // HBM tier: the states in one arena, the pass table, the items in round
   // order (round r: pass r of every circuit), and the tile operations and
   // values of every pass
@@ -3395,6 +3401,42 @@ int small_circuit_ops(int n, const dm_op *ops, int nops, const double *params, i
   return DM_OK;
 }
 
+// The register-resident program of a small circuit; *fits false (and no
+// error) if it holds operations that form does not take.  FP64: memory noise
+// and single-qubit maps between two CX gates on a qubit become one map.
+// FP32: every operation on its own and in order, as the LDS kernel rounds.
+template <typename T>
+int small_circuit_plan(int n, const dm_op *ops, int nops, const double *params, int64_t nparams, int ci, bool *fits,
+                       RegPlan *rp) {
+  std::vector<TileOp> tops;
+  std::vector<double> vals;
+  if (int rc = small_circuit_ops(n, ops, nops, params, nparams, ci, &tops, &vals)) return rc;
+  std::vector<TileOp> flat;
+  flat.reserve(tops.size() * 2);
+  for (const TileOp &op : tops) {
+    if (op.kind == TOP_2Q) {
+      *fits = false;
+      return DM_OK;
+    }
+    if (op.kind != TOP_ALLQ) {
+      flat.push_back(op);
+      continue;
+    }
+    for (int d = 0; d < n; ++d) {
+      TileOp one = op;
+      one.kind = TOP_1Q;
+      one.k = 1;
+      one.d[0] = d;
+      flat.push_back(one);
+    }
+  }
+  const int m = n == 7 ? 7 : 6;
+  const bool ordered = sizeof(T) == 4;
+  reg_plan(ordered ? reg_items_in_order(flat, vals) : reg_items(flat, vals, m), m, false, ordered, rp);
+  *fits = true;
+  return DM_OK;
+}
+
 size_t lds_bytes(int n, int dtype) {
   return ((size_t)1 << (2 * n)) * (dtype == DM_FP64 ? 8 : 4) + ((size_t)1 << n) * 8;
 }
@@ -3476,12 +3518,29 @@ template <typename T>
 int enqueue_batch(dm_batch *b) {
   HIP_TRY(hipEventRecord(b->fork, b->master));
   HIP_TRY(hipStreamWaitEvent(b->side, b->fork, 0));
-  // LDS tier on the side stream: one launch per width
+  // LDS tier on the side streams: the register-resident circuits, then one
+  // launch per width for the others
+  HIP_TRY(hipStreamWaitEvent(b->side2, b->fork, 0));
+  constexpr bool SEQ = sizeof(T) == 4;
+  const RegCirc *rc = static_cast<const RegCirc *>(b->d_rcircs);
+  const uint32_t *rrecs = static_cast<const uint32_t *>(b->d_rrecs);
+  const T *rvals = static_cast<const T *>(b->d_rvals);
+  if (b->nreg7) {
+    hipLaunchKernelGGL((k_circuit_reg<T, 7, SEQ>), dim3(b->nreg7), dim3(RegCircShape<7>::threads), 0, b->side2,
+                       rc + b->nreg6, rrecs, rvals, b->d_probs, b->d_stamps + 2 * (size_t)b->nreg6);
+    if (int rc2 = last_launch("k_circuit_reg")) return rc2;
+  }
+  if (b->nreg6) {
+    hipLaunchKernelGGL((k_circuit_reg<T, 6, SEQ>), dim3(b->nreg6), dim3(RegCircShape<6>::threads), 0, b->side, rc,
+                       rrecs, rvals, b->d_probs, b->d_stamps);
+    if (int rc2 = last_launch("k_circuit_reg")) return rc2;
+  }
+  const int reg = b->nreg6 + b->nreg7;
   for (int w = 1; w <= 7; ++w) {
     const int lo = b->small_width_start[w], hi = b->small_width_start[w + 1];
     if (hi <= lo) continue;
     hipLaunchKernelGGL((k_circuit_lds<T>), dim3(hi - lo), dim3(b->lds_threads), lds_bytes(w, b->dtype), b->side,
-                       static_cast<const BatchCirc *>(b->d_circs) + lo, static_cast<const TileOp *>(b->d_tops),
+                       static_cast<const BatchCirc *>(b->d_circs) + (lo - reg), static_cast<const TileOp *>(b->d_tops),
                        static_cast<const T *>(b->d_vals), b->d_probs, b->d_stamps + 2 * (size_t)lo);
     if (int rc = last_launch("k_circuit_lds")) return rc;
   }
@@ -3565,6 +3624,8 @@ int enqueue_batch(dm_batch *b) {
   }
   HIP_TRY(hipEventRecord(b->join, b->side));
   HIP_TRY(hipStreamWaitEvent(b->master, b->join, 0));
+  HIP_TRY(hipEventRecord(b->join2, b->side2));
+  HIP_TRY(hipStreamWaitEvent(b->master, b->join2, 0));
   return DM_OK;
 }
 
@@ -3599,12 +3660,66 @@ static int batch_create_t(dm_batch *b, const int64_t *op_start, const dm_op *ops
   std::vector<BatchCirc> circs;
   std::vector<TileOp> tops;
   std::vector<double> vals;
+  // register-resident: circuits of single-qubit maps, CX and memory noise,
+  // the longest first
+  std::vector<RegCirc> rcircs;
+  std::vector<uint32_t> rrecs;
+  std::vector<double> rvals;
+  std::vector<char> in_reg(b->ncirc, 0);
+  {
+    struct Planned {
+      int c;
+      RegPlan rp;
+    };
+    std::vector<Planned> planned[2];
+    for (int c = 0; c < b->ncirc; ++c) {
+      if (b->nq[c] > lds_max_qubits) continue;
+      Planned p;
+      p.c = c;
+      bool fits = false;
+      if (int rc = small_circuit_plan<T>(b->nq[c], ops + op_start[c], (int)(op_start[c + 1] - op_start[c]), params,
+                                         nparams, c, &fits, &p.rp))
+        return rc;
+      if (!fits) continue;
+      in_reg[c] = 1;
+      planned[b->nq[c] == 7].push_back(std::move(p));
+    }
+    for (auto &list : planned)
+      std::stable_sort(list.begin(), list.end(),
+                       [](const Planned &x, const Planned &y) { return x.rp.vals.size() > y.rp.vals.size(); });
+    b->nreg6 = (int)planned[0].size();
+    b->nreg7 = (int)planned[1].size();
+    for (auto &list : planned)
+      for (Planned &p : list) {
+        RegCirc rc;
+        memset(&rc, 0, sizeof(rc));
+        rc.n = b->nq[p.c];
+        rc.ns = p.rp.ns;
+        rc.st_off = (int64_t)rrecs.size();
+        rc.val_off = (int64_t)rvals.size();
+        rc.out_off = b->prob_off[p.c];
+        rc.err = b->err[p.c];
+        for (int j = 0; j < 3; ++j) {
+          rc.fr[j] = p.rp.first.r[j];
+          rc.fl[j] = p.rp.first.l[j];
+          rc.lr[j] = p.rp.last.r[j];
+          rc.ll[j] = p.rp.last.l[j];
+        }
+        rc.fw = p.rp.first.w;
+        rc.lw = p.rp.last.w;
+        rrecs.insert(rrecs.end(), p.rp.words.begin(), p.rp.words.end());
+        rvals.insert(rvals.end(), p.rp.vals.begin(), p.rp.vals.end());
+        rcircs.push_back(rc);
+        b->small.push_back(p.c);
+      }
+    b->launches += (b->nreg6 > 0) + (b->nreg7 > 0);
+  }
   b->small_width_start.assign(9, 0);
   for (int w = 1; w <= 7; ++w) {
     b->small_width_start[w] = (int)b->small.size();
     if (w > lds_max_qubits) continue;
     for (int c = 0; c < b->ncirc; ++c) {
-      if (b->nq[c] != w) continue;
+      if (b->nq[c] != w || in_reg[c]) continue;
       BatchCirc bc;
       bc.n = w;
       bc.op_off = (int64_t)tops.size();
@@ -3772,6 +3887,8 @@ static int batch_create_t(dm_batch *b, const int64_t *op_start, const dm_op *ops
   HIP_TRY(hipStreamCreateWithFlags(&b->side, hipStreamNonBlocking));
   HIP_TRY(hipEventCreateWithFlags(&b->fork, hipEventDisableTiming));
   HIP_TRY(hipEventCreateWithFlags(&b->join, hipEventDisableTiming));
+  HIP_TRY(hipStreamCreateWithFlags(&b->side2, hipStreamNonBlocking));
+  HIP_TRY(hipEventCreateWithFlags(&b->join2, hipEventDisableTiming));
   HIP_TRY(hipStreamCreateWithFlags(&b->side6, hipStreamNonBlocking));
   HIP_TRY(hipStreamCreateWithFlags(&b->side7, hipStreamNonBlocking));
   HIP_TRY(hipEventCreateWithFlags(&b->forkr, hipEventDisableTiming));
@@ -3784,6 +3901,12 @@ static int batch_create_t(dm_batch *b, const int64_t *op_start, const dm_op *ops
     if (bytes) HIP_TRY(hipMemcpy(*dst, src, bytes, hipMemcpyHostToDevice));
     return DM_OK;
   };
+  if (!rcircs.empty()) {
+    std::vector<T> tv(rvals.begin(), rvals.end());
+    if (int rc = upload(&b->d_rcircs, rcircs.data(), rcircs.size() * sizeof(RegCirc))) return rc;
+    if (int rc = upload(&b->d_rrecs, rrecs.data(), rrecs.size() * 4)) return rc;
+    if (int rc = upload(&b->d_rvals, tv.data(), tv.size() * sizeof(T))) return rc;
+  }
   if (!circs.empty()) {
     std::vector<T> tv(vals.begin(), vals.end());
     if (int rc = upload(&b->d_circs, circs.data(), circs.size() * sizeof(BatchCirc))) return rc;
@@ -4181,16 +4304,17 @@ int dm_batch_destroy(dm_batch *b) {
   if (!b) return DM_OK;
   if (b->master) hipStreamSynchronize(b->master);
   if (b->side) hipStreamSynchronize(b->side);
+  if (b->side2) hipStreamSynchronize(b->side2);
   if (b->side6) hipStreamSynchronize(b->side6);
   if (b->side7) hipStreamSynchronize(b->side7);
   if (b->exec) hipGraphExecDestroy(b->exec);
   if (b->graph) hipGraphDestroy(b->graph);
   for (void *p : {b->d_circs, b->d_tops, b->d_vals, b->d_arena, b->d_passes, b->d_items, b->d_qtops, b->d_qvals, b->d_recs,
-                  (void *)b->d_probs, (void *)b->d_stamps})
+                  b->d_rcircs, b->d_rrecs, b->d_rvals, (void *)b->d_probs, (void *)b->d_stamps})
     if (p) hipFree(p);
-  for (hipEvent_t e : {b->fork, b->join, b->ev0, b->ev1, b->forkr, b->join6, b->join7})
+  for (hipEvent_t e : {b->fork, b->join, b->join2, b->ev0, b->ev1, b->forkr, b->join6, b->join7})
     if (e) hipEventDestroy(e);
-  for (hipStream_t st : {b->side, b->side6, b->side7, b->master})
+  for (hipStream_t st : {b->side, b->side2, b->side6, b->side7, b->master})
     if (st) hipStreamDestroy(st);
   delete b;
   return DM_OK;

@@ -57,7 +57,9 @@ __device__ __forceinline__ double reg_fma(double a, double x, double c) {
   return r;
 }
 
-template <typename T, int SLOT, bool AFF>
+// SEQ: products and sums rounded one by one, as k_circuit_lds does; otherwise
+// fused multiply-adds, as the tile kernels.
+template <typename T, int SLOT, bool AFF, bool SEQ>
 __device__ __forceinline__ void reg_1q(T (&v)[64], const T (&pv)[kRegVals]) {
   constexpr int S = 1 << (2 * SLOT);
   constexpr int C = AFF ? 4 : 3;
@@ -71,6 +73,16 @@ __device__ __forceinline__ void reg_1q(T (&v)[64], const T (&pv)[kRegVals]) {
     const int b = SLOT == 0 ? 4 * o : SLOT == 1 ? (o & 3) + 16 * (o >> 2) : o;
     const T x0 = v[b], x1 = v[b + S], x2 = v[b + 2 * S], x3 = v[b + 3 * S];
     T t[3];
+    if constexpr (SEQ) {
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        const T *q = &r[i][AFF ? 1 : 0];
+        t[i] = (AFF ? r[i][0] * x0 + q[0] * x1 : q[0] * x1) + q[1] * x2 + q[2] * x3;
+      }
+#pragma unroll
+      for (int i = 0; i < 3; ++i) v[b + (i + 1) * S] = t[i];
+      continue;
+    }
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
       const T *q = &r[i][AFF ? 1 : 0];
@@ -137,7 +149,7 @@ __device__ __forceinline__ void reg_d2(T (&v)[64], const T (&pv)[kRegVals]) {
 
 // The members of a stage in order.  The next member's kind and values are
 // loaded (scalar loads) while the current one computes.
-template <typename T>
+template <typename T, bool SEQ>
 __device__ __forceinline__ void reg_members(T (&v)[64], const uint32_t *__restrict__ kinds, uint32_t nm,
                                             const T *__restrict__ prm) {
   if (nm == 0) return;
@@ -160,12 +172,12 @@ __device__ __forceinline__ void reg_members(T (&v)[64], const uint32_t *__restri
     for (int i = 0; i < kRegVals; ++i) next[i] = prm[i];
     __builtin_amdgcn_sched_barrier(0);
     switch (kind) {
-      case RM_U1 + 0: reg_1q<T, 0, false>(v, pv); break;
-      case RM_U1 + 1: reg_1q<T, 1, false>(v, pv); break;
-      case RM_U1 + 2: reg_1q<T, 2, false>(v, pv); break;
-      case RM_A1 + 0: reg_1q<T, 0, true>(v, pv); break;
-      case RM_A1 + 1: reg_1q<T, 1, true>(v, pv); break;
-      case RM_A1 + 2: reg_1q<T, 2, true>(v, pv); break;
+      case RM_U1 + 0: reg_1q<T, 0, false, SEQ>(v, pv); break;
+      case RM_U1 + 1: reg_1q<T, 1, false, SEQ>(v, pv); break;
+      case RM_U1 + 2: reg_1q<T, 2, false, SEQ>(v, pv); break;
+      case RM_A1 + 0: reg_1q<T, 0, true, SEQ>(v, pv); break;
+      case RM_A1 + 1: reg_1q<T, 1, true, SEQ>(v, pv); break;
+      case RM_A1 + 2: reg_1q<T, 2, true, SEQ>(v, pv); break;
       case RM_CX + 0: reg_cx<T, 0, 1>(v); break;
       case RM_CX + 1: reg_cx<T, 1, 0>(v); break;
       case RM_CX + 2: reg_cx<T, 0, 2>(v); break;
@@ -186,10 +198,11 @@ __device__ __forceinline__ void reg_members(T (&v)[64], const uint32_t *__restri
 // digit in SLOT (a register digit before and after) lies in the h-th part of
 // its range, from and into the same registers, so that a phase needs only
 // 1/PH of the tile's bytes of LDS and several workgroups fit a CU.
-template <typename T, int SLOT, int PH>
+template <typename T, int M, int SLOT, int PH>
 __device__ __forceinline__ void reg_exchange(T (&v)[64], T *s, const RegStage &st, int lane, int wave) {
   constexpr int S = 1 << (2 * SLOT);
   constexpr int IN = 4 / PH;  // digit values per phase
+  constexpr uint32_t PART = 1u << (2 * (M - 1));  // coefficients of one digit value
   const uint32_t l0 = lane & 3, l1 = (lane >> 2) & 3, l2 = lane >> 4;
   constexpr uint32_t B = sizeof(T);
   const uint32_t tw = ((l0 * st.wl[0]) ^ (l1 * st.wl[1]) ^ (l2 * st.wl[2]) ^ ((uint32_t)wave * st.ww)) * B;
@@ -204,7 +217,7 @@ __device__ __forceinline__ void reg_exchange(T (&v)[64], T *s, const RegStage &s
       const int d = (i / S) & 3;
       if (d / IN != h) continue;
       const uint32_t o = ((((i >> (2 * SA)) & 3) * st.wr[SA]) ^ (((i >> (2 * SB)) & 3) * st.wr[SB])) * B;
-      *reinterpret_cast<T *>(c + (tw ^ o) + (d % IN) * 4096 * B) = v[i];
+      *reinterpret_cast<T *>(c + (tw ^ o) + (d % IN) * PART * B) = v[i];
     }
     __syncthreads();
 #pragma unroll
@@ -212,7 +225,7 @@ __device__ __forceinline__ void reg_exchange(T (&v)[64], T *s, const RegStage &s
       const int d = (i / S) & 3;
       if (d / IN != h) continue;
       const uint32_t o = ((((i >> (2 * SA)) & 3) * st.rr[SA]) ^ (((i >> (2 * SB)) & 3) * st.rr[SB])) * B;
-      v[i] = *reinterpret_cast<const T *>(c + (tr ^ o) + (d % IN) * 4096 * B);
+      v[i] = *reinterpret_cast<const T *>(c + (tr ^ o) + (d % IN) * PART * B);
     }
   }
 }
@@ -235,6 +248,22 @@ struct RegShape {
   static constexpr int phases = sizeof(T) == 4 ? 2 : 4;
   static constexpr int lds = (1 << (2 * kRegTile)) / phases;  // coefficients
 };
+
+// The stages of a program on the tile in v (the first one's layout).
+template <typename T, int M, int PH, bool SEQ>
+__device__ __forceinline__ void reg_stages(T (&v)[64], T *s, const RegStage *__restrict__ st, int ns,
+                                           const uint32_t *__restrict__ kinds, const T *__restrict__ prm, int lane,
+                                           int wave) {
+  for (int k = 0; k < ns; ++k) {
+    const RegStage sg = st[k];
+    if (k) {
+      if (sg.slot == 0) reg_exchange<T, M, 0, PH>(v, s, sg, lane, wave);
+      else if (sg.slot == 1) reg_exchange<T, M, 1, PH>(v, s, sg, lane, wave);
+      else reg_exchange<T, M, 2, PH>(v, s, sg, lane, wave);
+    }
+    reg_members<T, SEQ>(v, kinds + sg.mem, sg.nm, prm + (size_t)sg.mem * kRegVals);
+  }
+}
 
 template <typename T, bool NTM>
 __device__ __forceinline__ void reg_tile(T *__restrict__ a, T *s, const RegGeom &geo, uint32_t tile,
@@ -259,15 +288,7 @@ __device__ __forceinline__ void reg_tile(T *__restrict__ a, T *s, const RegGeom 
     for (int i = 0; i < 64; ++i)
       v[i] = reg_load<T, NTM>(p + (i & 3) * geo.is[0] + ((i >> 2) & 3) * geo.is[1] + (i >> 4) * geo.is[2], loff);
   }
-  for (int k = 0; k < ns; ++k) {
-    const RegStage sg = st[k];
-    if (k) {
-      if (sg.slot == 0) reg_exchange<T, 0, PH>(v, s, sg, lane, wave);
-      else if (sg.slot == 1) reg_exchange<T, 1, PH>(v, s, sg, lane, wave);
-      else reg_exchange<T, 2, PH>(v, s, sg, lane, wave);
-    }
-    reg_members<T>(v, kinds + sg.mem, sg.nm, prm + (size_t)sg.mem * kRegVals);
-  }
+  reg_stages<T, kRegTile, PH, false>(v, s, st, ns, kinds, prm, lane, wave);
   {
     T *p = a + base + wave * geo.ow;
 #pragma unroll
@@ -284,6 +305,90 @@ __global__ __launch_bounds__(kRegThreads, sizeof(T) == 4 ? 4 : 2) void k_tile_re
   __shared__ __align__(16) T s[RegShape<T>::lds];
   if (blockIdx.x >= geo.tiles) return;  // uniform over the workgroup
   reg_tile<T, NTM>(a, s, geo, blockIdx.x, st, ns, kinds, prm);
+}
+
+// A whole circuit of up to M qubits (6: one wave; 7: four) in registers, from
+// |0...0> to the Z-ensemble probabilities: its program is one list of stages.
+// Qubits fewer than 6 leave digits that no operation touches; only their
+// component 0 is initialised and read.  What bounds it is one circuit's
+// serial chain of members and redistributions: a circuit is one workgroup.
+// 512 circuits of 2-7 qubits and 50-300 gates, memory noise after every gate,
+// FP64: 8.2 ms one workgroup a circuit in LDS (an LDS round trip per gate and
+// per qubit's noise, the widths one after another) -> 0.62 ms.
+struct RegCirc {
+  int32_t n, ns;
+  int64_t st_off;   // first record word
+  int64_t val_off;  // first value
+  int64_t out_off;  // first probability
+  double err;       // measurement polarisation retention
+  // digits of the register slots, lanes and waves in the first and the last
+  // stage's layout
+  int32_t fr[3], fl[3], fw, lr[3], ll[3], lw;
+};
+
+template <int M>
+struct RegCircShape {
+  static constexpr int threads = M == 7 ? 256 : 64;
+  static constexpr int phases = 2;
+};
+
+template <typename T, int M, bool SEQ>
+__global__ __launch_bounds__(RegCircShape<M>::threads, 2) void k_circuit_reg(const RegCirc *__restrict__ circs,
+                                                                             const uint32_t *__restrict__ recs,
+                                                                             const T *__restrict__ prm,
+                                                                             double *__restrict__ probs,
+                                                                             uint64_t *__restrict__ stamps) {
+  constexpr int PH = RegCircShape<M>::phases;
+  constexpr int NT = RegCircShape<M>::threads;
+  __shared__ __align__(16) T s[(1 << (2 * M)) / PH];
+  const RegCirc c = circs[blockIdx.x];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = M == 7 ? __builtin_amdgcn_readfirstlane(tid >> 6) : 0;
+  if (tid == 0) stamps[2 * blockIdx.x] = wall_clock64();
+  const RegStage *st = reinterpret_cast<const RegStage *>(recs + c.st_off);
+  // components of a digit with a value: I and Z of a qubit, 0 of the others
+  auto ok = [&](int digit, int x) { return ((digit < c.n ? 9 : 1) >> x) & 1; };
+  auto lanes_ok = [&](const int32_t *l, int32_t w) {
+    return ok(l[0], lane & 3) && ok(l[1], (lane >> 2) & 3) && ok(l[2], lane >> 4) && (M != 7 || ok(w, wave));
+  };
+  T v[64];
+  {
+    const T amp = lanes_ok(c.fl, c.fw) ? (T)ldexp(1.0, -c.n) : T(0);
+#pragma unroll
+    for (int i = 0; i < 64; ++i)
+      v[i] = ok(c.fr[0], i & 3) && ok(c.fr[1], (i >> 2) & 3) && ok(c.fr[2], i >> 4) ? amp : T(0);
+  }
+  reg_stages<T, M, PH, SEQ>(v, s, st, c.ns, reinterpret_cast<const uint32_t *>(st + c.ns), prm + c.val_off, lane,
+                            wave);
+  __syncthreads();  // the last redistribution has been read
+  // Z ensemble: bit q of an index is the I / Z choice of digit q (qubit
+  // n-1-q), which is the order of the outcomes too
+  double *z = reinterpret_cast<double *>(s);
+  if (lanes_ok(c.ll, c.lw)) {
+    const int hi = ((lane & 3) ? 1 << c.ll[0] : 0) | ((lane & 12) ? 1 << c.ll[1] : 0) |
+                   ((lane & 48) ? 1 << c.ll[2] : 0) | (M == 7 && wave ? 1 << c.lw : 0);
+#pragma unroll
+    for (int i = 0; i < 64; ++i)
+      if ((i & 3) % 3 == 0 && ((i >> 2) & 3) % 3 == 0 && (i >> 4) % 3 == 0)
+        if (ok(c.lr[0], i & 3) && ok(c.lr[1], (i >> 2) & 3) && ok(c.lr[2], i >> 4))
+          z[hi | ((i & 3) ? 1 << c.lr[0] : 0) | ((i & 12) ? 1 << c.lr[1] : 0) | ((i & 48) ? 1 << c.lr[2] : 0)] =
+              (double)v[i];
+  }
+  __syncthreads();
+  const int nv = 1 << c.n;
+  for (int q = 0; q < c.n; ++q) {  // butterfly on bit q: (u, w) -> (u + e w, u - e w)
+    for (int x = tid; x < nv / 2; x += NT) {
+      const int lo = x & ((1 << q) - 1);
+      const int b = ((x >> q) << (q + 1)) | lo;
+      const double u = z[b], w = z[b | (1 << q)];
+      z[b] = u + c.err * w;
+      z[b | (1 << q)] = u - c.err * w;
+    }
+    __syncthreads();
+  }
+  for (int x = tid; x < nv; x += NT) probs[c.out_off + x] = z[x];
+  if (tid == 0) stamps[2 * blockIdx.x + 1] = wall_clock64();
 }
 
 // ---------------------------------------------------------------------------
@@ -475,9 +580,13 @@ inline int reg_absorb(const std::vector<RegItem> &items, const std::vector<char>
   return n;
 }
 
+struct RegLay {
+  int r[3], l[3], w, slot;  // register, lane and wave digits, slot that orders the phases
+};
+
 struct RegPlan {
-  RegGeom geo;
   int ns = 0;
+  RegLay first, last;           // layouts of the first and the last stage
   std::vector<uint32_t> words;  // RegStage records, then the members' kinds and one spare
   std::vector<double> vals;     // kRegVals values a member, and one spare block
 };
@@ -488,12 +597,11 @@ struct RegPlan {
 // least one: an item's digits and one kept from the stage before), and
 // a last, possibly empty one on a layout that stores directly.  With
 // `ordered` the operations keep their order (see reg_absorb).
-inline void reg_plan(const std::vector<TileOp> &ops, const std::vector<double> &vals, const int *tpos, const int *rpos,
-                     int nr, bool ordered, RegPlan *out) {
-  constexpr int m = kRegTile;
-  const std::vector<RegItem> items = ordered ? reg_items_in_order(ops, vals) : reg_items(ops, vals, m);
+// `io`: a tile of a state; otherwise (a whole circuit) any layout may come
+// first and last.  m digits (6: no wave digit).
+inline void reg_plan(const std::vector<RegItem> &items, int m, bool io, bool ordered, RegPlan *out) {
   uint32_t triples[35], nt = 0;
-  for (int a = 3; a < m; ++a)  // the 4 load / store layouts first
+  for (int a = 3; a < m; ++a)  // the 4 load / store layouts of 7 digits first
     for (int b = a + 1; b < m; ++b)
       for (int c = b + 1; c < m; ++c) triples[nt++] = (1u << a) | (1u << b) | (1u << c);
   const uint32_t nio = nt;
@@ -507,8 +615,10 @@ inline void reg_plan(const std::vector<TileOp> &ops, const std::vector<double> &
   while (left || stage.empty()) {
     uint32_t best = 0;
     int most = -1;
-    for (uint32_t t = 0; t < (stage.empty() ? nio : nt); ++t) {
+    for (uint32_t t = 0; t < (io && stage.empty() ? nio : nt); ++t) {
       if (!stage.empty() && !(triples[t] & stage.back())) continue;  // a redistribution keeps one digit
+      // in order, the first pending item comes first
+      if (ordered && left && !(io && stage.empty()) && (items[first].mask & ~triples[t])) continue;
       const int n = reg_absorb(items, done, first, triples[t], ordered, nullptr);
       if (n > most) {
         most = n;
@@ -523,7 +633,7 @@ inline void reg_plan(const std::vector<TileOp> &ops, const std::vector<double> &
     stage.push_back(triples[best]);
     members.push_back(std::move(take));
   }
-  if (stage.back() & 7u) {  // an empty stage that stores directly
+  if (io && (stage.back() & 7u)) {  // an empty stage that stores directly
     const uint32_t last = stage.back();
     uint32_t best = nio;
     for (uint32_t t = 0; t < nio; ++t)
@@ -539,12 +649,9 @@ inline void reg_plan(const std::vector<TileOp> &ops, const std::vector<double> &
     members.emplace_back();
   }
   const int ns = (int)stage.size();
-  struct Lay {
-    int r[3], l[3], w, slot;
-  };
-  std::vector<Lay> lay(ns);
+  std::vector<RegLay> lay(ns);
   for (int k = 0; k < ns; ++k) {
-    Lay &y = lay[k];
+    RegLay &y = lay[k];
     int reg[3], nreg = 0, rest[4], nrest = 0;
     for (int d = 0; d < m; ++d) {
       if ((stage[k] >> d) & 1) reg[nreg++] = d;
@@ -576,7 +683,7 @@ inline void reg_plan(const std::vector<TileOp> &ops, const std::vector<double> &
     // highest of the others
     for (int j = 0; j < 3; ++j) y.l[j] = -1;
     bool used[8] = {false};
-    for (int x = 0; x < 4; ++x)
+    for (int x = 0; x < nrest; ++x)
       if (rest[x] < 3) {
         y.l[rest[x]] = rest[x];
         used[rest[x]] = true;
@@ -596,19 +703,12 @@ inline void reg_plan(const std::vector<TileOp> &ops, const std::vector<double> &
         y.l[j] = rest[x];
         used[rest[x]] = true;
       }
-    for (int q = 0; q < 4; ++q)
+    y.w = m;  // (no wave digit)
+    for (int q = 0; q < nrest; ++q)
       if (!used[rest[q]]) y.w = rest[q];
   }
-  memset(&out->geo, 0, sizeof(out->geo));
-  out->geo.nr = nr;
-  for (int j = 0; j < nr; ++j) out->geo.rpos[j] = rpos[j];
-  out->geo.tiles = 1u << (2 * nr);
-  for (int j = 0; j < 3; ++j) {
-    out->geo.is[j] = pow4(tpos[lay[0].r[j]]);
-    out->geo.os[j] = pow4(tpos[lay[ns - 1].r[j]]);
-  }
-  out->geo.iw = pow4(tpos[lay[0].w]);
-  out->geo.ow = pow4(tpos[lay[ns - 1].w]);
+  out->first = lay[0];
+  out->last = lay[ns - 1];
   out->ns = ns;
   out->words.clear();
   out->vals.clear();
@@ -653,7 +753,7 @@ inline void reg_plan(const std::vector<TileOp> &ops, const std::vector<double> &
       // to the place of one that is no lane of the reader, so that the lanes of a wave fall on
       // distinct banks on both sides.  Every digit but the writer's lanes
       // and the phase digit also has a place of its own above them.
-      const Lay &w = lay[k - 1], &y = lay[k];
+      const RegLay &w = lay[k - 1], &y = lay[k];
       uint32_t co[8] = {0};
       for (int j = 0; j < 3; ++j) co[w.l[j]] = 1u << (2 * j);
       int high = 3;
@@ -686,4 +786,20 @@ inline void reg_plan(const std::vector<TileOp> &ops, const std::vector<double> &
   kinds.push_back(0);
   out->words.insert(out->words.end(), kinds.begin(), kinds.end());
   out->vals.resize(out->vals.size() + kRegVals, 0.0);
+}
+
+// HBM strides of a tile's load and store layouts.
+inline RegGeom reg_geom(const RegPlan &rp, const int *tpos, const int *rpos, int nr) {
+  RegGeom geo;
+  memset(&geo, 0, sizeof(geo));
+  geo.nr = nr;
+  for (int j = 0; j < nr; ++j) geo.rpos[j] = rpos[j];
+  geo.tiles = 1u << (2 * nr);
+  for (int j = 0; j < 3; ++j) {
+    geo.is[j] = pow4(tpos[rp.first.r[j]]);
+    geo.os[j] = pow4(tpos[rp.last.r[j]]);
+  }
+  geo.iw = pow4(tpos[rp.first.w]);
+  geo.ow = pow4(tpos[rp.last.w]);
+  return geo;
 }

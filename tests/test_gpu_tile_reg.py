@@ -125,3 +125,93 @@ def test_every_pass_from_12_qubits(qubits, members, precision):
         assert np.abs(got - want).max() <= members * 8 * EPS[precision] * np.abs(a).max()
         return
     check(12, 7, qubits, members, precision, 7)
+
+
+def with_identity(sub, qubits):
+    """The same operations and an identity two-qubit map, which the
+    register-resident kernels leave to the tile-in-LDS form."""
+    return sub + [(native.SUB_2Q, list(qubits[:2]), np.eye(16))]
+
+
+@pytest.mark.parametrize('n,m,qubits', [(8, 7, [0, 2, 3, 7]), (9, 6, [0, 1, 4]), (12, 7, [0, 1, 10, 11])])
+def test_fp32_passes_equal_the_lds_form_bit_for_bit(n, m, qubits):
+    """FP32 keeps the order of operations: the state is the same whichever
+    form ran."""
+    rng = np.random.default_rng(n)
+    sub = []
+    for _ in range(40):
+        if rng.random() < 0.5:
+            R = random_map(rng, rng.choice(['unital', 'general', 'diag']))
+            sub.append((native.SUB_1Q, [int(rng.choice(qubits))], ptm.rows3(R)))
+        else:
+            c, t = (int(x) for x in rng.choice(qubits, 2, replace=False))
+            sub.append((native.SUB_CX, [c, t], random_scale(rng, rng.choice(['none', 'separable', 'general']))))
+    a = rng.normal(size=4 ** n) * 2.0 ** -n
+    got = []
+    for ops in (sub, with_identity(sub, qubits)):
+        prog = Program(n)
+        prog.fused(m, qubits, ops)
+        st = native.DeviceState(n, 'fp32')
+        st.upload(a)
+        prog.run(st)
+        got.append(st.download())
+        st.close()
+    assert np.array_equal(got[0], got[1])
+
+
+def small_circuit(rng, n, ngates, noise):
+    """(Program, the oracle's probabilities) of a random circuit with memory
+    noise after every gate, depolarising CX scales and a final measurement
+    with retention 0.97."""
+    prog = Program(n)
+    a = refsim.initial_state(n).reshape(-1)
+    for _ in range(ngates):
+        if n == 1 or rng.random() < 0.6:
+            q = int(rng.integers(n))
+            R = random_map(rng, rng.choice(['unital', 'general', 'diag']))
+            prog.one_qubit(q, R)
+            a = oracle_1q(a, n, q, R)
+        else:
+            c, t = (int(x) for x in rng.choice(n, 2, replace=False))
+            s = random_scale(rng, rng.choice(['none', 'separable', 'general']))
+            prog.cx(c, t, s)
+            a = oracle_cx(a, n, c, t, s)
+        if noise is not None:
+            prog.memory_noise(*noise)
+            a = refsim.apply_memory_noise(a.copy().reshape(n * [4]), n, *noise).reshape(-1)
+    x = a.reshape(n * [4])
+    for _ in range(n):
+        x = np.stack([x[0] + 0.97 * x[3], x[0] - 0.97 * x[3]], axis=-1)
+    return prog, x.reshape(-1)
+
+
+@pytest.mark.parametrize('noise', [None, (0.98, 0.8, 0.995), (0.98, 0.5, 1.0)])
+@pytest.mark.parametrize('precision,tol', [('fp64', 1e-12), ('fp32', 2e-5)])
+def test_whole_circuits_in_registers(precision, tol, noise):
+    """Registers of 1-7 qubits, programs of 0-60 gates (the batch tests'
+    tolerances: 1e-12 in FP64, 2e-5 in FP32)."""
+    from dmsim import batch
+    rng = np.random.default_rng(11)
+    cases = [(n, *small_circuit(rng, n, g, noise)) for n in range(1, 8) for g in (0, 1, 7, 60)]
+    b = batch.Batch([(n, prog, 0.97) for n, prog, _ in cases], precision, lds_max_qubits=7, lds_threads=256)
+    for graph in (False, True, True):
+        probs, us, _ = b.run(graph)
+        assert np.all(us > 0)
+        for (n, _, want), got in zip(cases, probs):
+            assert np.max(np.abs(got - want)) <= tol, n
+    b.close()
+
+
+def test_fp32_whole_circuits_equal_the_lds_kernel_bit_for_bit():
+    from dmsim import batch
+    rng = np.random.default_rng(3)
+    out = []
+    circuits = [(n, small_circuit(rng, n, 40, (0.98, 0.8, 0.995))[0], 0.97) for n in range(2, 8)]
+    for lds in (False, True):
+        if lds:  # an identity two-qubit map: whole circuits in LDS
+            for n, prog, _ in circuits:
+                prog.two_qubit(0, 1, np.eye(16))
+        b = batch.Batch(circuits, 'fp32', lds_max_qubits=7, lds_threads=256)
+        out.append(np.concatenate(b.run(False)[0]))
+        b.close()
+    assert np.array_equal(out[0], out[1])
