@@ -62,6 +62,21 @@ def zero_state(st, n):
     st.init_product(np.tile([1.0, 0.0, 0.0, 1.0], n), 0.5 ** n)
 
 
+class PlainProgram:
+    """One kernel per noisy gate: a program of its own for every gate (the
+    library fuses the single operations of one FP64 program)."""
+
+    def __init__(self, noisy, n):
+        self.programs = [fusion.plain_program([g], n) for g in noisy]
+
+    def __len__(self):
+        return len(self.programs)
+
+    def run(self, st):
+        for prog in self.programs:
+            prog.run(st)
+
+
 def time_program(prog, n, precision, steps, warmup, st=None):
     """Wall time of `steps` program applications (after `warmup`), with HIP
     event timing of every launch on the handle's stream.  With ``st`` given
@@ -258,7 +273,7 @@ def kernels_mode(args):
         st.close()
     st = native.DeviceState(n, 'fp64')
     zero_state(st, n)
-    fusion.plain_program(noisy[:60], n).run(st)
+    PlainProgram(noisy[:60], n).run(st)
     st.synchronize()
     st.close()
     return out
@@ -548,7 +563,7 @@ def headline(args):
     noisy = fusion.noisy_gates(gates, 1e-3)
 
     fused, blocks, method, plan_s = headline_plan(noisy, n, args.fusion)
-    plain = fusion.plain_program(noisy, n)
+    plain = PlainProgram(noisy, n)
     ks = [len(q) if len(m) > 1 else 0 for q, m in blocks]
     log('plan: %s, %d passes for %d gates (%.2f s host); k histogram %s'
         % (method, len(fused), G, plan_s, np.bincount(ks, minlength=6).tolist()))
@@ -559,7 +574,7 @@ def headline(args):
     log('timing plain fp64 (%d application(s)) ...' % args.plain_steps)
     st64 = native.DeviceState(n, 'fp64')
     zero_state(st64, n)
-    fusion.plain_program(noisy[:PLAIN_WARMUP_GATES], n).run(st64)
+    PlainProgram(noisy[:PLAIN_WARMUP_GATES], n).run(st64)
     zero_state(st64, n)
     t_plain, f_plain = time_program(plain, n, 'fp64', args.plain_steps, 0, st=st64)
     log('  %.3f s for %d application(s)' % (t_plain, args.plain_steps))

@@ -144,6 +144,9 @@ int dm_to_dense(dm_state *h, double *out_c128);
 
 /* A program: a list of operations executed back to back on the handle's
  * stream with one upload of all block matrices and no host synchronisation.
+ * On an FP64 state, consecutive DM_OP_1Q, DM_OP_CX[_SCALED] and
+ * DM_OP_MEMORY_NOISE operations run as fused passes where that is faster
+ * than one kernel each (same results to rounding).
  * Replaces the per-level dispatch loop of run_experiment (dm_simulator.py:
  * 1005-1177) for the unitary / channel part of a circuit.
  * Parameters of op i start at params[ops[i].param]:

@@ -1864,7 +1864,10 @@ struct FusedPass {
   std::vector<double> vals;    // values in kernel layout (FP64; converted at upload)
   bool reg = false;            // register-resident form (reg_geo, recs) instead of geo and ops
   RegGeom reg_geo;
+  bool whole = false;          // reg, on a whole state of up to 6 qubits (k_state_reg, reg_whole)
+  RegWhole reg_whole;
   int reg_stages = 0;
+  int plain = -1;              // stands for this operation of the program, run by its own kernel
   std::vector<uint32_t> recs;  // its device records: the stages, then the members' kinds
   // device records as 32-bit words
   size_t rec_words() const { return reg ? recs.size() : ops.size() * (sizeof(TileOp) / 4); }
@@ -1891,6 +1894,10 @@ struct dm_state {
   size_t red_cap = 0;           // doubles
   void *d_mat = nullptr;        // program image: tile-operation records, block matrices (storage dtype)
   size_t mat_cap = 0;           // bytes
+  void *h_img = nullptr;        // pinned copy of the image on its way to d_mat
+  size_t img_cap = 0;           // bytes
+  hipEvent_t img_ev = nullptr;  // that copy's end
+  bool img_busy = false;
   double *d_aux = nullptr;      // gathered vectors / overlap operand
   size_t aux_cap = 0;           // bytes
   // memory noise with a thermal feed as tile passes: the passes, and their
@@ -2620,6 +2627,43 @@ void group_stages(FusedPass *fp) {
   fp->ops.swap(out);
 }
 
+// A 7-digit tile: the given positions (at most 7) completed with the lowest
+// others.  False if the positions 0-2 are not all in it.
+struct RegTile {
+  int tpos[kRegTile], rpos[kMaxQubits], digit[kMaxQubits], nr;
+};
+
+bool reg_tile_of(int n, const int *pos, int count, RegTile *t) {
+  bool in[kMaxQubits] = {false};
+  for (int j = 0; j < count; ++j) in[pos[j]] = true;
+  for (int p = 0; p < n && count < kRegTile; ++p)
+    if (!in[p]) {
+      in[p] = true;
+      ++count;
+    }
+  if (!in[0] || !in[1] || !in[2]) return false;
+  int nt = 0;
+  t->nr = 0;
+  for (int p = 0; p < n; ++p) {
+    if (in[p]) {
+      t->digit[p] = nt;
+      t->tpos[nt++] = p;
+    } else {
+      t->rpos[t->nr++] = p;
+    }
+  }
+  return true;
+}
+
+void set_reg(FusedPass *fp, RegPlan &&rp, const RegTile &t) {
+  fp->reg = true;
+  fp->reg_geo = reg_geom(rp, t.tpos, t.rpos, t.nr);
+  fp->reg_stages = rp.ns;
+  fp->recs = std::move(rp.words);
+  fp->vals = std::move(rp.vals);
+  fp->ops.clear();
+}
+
 // The register-resident form (k_tile_reg) of a parsed pass, its tile
 // completed to 7 digits with the lowest other positions, where that is the
 // faster one; false leaves the pass as it is.  It takes single-qubit and CX
@@ -2641,24 +2685,8 @@ bool plan_reg(const dm_state *h, FusedPass *fp) {
   if (few && fp->ops.size() < 12) return false;
   for (const TileOp &op : fp->ops)
     if (op.kind != TOP_1Q && op.kind != TOP_CX) return false;
-  bool in[kMaxQubits] = {false};
-  for (int j = 0; j < fp->m; ++j) in[fp->geo.tpos[j]] = true;
-  int count = fp->m;
-  for (int pos = 0; pos < h->n && count < kRegTile; ++pos)
-    if (!in[pos]) {
-      in[pos] = true;
-      ++count;
-    }
-  if (!in[0] || !in[1] || !in[2]) return false;
-  int tpos[kRegTile], rpos[kMaxQubits], digit[kMaxQubits], nt = 0, nr = 0;
-  for (int pos = 0; pos < h->n; ++pos) {
-    if (in[pos]) {
-      digit[pos] = nt;
-      tpos[nt++] = pos;
-    } else {
-      rpos[nr++] = pos;
-    }
-  }
+  RegTile t;
+  if (!reg_tile_of(h->n, fp->geo.tpos, fp->m, &t)) return false;
   // FP32 keeps the order of operations of the tile-in-LDS form, and with it
   // every rounding: a state does not depend on which form ran.  FP64 may
   // reorder what commutes (differences of 1e-15).
@@ -2678,17 +2706,176 @@ bool plan_reg(const dm_state *h, FusedPass *fp) {
     vals = fp->vals;
   }
   for (TileOp &op : ops)
-    for (int x = 0; x < (op.kind == TOP_CX ? 2 : 1); ++x) op.d[x] = digit[fp->geo.tpos[op.d[x]]];
+    for (int x = 0; x < (op.kind == TOP_CX ? 2 : 1); ++x) op.d[x] = t.digit[fp->geo.tpos[op.d[x]]];
   RegPlan rp;
   reg_plan(ordered ? reg_items_in_order(ops, vals) : reg_items(ops, vals, kRegTile), kRegTile, true, ordered, &rp);
   if (few && ops.size() < 4 * (size_t)rp.ns) return false;
-  fp->reg = true;
-  fp->reg_geo = reg_geom(rp, tpos, rpos, nr);
-  fp->reg_stages = rp.ns;
-  fp->recs = std::move(rp.words);
-  fp->vals = std::move(rp.vals);
-  fp->ops.clear();
+  set_reg(fp, std::move(rp), t);
   return true;
+}
+
+// Runs of single-qubit, CX and memory-noise operations of a program on an
+// FP64 state as fused passes (an FP32 state keeps one kernel per operation:
+// its kernels round differently).
+struct PlainRun {
+  std::vector<TileOp> ops;      // digits are positions
+  std::vector<double> vals;
+  std::vector<int> src;         // program operation of each
+};
+
+bool plain_op(const dm_op &op) {
+  return op.kind == DM_OP_1Q || op.kind == DM_OP_CX || op.kind == DM_OP_CX_SCALED || op.kind == DM_OP_MEMORY_NOISE;
+}
+
+void add_plain(int n, const dm_op &op, const double *params, int src, PlainRun *run) {
+  TileOp t;
+  memset(&t, 0, sizeof(t));
+  t.param = (int32_t)run->vals.size();
+  auto put = [&](const double *v, int nv) { run->vals.insert(run->vals.end(), v, v + nv); };
+  const double *pv = params + op.param;
+  if (op.kind == DM_OP_MEMORY_NOISE) {
+    const double f = pv[0], p = pv[1], g = pv[2];
+    if (f == 1.0 && g == 1.0) return;
+    const double od = sqrt(g) * f, dd = (1 - g) * (2 * p - 1);
+    const double R[12] = {0, od, 0, 0, 0, 0, od, 0, dd, 0, 0, g};
+    put(R, 12);
+    t.kind = TOP_1Q;
+    t.k = 1;
+    for (int d = 0; d < n; ++d) {
+      t.d[0] = d;
+      run->ops.push_back(t);
+      run->src.push_back(src);
+    }
+    return;
+  }
+  t.d[0] = n - 1 - op.qubits[0];
+  if (op.kind == DM_OP_1Q) {
+    t.kind = TOP_1Q;
+    t.k = 1;
+    put(pv, 12);
+  } else {
+    t.kind = TOP_CX;
+    t.d[1] = n - 1 - op.qubits[1];
+    t.k = op.kind == DM_OP_CX_SCALED ? 1 : 0;
+    if (t.k) put(pv, 16);
+  }
+  run->ops.push_back(t);
+  run->src.push_back(src);
+}
+
+// Blocks of the run: the operations that the tile of the positions 0-2 and
+// up to four others takes (an operation joins unless it, or an earlier one
+// left out that shares a position with it, reaches outside), the others
+// chosen by growth from the first pending operation, with and without one
+// position forced in, whichever takes the most operations.
+std::vector<std::vector<int>> plain_blocks(int n, const PlainRun &run) {
+  const int no = (int)run.ops.size();
+  std::vector<uint32_t> mask(no);
+  for (int i = 0; i < no; ++i) {
+    mask[i] = 1u << run.ops[i].d[0];
+    if (run.ops[i].kind == TOP_CX) mask[i] |= 1u << run.ops[i].d[1];
+  }
+  const uint32_t low = 7u, full = (1u << n) - 1u;
+  const int most_high = std::min(4, n - 3);
+  std::vector<char> done(no, 0);
+  std::vector<std::vector<int>> out;
+  int first = 0, left = no;
+  std::vector<int> cur, best;
+  while (left) {
+    while (done[first]) ++first;
+    best.clear();
+    for (int force = -1; force < n; ++force) {
+      if (force >= 0 && force < 3) continue;
+      uint32_t T = force < 0 ? 0 : 1u << force, blocked = 0;
+      cur.clear();
+      for (int i = first; i < no; ++i) {
+        if (done[i]) continue;
+        const uint32_t m = mask[i], t2 = T | (m & ~low);
+        if ((m & blocked) || __builtin_popcount(t2) > most_high) {
+          blocked |= m;
+          const uint32_t open = __builtin_popcount(T) < most_high ? full : T | low;
+          if (!(open & ~blocked)) break;
+        } else {
+          T = t2;
+          cur.push_back(i);
+        }
+      }
+      if (cur.size() > best.size()) best = cur;
+    }
+    for (int i : best) done[i] = 1;
+    left -= (int)best.size();
+    out.push_back(best);
+  }
+  return out;
+}
+
+// The passes that replace the run, or none if one kernel per operation is
+// expected to be as fast.  Kernels of 3-5 us below 12 qubits, the passes
+// 9-20; from 12 qubits on a pass takes 1.0-1.4 times the kernels' time.
+template <typename T>
+std::vector<FusedPass> fuse_plain_run(const dm_state *h, const PlainRun &run, const dm_op *ops, const double *params) {
+  std::vector<FusedPass> out;
+  const int n = h->n;
+  if (run.ops.size() < 2 || n > 18) return out;
+  if (n <= 6) {
+    RegPlan rp;
+    reg_plan(reg_items(run.ops, run.vals, 6), 6, false, false, &rp);
+    FusedPass fp;
+    fp.reg = fp.whole = true;
+    memset(&fp.reg_whole, 0, sizeof(fp.reg_whole));
+    fp.reg_whole.n = n;
+    fp.reg_whole.ns = rp.ns;
+    for (int j = 0; j < 3; ++j) {
+      fp.reg_whole.fr[j] = rp.first.r[j];
+      fp.reg_whole.fl[j] = rp.first.l[j];
+      fp.reg_whole.lr[j] = rp.last.r[j];
+      fp.reg_whole.ll[j] = rp.last.l[j];
+    }
+    fp.reg_stages = rp.ns;
+    fp.recs = std::move(rp.words);
+    fp.vals = std::move(rp.vals);
+    out.push_back(std::move(fp));
+    return out;
+  }
+  // kernels of the run one by one
+  double kernels = 0.0;
+  int last = -1;
+  for (int i : run.src) {
+    if (i == last) continue;
+    last = i;
+    const double *pv = params + ops[i].param;
+    const bool feed = ops[i].kind == DM_OP_MEMORY_NOISE && (1 - pv[2]) * (2 * pv[1] - 1) != 0.0;
+    kernels += !feed ? 1 : n >= 12 ? 1 + (n - 4) / 4 : 1 + (n - 4) / 3;
+  }
+  const std::vector<std::vector<int>> blocks = plain_blocks(n, run);
+  if (blocks.size() * (n < 12 ? 2.0 : 1.4) >= kernels) return out;
+  for (const std::vector<int> &b : blocks) {
+    FusedPass fp;
+    if (b.size() == 1 && ops[run.src[b[0]]].kind != DM_OP_MEMORY_NOISE) {
+      fp.plain = run.src[b[0]];  // its own kernel
+      out.push_back(std::move(fp));
+      continue;
+    }
+    int tpos[kRegTile], count = 0;
+    uint32_t used = 7u;
+    for (int i : b) used |= (1u << run.ops[i].d[0]) | (run.ops[i].kind == TOP_CX ? 1u << run.ops[i].d[1] : 0u);
+    for (int pos = 0; pos < n; ++pos)
+      if ((used >> pos) & 1) tpos[count++] = pos;
+    RegTile t;
+    reg_tile_of(n, tpos, count, &t);
+    std::vector<TileOp> tops;
+    for (int i : b) {
+      TileOp op = run.ops[i];
+      op.d[0] = t.digit[op.d[0]];
+      if (op.kind == TOP_CX) op.d[1] = t.digit[op.d[1]];
+      tops.push_back(op);
+    }
+    RegPlan rp;
+    reg_plan(reg_items(tops, run.vals, kRegTile), kRegTile, true, false, &rp);
+    set_reg(&fp, std::move(rp), t);
+    out.push_back(std::move(fp));
+  }
+  return out;
 }
 
 int parse_fused(const dm_state *h, const double *p, int64_t avail, int opi, FusedPass *fp, bool allow_reg = false) {
@@ -2904,6 +3091,11 @@ int launch_fused(dm_state *h, const FusedPass &fp, const uint32_t *d_recs, const
   if (fp.reg) {
     const RegStage *st = reinterpret_cast<const RegStage *>(d_recs);
     const uint32_t *mem = reinterpret_cast<const uint32_t *>(st + fp.reg_stages);
+    if (fp.whole) {
+      hipLaunchKernelGGL((k_state_reg<T>), dim3(1), dim3(64), 0, h->stream, static_cast<T *>(h->d_a), fp.reg_whole, st,
+                         mem, d_vals);
+      return last_launch("k_state_reg");
+    }
     // states above the 256 MB of the last-level cache stream with
     // nontemporal accesses (16 qubits, FP32: 6.0 against 6.4 ms a pass), the
     // others stay in it from pass to pass with plain ones (13 qubits, FP32,
@@ -3096,24 +3288,58 @@ struct Prepared {
 };
 
 template <typename T>
-int stage_program(dm_state *h, const dm_op *ops, int nops, const double *params, int64_t nparams, Prepared *pp) {
-  pp->ops.assign(ops, ops + nops);
+int stage_program(dm_state *h, const dm_op *ops, int nops, const double *params, int64_t nparams, Prepared *pp,
+                  bool fuse_plain = true) {
   pp->params.assign(params, params + (nparams > 0 ? nparams : 0));
+  pp->ops.clear();
   pp->fused.clear();
-  pp->fused_of.assign(nops, -1);
-  size_t pool = 0;
-  for (int i = 0; i < nops; ++i) {
+  pp->fused_of.clear();
+  for (int i = 0; i < nops; ++i)
     if (int rc = validate_op(h, ops[i], i, nparams)) return rc;
-    if (ops[i].kind == DM_OP_BLOCK) pool += (size_t)1 << (4 * ops[i].k);
+  size_t pool = 0;
+  auto add_fused = [&](const dm_op &op, FusedPass &&fp) {
+    pool += fp.vals.size();
+    pp->ops.push_back(op);
+    pp->fused_of.push_back((int)pp->fused.size());
+    pp->fused.push_back(std::move(fp));
+  };
+  for (int i = 0; i < nops; ++i) {
     if (ops[i].kind == DM_OP_FUSED) {
       if (ops[i].param < 0 || ops[i].param >= nparams) return fail(DM_ERR_ARG, "op %d: bad parameter offset", i);
       FusedPass fp;
       if (int rc = parse_fused(h, params + ops[i].param, nparams - ops[i].param, i, &fp, true)) return rc;
-      pp->fused_of[i] = (int)pp->fused.size();
-      pool += fp.vals.size();
-      pp->fused.push_back(std::move(fp));
+      add_fused(ops[i], std::move(fp));
+      continue;
     }
+    if (sizeof(T) == 8 && fuse_plain && plain_op(ops[i])) {
+      PlainRun run;
+      int e = i;
+      for (; e < nops && plain_op(ops[e]); ++e) add_plain(h->n, ops[e], params, e, &run);
+      std::vector<FusedPass> fps = fuse_plain_run<T>(h, run, ops, params);
+      dm_op synth;
+      memset(&synth, 0, sizeof(synth));
+      synth.kind = DM_OP_FUSED;
+      for (FusedPass &fp : fps) {
+        if (fp.plain < 0) {
+          add_fused(synth, std::move(fp));
+          continue;
+        }
+        pp->ops.push_back(ops[fp.plain]);
+        pp->fused_of.push_back(-1);
+      }
+      for (int j = i; fps.empty() && j < e; ++j) {
+        pp->ops.push_back(ops[j]);
+        pp->fused_of.push_back(-1);
+      }
+      i = e - 1;
+      continue;
+    }
+    if (ops[i].kind == DM_OP_BLOCK) pool += (size_t)1 << (4 * ops[i].k);
+    pp->ops.push_back(ops[i]);
+    pp->fused_of.push_back(-1);
   }
+  ops = pp->ops.data();
+  nops = (int)pp->ops.size();
   pp->offs.assign(nops, 0);
   pp->pos.assign(4 * (size_t)nops, 0);
   pp->top_off.assign(pp->fused.size(), 0);
@@ -3159,6 +3385,39 @@ int upload_image(dm_state *h, Prepared *pp, void *dev) {
   return DM_OK;
 }
 
+// The same into the handle's own buffer, in stream order through a pinned
+// copy: nothing waits for the device unless the previous image is still on
+// its way.
+int enqueue_image(dm_state *h, Prepared *pp) {
+  const size_t bytes = pp->image_bytes();
+  if (h->img_busy) {
+    HIP_TRY(hipEventSynchronize(h->img_ev));
+    h->img_busy = false;
+  }
+  if (h->img_cap < bytes) {
+    if (h->h_img) hipHostFree(h->h_img);
+    h->h_img = nullptr;
+    h->img_cap = 0;
+    const size_t cap = std::max<size_t>(2 * bytes, 64 << 10);
+    if (hipHostMalloc(&h->h_img, cap, hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();
+      h->h_img = nullptr;
+      return upload_image(h, pp, h->d_mat);
+    }
+    h->img_cap = cap;
+  }
+  if (!h->img_ev) HIP_TRY(hipEventCreateWithFlags(&h->img_ev, hipEventDisableTiming));
+  char *img = static_cast<char *>(h->h_img);
+  if (!pp->tops.empty()) memcpy(img, pp->tops.data(), pp->tops.size() * 4);
+  if (!pp->values.empty()) memcpy(img + pp->vals_at, pp->values.data(), pp->values.size());
+  HIP_TRY(hipMemcpyAsync(h->d_mat, img, bytes, hipMemcpyHostToDevice, h->stream));
+  HIP_TRY(hipEventRecord(h->img_ev, h->stream));
+  h->img_busy = true;
+  pp->d_ops = h->d_mat;
+  pp->d_mat = static_cast<const char *>(h->d_mat) + pp->vals_at;
+  return DM_OK;
+}
+
 // Stage, then upload into the handle's own buffer (grown with hipMalloc).
 template <typename T>
 int prepare_program(dm_state *h, const dm_op *ops, int nops, const double *params, int64_t nparams, Prepared *pp) {
@@ -3166,7 +3425,7 @@ int prepare_program(dm_state *h, const dm_op *ops, int nops, const double *param
   if (pp->tops.empty() && pp->values.empty()) return DM_OK;
   if (h->mat_cap < pp->image_bytes()) HIP_TRY(hipStreamSynchronize(h->stream));  // the old buffer may be in use
   if (int rc = ensure(&h->d_mat, &h->mat_cap, pp->image_bytes())) return rc;
-  return upload_image(h, pp, h->d_mat);
+  return enqueue_image(h, pp);
 }
 
 template <typename T>
@@ -3256,6 +3515,10 @@ template <typename T>
 int run_program_noalloc(dm_state *h, const dm_op *ops, int nops, const double *params, int64_t nparams) {
   Prepared pp;
   if (int rc = stage_program<T>(h, ops, nops, params, nparams, &pp)) return rc;
+  // the image of fused runs is not what a program of single operations may
+  // be refused for
+  if (pp.image_bytes() > kNoAllocScratchBytes)
+    if (int rc = stage_program<T>(h, ops, nops, params, nparams, &pp, false)) return rc;
   if (pp.image_bytes() > kNoAllocScratchBytes)
     return fail(DM_ERR_ARG, "program image of %zu bytes exceeds the %zu-byte scratch of dm_run_program_noalloc",
                 pp.image_bytes(), kNoAllocScratchBytes);
@@ -4024,6 +4287,8 @@ int dm_destroy(dm_state *h) {
   if (h->d_a) hipFree(h->d_a);
   if (h->d_red) hipFree(h->d_red);
   if (h->d_mat) hipFree(h->d_mat);
+  if (h->h_img) hipHostFree(h->h_img);
+  if (h->img_ev) hipEventDestroy(h->img_ev);
   if (h->d_aux) hipFree(h->d_aux);
   if (h->d_mn) hipFree(h->d_mn);
   if (h->ev0) hipEventDestroy(h->ev0);

@@ -391,6 +391,49 @@ __global__ __launch_bounds__(RegCircShape<M>::threads, 2) void k_circuit_reg(con
   if (tid == 0) stamps[2 * blockIdx.x + 1] = wall_clock64();
 }
 
+// A run of operations on a whole state of up to 6 qubits: one wave, loaded
+// and stored in the layouts of the first and the last stage.  Latency bound.
+struct RegWhole {
+  int32_t n, ns;
+  int32_t fr[3], fl[3], lr[3], ll[3];
+};
+
+template <typename T>
+__global__ __launch_bounds__(64, 2) void k_state_reg(T *__restrict__ a, RegWhole w, const RegStage *__restrict__ st,
+                                                     const uint32_t *__restrict__ kinds,
+                                                     const T *__restrict__ prm) {
+  constexpr int M = 6, PH = RegCircShape<M>::phases;
+  __shared__ __align__(16) T s[(1 << (2 * M)) / PH];
+  const int lane = threadIdx.x;
+  // digits from n on do not exist: only their component 0 is in the state
+  auto at = [&](int digit, int x, bool &in) -> uint32_t {
+    in = in && (digit < w.n || x == 0);
+    return (uint32_t)x << (2 * digit);
+  };
+  T v[64];
+  {
+    bool lin = true;
+    const uint32_t lo = at(w.fl[0], lane & 3, lin) + at(w.fl[1], (lane >> 2) & 3, lin) + at(w.fl[2], lane >> 4, lin);
+#pragma unroll
+    for (int i = 0; i < 64; ++i) {
+      bool in = lin;
+      const uint32_t o = lo + at(w.fr[0], i & 3, in) + at(w.fr[1], (i >> 2) & 3, in) + at(w.fr[2], i >> 4, in);
+      v[i] = in ? a[o] : T(0);
+    }
+  }
+  reg_stages<T, M, PH, false>(v, s, st, w.ns, kinds, prm, lane, 0);
+  {
+    bool lin = true;
+    const uint32_t lo = at(w.ll[0], lane & 3, lin) + at(w.ll[1], (lane >> 2) & 3, lin) + at(w.ll[2], lane >> 4, lin);
+#pragma unroll
+    for (int i = 0; i < 64; ++i) {
+      bool in = lin;
+      const uint32_t o = lo + at(w.lr[0], i & 3, in) + at(w.lr[1], (i >> 2) & 3, in) + at(w.lr[2], i >> 4, in);
+      if (in) a[o] = v[i];
+    }
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Host: the register program of a fused pass.
 // ---------------------------------------------------------------------------

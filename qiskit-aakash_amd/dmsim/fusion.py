@@ -505,7 +505,8 @@ def add_block(prog, gates, qs, mem, mode='seq', tile=None, precision='fp32'):
 
 
 def plain_program(gates, n):
-    """One pass per noisy gate."""
+    """One operation per noisy gate, in order.  (FP32 states run one kernel
+    each; on FP64 states the library fuses consecutive ones into passes.)"""
     prog = Program(n)
     for i in range(len(gates)):
         add_block(prog, gates, list(gates[i].qubits), [i])

@@ -215,3 +215,46 @@ def test_fp32_whole_circuits_equal_the_lds_kernel_bit_for_bit():
         out.append(np.concatenate(b.run(False)[0]))
         b.close()
     assert np.array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize('n', [1, 2, 3, 5, 6, 7, 8, 10, 12])
+@pytest.mark.parametrize('noise', [None, (0.98, 0.8, 0.995), (0.98, 0.5, 1.0)])
+def test_fp64_runs_of_single_operations(n, noise):
+    """Programs of single-qubit, CX and memory-noise operations, which an
+    FP64 state runs as fused passes, against the oracle: runs of 2 to 30
+    operations, broken by a diagonal operation that keeps its own kernel.
+    Tolerance: each of the at most 30 (1 + n) maps rounds a coefficient by
+    at most 8 eps of the largest one."""
+    rng = np.random.default_rng(40 + n)
+    for ngates in ((2, 9, 30) if n < 12 else (12,)):
+        prog, _ = small_circuit(rng, n, ngates, noise)
+        keep = rng.uniform(0.9, 1.0, (n, 4))
+        keep[:, 0] = 1.0
+        prog.diag(keep.reshape(-1))
+        q = int(rng.integers(n))
+        prog.one_qubit(q, ptm.memory_noise(0.9, 0.8, 0.7))
+        st = native.DeviceState(n, 'fp64')
+        a = rng.normal(size=4 ** n) * 2.0 ** -n
+        a[0] = 2.0 ** -n
+        st.upload(a)
+        prog.run(st)
+        arr, params = prog.compile()
+        want = a
+        for i in range(len(prog)):
+            op, v = arr[i], params[arr[i].param:]
+            if op.kind == native.OP_1Q:
+                want = oracle_1q(want, n, op.qubits[0], np.vstack([[1.0, 0, 0, 0], v[:12].reshape(3, 4)]))
+            elif op.kind in (native.OP_CX, native.OP_CX_SCALED):
+                s = v[:16] if op.kind == native.OP_CX_SCALED else None
+                want = oracle_cx(want, n, op.qubits[0], op.qubits[1], s)
+            elif op.kind == native.OP_MEMORY_NOISE:
+                want = refsim.apply_memory_noise(want.copy().reshape(n * [4]), n, *v[:3]).reshape(-1)
+            else:
+                x = want.reshape(n * [4])
+                for p in range(n):
+                    x = np.moveaxis(np.moveaxis(x, p, -1) * v[4 * p:4 * p + 4], -1, p)
+                want = np.ascontiguousarray(x).reshape(-1)
+        got = st.download()
+        st.close()
+        assert got[0] == 2.0 ** -n
+        assert np.abs(got - want).max() <= 30 * (1 + n) * 8 * EPS['fp64'] * np.abs(a).max()
