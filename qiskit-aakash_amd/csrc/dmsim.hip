@@ -395,26 +395,42 @@ struct Tab4 {
   double t[kMaxQubits * 4];
 };
 
-template <typename T, bool WRITE_ONLY>
-__global__ __launch_bounds__(kBlock) void k_diag_tab(T *__restrict__ a, uint64_t units, int n, Tab4 tab,
+// The factor of a coefficient is the product of one table entry per digit:
+// a workgroup keeps the products over the lowest kTabDigits digits in LDS and
+// multiplies them with the product over the others, which is the same for
+// the 4^kTabDigits consecutive coefficients of a chunk.  Bound by HBM: 16
+// qubits, FP32, |0..0>: 8.4 ms with n multiplications a coefficient, 2.7 ms
+// (6.4 TB/s) so.  NT: nontemporal accesses (states above the last-level
+// cache).
+constexpr int kTabDigits = 5;
+
+template <typename T, bool WRITE_ONLY, bool NT>
+__global__ __launch_bounds__(kBlock) void k_diag_tab(T *__restrict__ a, uint64_t chunks, int low, int n, Tab4 tab,
                                                      double scale) {
   constexpr int W = 16 / sizeof(T);
   using P = Pack<T, W>;
-  __shared__ double s_tab[kMaxQubits * 4];
-  for (int i = threadIdx.x; i < 4 * n; i += kBlock) s_tab[i] = tab.t[i];
+  __shared__ double s_low[1 << (2 * kTabDigits)];
+  const int len = 1 << (2 * low);
+  for (int i = threadIdx.x; i < len; i += kBlock) {
+    double f = 1.0;
+    for (int p = 0; p < low; ++p) f *= tab.t[4 * p + ((i >> (2 * p)) & 3)];
+    s_low[i] = f;
+  }
   __syncthreads();
-  const uint64_t step = (uint64_t)gridDim.x * kBlock;
-  for (uint64_t u = (uint64_t)blockIdx.x * kBlock + threadIdx.x; u < units; u += step) {
-    P x;
-    if (!WRITE_ONLY) x = ldp<P>(a + u * W);
+  for (uint64_t c = blockIdx.x; c < chunks; c += gridDim.x) {
+    double hi = scale;
+    for (int p = low; p < n; ++p) hi *= tab.t[4 * p + ((c >> (2 * (p - low))) & 3)];
+    T *b = a + c * len;
+    for (int u = threadIdx.x; u < len / W; u += kBlock) {
+      P x;
+      if (!WRITE_ONLY) x = ld16<T, NT>(b + u * W);
 #pragma unroll
-    for (int e = 0; e < W; ++e) {
-      const uint64_t i = u * W + e;
-      double f = scale;
-      for (int p = 0; p < n; ++p) f *= s_tab[4 * p + ((i >> (2 * p)) & 3)];
-      x.v[e] = WRITE_ONLY ? (T)f : (T)(x.v[e] * f);
+      for (int e = 0; e < W; ++e) {
+        const double f = hi * s_low[u * W + e];
+        x.v[e] = WRITE_ONLY ? (T)f : (T)(x.v[e] * f);
+      }
+      st16<T, NT>(b + u * W, x);
     }
-    stp(a + u * W, x);
   }
 }
 
@@ -1318,15 +1334,39 @@ __device__ __forceinline__ double block_sum(double v) {
   return t;
 }
 
+// Four consecutive coefficients as FP64 (16-byte loads).
 template <typename T>
-__global__ __launch_bounds__(kBlock) void k_sumsq(const T *__restrict__ a, uint64_t N, double *part) {
-  double s = 0.0;
+__device__ __forceinline__ void load4(const T *p, double (&x)[4]) {
+  const Pack<T, 4> q = ldq<T, true>(p);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) x[e] = (double)q.v[e];
+}
+
+// Sums over N coefficients, N a multiple of 4: each thread takes quads with
+// the stride of the grid, two in flight.  Bound by HBM (15 qubits, FP32: one
+// coefficient per load 1.15 ms, 3.7 TB/s; quads 0.70 ms).
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_sumsq(const T *__restrict__ a, uint64_t quads, double *part) {
+  double s0 = 0.0, s1 = 0.0;
   const uint64_t step = (uint64_t)gridDim.x * kBlock;
-  for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < N; i += step) {
-    const double v = (double)a[i];
-    s += v * v;
+  uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
+  for (; i + step < quads; i += 2 * step) {
+    double x[4], y[4];
+    load4(a + 4 * i, x);
+    load4(a + 4 * (i + step), y);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      s0 += x[e] * x[e];
+      s1 += y[e] * y[e];
+    }
   }
-  s = block_sum(s);
+  if (i < quads) {
+    double x[4];
+    load4(a + 4 * i, x);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) s0 += x[e] * x[e];
+  }
+  const double s = block_sum(s0 + s1);
   if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
@@ -1341,18 +1381,23 @@ __global__ __launch_bounds__(kBlock) void k_dot(const T *__restrict__ a, const T
   if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
-// per block: max |a-b|, sum a*b, sum a*a, sum b*b
+// per block: max |a-b|, sum a*b, sum a*a, sum b*b (columns of gridDim.x)
 template <typename TA, typename TB>
-__global__ __launch_bounds__(kBlock) void k_diff(const TA *__restrict__ a, const TB *__restrict__ b, uint64_t N,
+__global__ __launch_bounds__(kBlock) void k_diff(const TA *__restrict__ a, const TB *__restrict__ b, uint64_t quads,
                                                  double *part) {
   double mx = 0.0, ab = 0.0, aa = 0.0, bb = 0.0;
   const uint64_t step = (uint64_t)gridDim.x * kBlock;
-  for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < N; i += step) {
-    const double x = (double)a[i], y = (double)b[i];
-    mx = fmax(mx, fabs(x - y));
-    ab += x * y;
-    aa += x * x;
-    bb += y * y;
+  for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < quads; i += step) {
+    double x[4], y[4];
+    load4(a + 4 * i, x);
+    load4(b + 4 * i, y);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      mx = fmax(mx, fabs(x[e] - y[e]));
+      ab += x[e] * y[e];
+      aa += x[e] * x[e];
+      bb += y[e] * y[e];
+    }
   }
   __shared__ double s_m[kBlock];
   s_m[threadIdx.x] = mx;
@@ -1369,11 +1414,34 @@ __global__ __launch_bounds__(kBlock) void k_diff(const TA *__restrict__ a, const
   __syncthreads();
   bb = block_sum(bb);
   if (threadIdx.x == 0) {
-    part[4 * blockIdx.x] = m;
-    part[4 * blockIdx.x + 1] = ab;
-    part[4 * blockIdx.x + 2] = aa;
-    part[4 * blockIdx.x + 3] = bb;
+    const int g = gridDim.x;
+    part[blockIdx.x] = m;
+    part[g + blockIdx.x] = ab;
+    part[2 * g + blockIdx.x] = aa;
+    part[3 * g + blockIdx.x] = bb;
   }
+}
+
+// The partials of k_diff: out[0] their maximum, out[1..3] their sums.
+__global__ __launch_bounds__(kBlock) void k_diff_parts(const double *part, int nparts, double *out) {
+  const double *p = part + (size_t)blockIdx.x * nparts;
+  if (blockIdx.x == 0) {
+    __shared__ double s_m[kBlock];
+    double m = 0.0;
+    for (int i = threadIdx.x; i < nparts; i += kBlock) m = fmax(m, p[i]);
+    s_m[threadIdx.x] = m;
+    __syncthreads();
+    for (int off = kBlock / 2; off > 0; off >>= 1) {
+      if ((int)threadIdx.x < off) s_m[threadIdx.x] = fmax(s_m[threadIdx.x], s_m[threadIdx.x + off]);
+      __syncthreads();
+    }
+    if (threadIdx.x == 0) out[0] = s_m[0];
+    return;
+  }
+  double s = 0.0;
+  for (int i = threadIdx.x; i < nparts; i += kBlock) s += p[i];
+  s = block_sum(s);
+  if (threadIdx.x == 0) out[blockIdx.x] = s;
 }
 
 __global__ __launch_bounds__(kBlock) void k_sum_parts(const double *part, int nparts, double *out) {
@@ -1409,23 +1477,104 @@ __global__ __launch_bounds__(kBlock) void k_gather(const T *__restrict__ a, uint
   }
 }
 
-// One contraction step over digit t: (pre, din, post) -> (pre, 2, post),
-// out[p,b,q] = sum_x w[b][x] in[p,x,q].
+// Gather and the contraction of the last `low` measured digits, in LDS: the
+// block's gathered values are those of the leading digits' index blockIdx.x.
+// Base 2 (components {I, k}): digit pairs (u, w) -> (u + e w, u - e w) in
+// place.  Base 4: values of 4 components -> 2 outcomes, the leading digit of
+// the remaining index first, ping-pong between two halves of LDS.  One launch
+// instead of a gather and one contraction per digit (latency bound: 16 qubits
+// 17 launches of 4.5 us).
+constexpr int kProbDigits2 = 12;  // 32 KB of LDS
+constexpr int kProbDigits4 = 6;   // 32 KB and 16 KB
+
+template <typename T>
+__global__ __launch_bounds__(1024) void k_probs(const T *__restrict__ a, GatherSpec gs, int low, double w1, double w2,
+                                                double w3, double *__restrict__ out) {
+  __shared__ double s[4096 + 2048];
+  const int bl = gs.base_log;
+  const uint32_t cnt = 1u << (bl * low);
+  uint64_t base = 0;
+  for (int t = 0; t < gs.m - low; ++t) {
+    const uint64_t d = ((uint64_t)blockIdx.x >> (bl * (gs.m - low - 1 - t))) & ((1u << bl) - 1u);
+    base += (bl == 1 ? (d ? (uint64_t)gs.comp : 0ull) : d) * gs.stride[t];
+  }
+  for (uint32_t j = threadIdx.x; j < cnt; j += blockDim.x) {
+    uint64_t idx = base;
+    for (int t = 0; t < low; ++t) {
+      const uint32_t d = (j >> (bl * (low - 1 - t))) & ((1u << bl) - 1u);
+      idx += (bl == 1 ? (d ? (uint64_t)gs.comp : 0ull) : (uint64_t)d) * gs.stride[gs.m - low + t];
+    }
+    s[j] = (double)a[idx];
+  }
+  __syncthreads();
+  double *src = s;
+  if (bl == 1) {
+    for (int q = 0; q < low; ++q) {
+      for (uint32_t x = threadIdx.x; x < cnt / 2; x += blockDim.x) {
+        const uint32_t lo = x & ((1u << q) - 1u), b = ((x >> q) << (q + 1)) | lo;
+        const double u = s[b], w = w1 * s[b | (1u << q)];
+        s[b] = u + w;
+        s[b | (1u << q)] = u - w;
+      }
+      __syncthreads();
+    }
+  } else {
+    double *dst = s + 4096;
+    for (int t = 0; t < low; ++t) {
+      // (2^t, 4, post) -> (2^t, 2, post)
+      const uint32_t post = 1u << (2 * (low - 1 - t)), total = (2u << t) * post;
+      for (uint32_t o = threadIdx.x; o < total / 2; o += blockDim.x) {
+        const uint32_t q = o & (post - 1), p = o / post;
+        const double *x = src + (size_t)p * 4 * post + q;
+        const double u = x[0], w = w1 * x[post] + w2 * x[2 * post] + w3 * x[3 * post];
+        dst[(size_t)p * 2 * post + q] = u + w;
+        dst[(size_t)p * 2 * post + post + q] = u - w;
+      }
+      __syncthreads();
+      double *const t2 = src;
+      src = dst;
+      dst = t2;
+    }
+  }
+  const uint32_t no = 1u << low;
+  for (uint32_t x = threadIdx.x; x < no; x += blockDim.x) out[(uint64_t)blockIdx.x * no + x] = src[x];
+}
+
+// Contraction of up to four leading base-2 digits in registers: column c of
+// (2^lead, 2^D, post) values.
+template <int D>
+__global__ __launch_bounds__(kBlock) void k_probs_lead(double *__restrict__ v, uint64_t cols, uint64_t post, double e) {
+  const uint64_t c = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (c >= cols) return;
+  double *p = v + (c / post) * (post << D) + c % post;
+  double x[1 << D];
+#pragma unroll
+  for (int i = 0; i < (1 << D); ++i) x[i] = p[(uint64_t)i * post];
+#pragma unroll
+  for (int q = 0; q < D; ++q)
+#pragma unroll
+    for (int i = 0; i < (1 << D); ++i)
+      if (!((i >> q) & 1)) {
+        const double u = x[i], w = e * x[i | (1 << q)];
+        x[i] = u + w;
+        x[i | (1 << q)] = u - w;
+      }
+#pragma unroll
+  for (int i = 0; i < (1 << D); ++i) p[(uint64_t)i * post] = x[i];
+}
+
+// One contraction step over a base-4 digit: (pre, 4, post) -> (pre, 2, post),
+// the outcomes u + w and u - w of u = in[p, 0, q], w = sum_k wk in[p, k, q].
 __global__ __launch_bounds__(kBlock) void k_contract(const double *__restrict__ in, double *__restrict__ out,
-                                                     uint64_t pre, int din, uint64_t post, double w00,
-                                                     double w01, double w02, double w03, double w10,
-                                                     double w11, double w12, double w13) {
-  const uint64_t total = pre * 2 * post;
+                                                     uint64_t pre, uint64_t post, double w1, double w2, double w3) {
+  const uint64_t total = pre * post;
   const uint64_t step = (uint64_t)gridDim.x * kBlock;
   for (uint64_t o = (uint64_t)blockIdx.x * kBlock + threadIdx.x; o < total; o += step) {
-    const uint64_t q = o % post;
-    const uint64_t b = (o / post) & 1ull;
-    const uint64_t p = o / (2 * post);
-    const double *src = in + p * din * post + q;
-    const double w0 = b ? w10 : w00, w1 = b ? w11 : w01, w2 = b ? w12 : w02, w3 = b ? w13 : w03;
-    double s = w0 * src[0] + w1 * src[post];
-    if (din == 4) s += w2 * src[2 * post] + w3 * src[3 * post];
-    out[o] = s;
+    const uint64_t q = o % post, p = o / post;
+    const double *x = in + p * 4 * post + q;
+    const double u = x[0], w = w1 * x[post] + w2 * x[2 * post] + w3 * x[3 * post];
+    out[p * 2 * post + q] = u + w;
+    out[p * 2 * post + post + q] = u - w;
   }
 }
 
@@ -2168,15 +2317,23 @@ int launch_diag_tab(dm_state *h, const double *tab_by_pos, bool write_only, doub
   Tab4 tab;
   memset(&tab, 0, sizeof(tab));
   memcpy(tab.t, tab_by_pos, sizeof(double) * 4 * h->n);
-  constexpr int W = 16 / sizeof(T);
-  const uint64_t units = h->N / W;
   ProfScope ps(h, write_only ? 7 : 4);
-  if (write_only)
-    hipLaunchKernelGGL((k_diag_tab<T, true>), dim3(grid_for(h, units)), dim3(kBlock), 0, h->stream,
-                       static_cast<T *>(h->d_a), units, h->n, tab, scale);
-  else
-    hipLaunchKernelGGL((k_diag_tab<T, false>), dim3(grid_for(h, units)), dim3(kBlock), 0, h->stream,
-                       static_cast<T *>(h->d_a), units, h->n, tab, scale);
+  const int low = std::min(h->n, kTabDigits);
+  const uint64_t chunks = h->N >> (2 * low);
+  // several chunks a workgroup, so that the LDS table is a small part of it
+  const dim3 grid((unsigned)std::min<uint64_t>(chunks, 8192));
+  const bool nt = h->N * sizeof(T) > (256ull << 20);
+  T *a = static_cast<T *>(h->d_a);
+#define DIAG_TAB(WO, NT) \
+  hipLaunchKernelGGL((k_diag_tab<T, WO, NT>), grid, dim3(kBlock), 0, h->stream, a, chunks, low, h->n, tab, scale)
+  if (write_only) {
+    if (nt) DIAG_TAB(true, true);
+    else DIAG_TAB(true, false);
+  } else {
+    if (nt) DIAG_TAB(false, true);
+    else DIAG_TAB(false, false);
+  }
+#undef DIAG_TAB
   return last_launch("k_diag_tab");
 }
 
@@ -2259,11 +2416,12 @@ int reserve_red(dm_state *h, size_t doubles) {
 
 template <typename T>
 int do_sumsq(dm_state *h, double *out) {
-  const int grid = std::min(grid_for(h, h->N), 4096);
+  const uint64_t quads = h->N / 4;
+  const int grid = std::min(grid_for(h, quads), 4096);
   int rc = reserve_red(h, (size_t)grid + 8);
   if (rc) return rc;
   ProfScope ps(h, 6);
-  hipLaunchKernelGGL((k_sumsq<T>), dim3(grid), dim3(kBlock), 0, h->stream, static_cast<const T *>(h->d_a), h->N,
+  hipLaunchKernelGGL((k_sumsq<T>), dim3(grid), dim3(kBlock), 0, h->stream, static_cast<const T *>(h->d_a), quads,
                      h->d_red);
   hipLaunchKernelGGL(k_sum_parts, dim3(1), dim3(kBlock), 0, h->stream, h->d_red, grid, h->d_red + grid);
   rc = last_launch("k_sumsq");
@@ -2359,18 +2517,13 @@ int do_probabilities(dm_state *h, const int *qubits, int m, char basis, const do
   GatherSpec gs;
   memset(&gs, 0, sizeof(gs));
   gs.m = m;
-  double w[2][4] = {{1, 0, 0, 0}, {1, 0, 0, 0}};
+  double w[3] = {err, 0, 0};  // outcomes u + w.x and u - w.x of a digit's components (u, x)
   if (basis == 'N') {
     gs.base_log = 2;
-    for (int k = 0; k < 3; ++k) {
-      w[0][k + 1] = nvec[k] * err;
-      w[1][k + 1] = -nvec[k] * err;
-    }
+    for (int k = 0; k < 3; ++k) w[k] = nvec[k] * err;
   } else {
     gs.base_log = 1;
     gs.comp = basis == 'X' ? 1 : basis == 'Y' ? 2 : 3;
-    w[0][1] = err;
-    w[1][1] = -err;
   }
   for (int t = 0; t < m; ++t) gs.stride[t] = pow4(h->n - 1 - qubits[t]);
   const uint64_t count = 1ull << (gs.base_log * m);
@@ -2380,19 +2533,35 @@ int do_probabilities(dm_state *h, const int *qubits, int m, char basis, const do
   if (rc) return rc;
   double *buf0 = h->d_aux, *buf1 = h->d_aux + count;
   ProfScope ps(h, 6);
-  hipLaunchKernelGGL((k_gather<T>), dim3(grid_for(h, count)), dim3(kBlock), 0, h->stream,
-                     static_cast<const T *>(h->d_a), count, gs, buf0);
   double *src = buf0, *dst = buf1;
-  const uint64_t din = 1ull << gs.base_log;
-  for (int t = 0; t < m; ++t) {
-    const uint64_t pre = 1ull << t;
-    uint64_t post = 1;
-    for (int r = t + 1; r < m; ++r) post *= din;
-    hipLaunchKernelGGL(k_contract, dim3(grid_for(h, pre * 2 * post)), dim3(kBlock), 0, h->stream, src, dst, pre,
-                       (int)din, post, w[0][0], w[0][1], w[0][2], w[0][3], w[1][0], w[1][1], w[1][2], w[1][3]);
-    std::swap(src, dst);
+  if (gs.base_log == 1 || m <= kProbDigits4) {
+    const int low = gs.base_log == 1 ? std::min(m, kProbDigits2) : m;
+    const int threads = std::max(64, std::min(1024, 1 << std::max(0, gs.base_log * low - 2)));
+    hipLaunchKernelGGL((k_probs<T>), dim3(1u << (m - low)), dim3(threads), 0, h->stream,
+                       static_cast<const T *>(h->d_a), gs, low, w[0], w[1], w[2], buf0);
+    for (int done = low; done < m;) {
+      const int d = std::min(4, m - done);
+      const uint64_t cols = outn >> d, post = 1ull << done;
+      const dim3 grid((unsigned)((cols + kBlock - 1) / kBlock));
+      switch (d) {
+        case 1: hipLaunchKernelGGL((k_probs_lead<1>), grid, dim3(kBlock), 0, h->stream, buf0, cols, post, err); break;
+        case 2: hipLaunchKernelGGL((k_probs_lead<2>), grid, dim3(kBlock), 0, h->stream, buf0, cols, post, err); break;
+        case 3: hipLaunchKernelGGL((k_probs_lead<3>), grid, dim3(kBlock), 0, h->stream, buf0, cols, post, err); break;
+        default: hipLaunchKernelGGL((k_probs_lead<4>), grid, dim3(kBlock), 0, h->stream, buf0, cols, post, err); break;
+      }
+      done += d;
+    }
+  } else {
+    hipLaunchKernelGGL((k_gather<T>), dim3(grid_for(h, count)), dim3(kBlock), 0, h->stream,
+                       static_cast<const T *>(h->d_a), count, gs, buf0);
+    for (int t = 0; t < m; ++t) {
+      const uint64_t pre = 1ull << t, post = pow4(m - 1 - t);
+      hipLaunchKernelGGL(k_contract, dim3(grid_for(h, pre * post)), dim3(kBlock), 0, h->stream, src, dst, pre, post,
+                         w[0], w[1], w[2]);
+      std::swap(src, dst);
+    }
   }
-  rc = last_launch("k_gather/k_contract");
+  rc = last_launch("k_probs");
   if (rc) return rc;
   HIP_TRY(hipMemcpyAsync(out, src, outn * sizeof(double), hipMemcpyDeviceToHost, h->stream));
   HIP_TRY(hipStreamSynchronize(h->stream));
@@ -4205,26 +4374,17 @@ static int batch_create_t(dm_batch *b, const int64_t *op_start, const dm_op *ops
 
 template <typename TA, typename TB>
 static int diff_t(dm_state *a, dm_state *b, double *out4) {
-  const int grid = std::min(grid_for(a, a->N), 2048);
-  if (int rc = reserve_red(a, 4 * (size_t)grid)) return rc;
+  const uint64_t quads = a->N / 4;
+  const int grid = std::min(grid_for(a, quads), 4096);
+  if (int rc = reserve_red(a, 4 * (size_t)grid + 8)) return rc;
   HIP_TRY(hipStreamSynchronize(b->stream));
   hipLaunchKernelGGL((k_diff<TA, TB>), dim3(grid), dim3(kBlock), 0, a->stream, static_cast<const TA *>(a->d_a),
-                     static_cast<const TB *>(b->d_a), a->N, a->d_red);
+                     static_cast<const TB *>(b->d_a), quads, a->d_red);
+  double *res = a->d_red + 4 * (size_t)grid;
+  hipLaunchKernelGGL(k_diff_parts, dim3(4), dim3(kBlock), 0, a->stream, a->d_red, grid, res);
   if (int rc = last_launch("k_diff")) return rc;
-  std::vector<double> part(4 * (size_t)grid);
-  HIP_TRY(hipMemcpyAsync(part.data(), a->d_red, part.size() * sizeof(double), hipMemcpyDeviceToHost, a->stream));
+  HIP_TRY(hipMemcpyAsync(out4, res, 4 * sizeof(double), hipMemcpyDeviceToHost, a->stream));
   HIP_TRY(hipStreamSynchronize(a->stream));
-  double m = 0, ab = 0, aa = 0, bb = 0;
-  for (int i = 0; i < grid; ++i) {
-    m = std::max(m, part[4 * i]);
-    ab += part[4 * i + 1];
-    aa += part[4 * i + 2];
-    bb += part[4 * i + 3];
-  }
-  out4[0] = m;
-  out4[1] = ab;
-  out4[2] = aa;
-  out4[3] = bb;
   return DM_OK;
 }
 
