@@ -396,26 +396,31 @@ struct Tab4 {
 };
 
 // The factor of a coefficient is the product of one table entry per digit:
-// a workgroup keeps the products over the lowest kTabDigits digits in LDS and
-// multiplies them with the product over the others, which is the same for
-// the 4^kTabDigits consecutive coefficients of a chunk.  Bound by HBM: 16
-// qubits, FP32, |0..0>: 8.4 ms with n multiplications a coefficient, 2.7 ms
-// (6.4 TB/s) so.  NT: nontemporal accesses (states above the last-level
-// cache).
-constexpr int kTabDigits = 5;
+// a workgroup keeps the products over the lowest kTabDigits digits in LDS
+// (built from the products over their two halves) and multiplies them with
+// the product over the others, which is the same for the 4^kTabDigits
+// consecutive coefficients of a chunk.  Bound by HBM writes.  |0..0>, FP32:
+// 16 qubits 8.4 ms with n multiplications a coefficient, 4.2 ms with chunks
+// of 4^5, 3.2 ms (5.4 TB/s) with 4^6; 13 qubits 148, 74 and 49 us.
+// NT: nontemporal accesses (states above the last-level cache).
+constexpr int kTabDigits = 6;
 
 template <typename T, bool WRITE_ONLY, bool NT>
 __global__ __launch_bounds__(kBlock) void k_diag_tab(T *__restrict__ a, uint64_t chunks, int low, int n, Tab4 tab,
                                                      double scale) {
   constexpr int W = 16 / sizeof(T);
   using P = Pack<T, W>;
-  __shared__ double s_low[1 << (2 * kTabDigits)];
-  const int len = 1 << (2 * low);
-  for (int i = threadIdx.x; i < len; i += kBlock) {
+  __shared__ double s_low[1 << (2 * kTabDigits)], s_half[2][1 << kTabDigits];
+  const int len = 1 << (2 * low), l0 = low / 2;
+  for (int i = threadIdx.x; i < 2 << kTabDigits; i += kBlock) {
+    const int half = i >> kTabDigits, k = i & ((1 << kTabDigits) - 1);
+    const int p0 = half ? l0 : 0, p1 = half ? low : l0;
     double f = 1.0;
-    for (int p = 0; p < low; ++p) f *= tab.t[4 * p + ((i >> (2 * p)) & 3)];
-    s_low[i] = f;
+    for (int p = p0; p < p1; ++p) f *= tab.t[4 * p + ((k >> (2 * (p - p0))) & 3)];
+    s_half[half][k] = f;
   }
+  __syncthreads();
+  for (int i = threadIdx.x; i < len; i += kBlock) s_low[i] = s_half[0][i & ((1 << (2 * l0)) - 1)] * s_half[1][i >> (2 * l0)];
   __syncthreads();
   for (uint64_t c = blockIdx.x; c < chunks; c += gridDim.x) {
     double hi = scale;

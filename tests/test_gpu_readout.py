@@ -1,6 +1,6 @@
 """Read-outs against the oracle at the sizes where their kernels change:
 probabilities around the digits one launch contracts (12 of two components,
-6 of four), product states around the digits of the LDS table (5), and the
+6 of four), product states around the digits of the LDS table (6), and the
 FP64 sums.  Tolerances: a probability is a sum of 2^m (4^m) FP64 products
 contracted pairwise, at most 3 m roundings of values <= its largest partial
 sum (1 for a state of unit trace); a product has n + 1 factors; a sum of N
@@ -61,7 +61,7 @@ def test_probabilities_of_one_to_all_qubits(n, precision):
 
 
 @pytest.mark.parametrize('precision', ['fp64', 'fp32'])
-@pytest.mark.parametrize('n', [1, 2, 4, 5, 6, 9])
+@pytest.mark.parametrize('n', [1, 2, 4, 5, 6, 7, 9])
 def test_product_states_and_diagonals(n, precision):
     rng = np.random.default_rng(20 + n)
     eps = EPS if precision == 'fp64' else 2.0 ** -24
