@@ -94,14 +94,22 @@ __device__ __forceinline__ void reg_1q(T (&v)[64], const T (&pv)[kRegVals]) {
   }
 }
 
+// In place (v_swap_b32): plain copies would keep a second set of registers
+// alive where the members' code paths join (FP64: 196 VGPRs, two waves per
+// SIMD, against 150 and three: 15 qubits 81.7 -> 76.9 ms, 10 qubits 366 -> 331
+// us).
 template <typename T>
 __device__ __forceinline__ void reg_swap(T &a, T &b) {
   if constexpr (sizeof(T) == 4) {
     asm("v_swap_b32 %0, %1" : "+v"(a), "+v"(b));
   } else {
-    const T t = a;
-    a = b;
-    b = t;
+    typedef uint32_t U2 __attribute__((ext_vector_type(2)));
+    const U2 x = __builtin_bit_cast(U2, a), y = __builtin_bit_cast(U2, b);
+    uint32_t xl = x.x, xh = x.y, yl = y.x, yh = y.y;
+    asm("v_swap_b32 %0, %1" : "+v"(xl), "+v"(yl));
+    asm("v_swap_b32 %0, %1" : "+v"(xh), "+v"(yh));
+    a = __builtin_bit_cast(T, U2{xl, xh});
+    b = __builtin_bit_cast(T, U2{yl, yh});
   }
 }
 
@@ -194,6 +202,14 @@ __device__ __forceinline__ void reg_members(T (&v)[64], const uint32_t *__restri
   }
 }
 
+// Barrier of the workgroup that orders LDS accesses only: global loads and
+// stores stay in flight.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // Redistribution through LDS in phases: phase h moves the coefficients whose
 // digit in SLOT (a register digit before and after) lies in the h-th part of
 // its range, from and into the same registers, so that a phase needs only
@@ -211,21 +227,27 @@ __device__ __forceinline__ void reg_exchange(T (&v)[64], T *s, const RegStage &s
   char *c = reinterpret_cast<char *>(s);
 #pragma unroll
   for (int h = 0; h < PH; ++h) {
-    __syncthreads();  // the previous phase has been read
+    // addresses are computed anew in each phase: kept over the phases they
+    // would cost the registers of another wave (FP32: 88 VGPRs and 5 waves
+    // per SIMD against 105 and 4: 13 qubits 2.80 against 2.86 ms, a batch of
+    // 512 circuits 58.5 against 60.2 ms)
+    uint32_t bw = tw, br = tr;
+    asm volatile("" : "+v"(bw), "+v"(br));
+    lds_barrier();  // the previous phase has been read
 #pragma unroll
     for (int i = 0; i < 64; ++i) {
       const int d = (i / S) & 3;
       if (d / IN != h) continue;
       const uint32_t o = ((((i >> (2 * SA)) & 3) * st.wr[SA]) ^ (((i >> (2 * SB)) & 3) * st.wr[SB])) * B;
-      *reinterpret_cast<T *>(c + (tw ^ o) + (d % IN) * PART * B) = v[i];
+      *reinterpret_cast<T *>(c + (bw ^ o) + (d % IN) * PART * B) = v[i];
     }
-    __syncthreads();
+    lds_barrier();
 #pragma unroll
     for (int i = 0; i < 64; ++i) {
       const int d = (i / S) & 3;
       if (d / IN != h) continue;
       const uint32_t o = ((((i >> (2 * SA)) & 3) * st.rr[SA]) ^ (((i >> (2 * SB)) & 3) * st.rr[SB])) * B;
-      v[i] = *reinterpret_cast<const T *>(c + (tr ^ o) + (d % IN) * PART * B);
+      v[i] = *reinterpret_cast<const T *>(c + (br ^ o) + (d % IN) * PART * B);
     }
   }
 }
@@ -291,20 +313,31 @@ __device__ __forceinline__ void reg_tile(T *__restrict__ a, T *s, const RegGeom 
   reg_stages<T, kRegTile, PH, false>(v, s, st, ns, kinds, prm, lane, wave);
   {
     T *p = a + base + wave * geo.ow;
+    // (a 32-bit offset of its own, so that the stores take a scalar base)
+    uint32_t soff = loff;
+    asm volatile("" : "+v"(soff));
 #pragma unroll
     for (int i = 0; i < 64; ++i)
-      reg_store<T, NTM>(p + (i & 3) * geo.os[0] + ((i >> 2) & 3) * geo.os[1] + (i >> 4) * geo.os[2], loff, v[i]);
+      reg_store<T, NTM>(p + (i & 3) * geo.os[0] + ((i >> 2) & 3) * geo.os[1] + (i >> 4) * geo.os[2], soff, v[i]);
   }
 }
 
 template <typename T, bool NTM>
-__global__ __launch_bounds__(kRegThreads, sizeof(T) == 4 ? 4 : 2) void k_tile_reg(T *__restrict__ a, RegGeom geo,
+__global__ __launch_bounds__(kRegThreads, sizeof(T) == 4 ? 5 : 3) void k_tile_reg(T *__restrict__ a, RegGeom geo,
                                                              const RegStage *__restrict__ st, int ns,
                                                              const uint32_t *__restrict__ kinds,
                                                              const T *__restrict__ prm) {
   __shared__ __align__(16) T s[RegShape<T>::lds];
   if (blockIdx.x >= geo.tiles) return;  // uniform over the workgroup
-  reg_tile<T, NTM>(a, s, geo, blockIdx.x, st, ns, kinds, prm);
+  // Workgroups go to the 8 XCDs in turn.  Streaming from HBM (NTM: at least
+  // 4^6 tiles), an XCD takes 64 consecutive tiles, whose low digits run over
+  // consecutive addresses, so that its requests fall on fewer DRAM pages:
+  // 16 qubits FP32 519 -> 504 ms, 15 qubits FP64 84.2 -> 81.7 ms; 32 to 256
+  // tiles measured the same.  States inside the last-level cache lose a
+  // little by it (13 qubits FP32 2.83 -> 2.87 ms) and keep the plain order.
+  uint32_t t = blockIdx.x;
+  if (NTM) t = (t & ~511u) + (t % 8) * 64 + (t / 8) % 64;
+  reg_tile<T, NTM>(a, s, geo, t, st, ns, kinds, prm);
 }
 
 // A whole circuit of up to M qubits (6: one wave; 7: four) in registers, from

@@ -159,6 +159,30 @@ def test_fp32_passes_equal_the_lds_form_bit_for_bit(n, m, qubits):
     assert np.array_equal(got[0], got[1])
 
 
+@pytest.mark.parametrize('n,precision', [(13, 'fp64'), (14, 'fp32')])
+def test_states_above_the_last_level_cache(n, precision):
+    """Every tile is visited once: passes of single-qubit maps take a product
+    state to the product of the mapped vectors (each coefficient a product of
+    n + 1 factors on either side, and one sum of 4 products a map)."""
+    rng = np.random.default_rng(n)
+    vecs = np.concatenate([np.ones((n, 1)), rng.uniform(-0.5, 0.5, (n, 3))], axis=1)
+    prog = Program(n)
+    st = native.DeviceState(n, precision)
+    st.init_product(vecs.reshape(-1), 2.0 ** -n)
+    for qubits in ([0, 1, 2, 3], [n - 7, n - 6, n - 5, n - 4], [n - 4, n - 3, n - 2, n - 1], [0, 4, n - 1]):
+        maps = [random_map(rng, 'general') for _ in qubits]
+        prog.fused(7, qubits, [(native.SUB_1Q, [q], ptm.rows3(R)) for q, R in zip(qubits, maps)])
+        for q, R in zip(qubits, maps):
+            vecs[q] = R @ vecs[q]
+    prog.run(st)
+    want = native.DeviceState(n, precision)
+    want.init_product(vecs.reshape(-1), 2.0 ** -n)
+    r = st.compare(want)
+    st.close()
+    want.close()
+    assert r['max_abs_diff'] <= (15 * 8 + 2 * (n + 2)) * EPS[precision] * 2.0 ** -n
+
+
 def small_circuit(rng, n, ngates, noise):
     """(Program, the oracle's probabilities) of a random circuit with memory
     noise after every gate, depolarising CX scales and a final measurement
