@@ -223,9 +223,10 @@ int dm_mlp_train(float *params, int n_features, int hidden, const float *X, cons
  * probabilities of all its qubits with polarisation retention meas_err[c]
  * (2^n values, most significant bit = qubit 0, circuits concatenated).
  * Circuits of at most lds_max_qubits (5..7) qubits run whole inside one
- * workgroup: in registers (one launch for up to 6 qubits, one for 7) when
- * they hold single-qubit maps, CX and memory noise only, else in LDS (one
- * launch per width, lds_threads threads per workgroup).
+ * workgroup: in registers when they hold single-qubit maps, CX and memory
+ * noise only (FP64: one launch for up to 6 qubits, one for 7; FP32: 7
+ * qubits), else in LDS (one launch per width, lds_threads threads per
+ * workgroup).
  * The others keep their state in one HBM arena: each operation becomes a
  * 6-digit tile pass (DM_OP_FUSED with tile size 6, DM_OP_1Q, DM_OP_CX[_SCALED],
  * DM_OP_2Q, DM_OP_MEMORY_NOISE; memory noise as 1-qubit channels, 6 qubits

@@ -2042,7 +2042,7 @@ struct dm_state {
   void *d_a = nullptr;
   hipStream_t stream = nullptr;
   bool owns_stream = true;
-  bool batched = false;  // stands for a circuit of a batch (host-side planning only)
+  bool batched = false;  // a circuit of a batch that fills the CUs (host-side planning only)
   // scratch
   double *d_red = nullptr;      // reduction partials + results
   size_t red_cap = 0;           // doubles
@@ -2849,14 +2849,19 @@ void set_reg(FusedPass *fp, RegPlan &&rp, const RegTile &t) {
 // against 6.7 / 7.7 / 14.3 with the tile in LDS, FP64 12.0 / 12.6 / 16.4
 // against 13.1 / 15.5 / 24.8).  Below, a launch is a few workgroups per CU
 // and its latency counts: the tile-in-LDS kernel's 6-digit tiles fill more
-// CUs, and only passes with many operations per redistribution gain (9
-// qubits, FP64: one pair 9.5 against 6.2 us, 8 pairs 18.8 against 20.3).
-// A batch's passes (h->batched) run side by side by the hundred, so that
-// throughput counts at every register size.
+// CUs, and in FP32 the operations in order need too many redistributions (300
+// gates on 9 / 11 qubits, matching, learned: 437 / 494 us in LDS against 463 /
+// 518).  FP64 passes of many operations per redistribution gain on 7 digits,
+// whose LDS form is one workgroup a CU (same circuits, 7 / 9 qubits: 360 / 458
+// us against 278 / 420), and on fewer digits from 11 qubits on (greedy, 800
+// against 769 us; 9 qubits 523 against 553).
+// A batch's passes run side by side; with 256 tiles and more between them
+// (h->batched) throughput counts at every register size (7 qubits, FP32, 328
+// circuits 797 -> 755 us, 49 circuits 431 -> 468).
 bool plan_reg(const dm_state *h, FusedPass *fp) {
   if (h->n < kRegTile || h->n > 18) return false;
   const bool few = h->n < 12 && !h->batched;
-  if (few && fp->ops.size() < 12) return false;
+  if (few && (h->dtype == DM_FP32 || fp->ops.size() < 12 || (fp->m < 7 && h->n < 11))) return false;
   for (const TileOp &op : fp->ops)
     if (op.kind != TOP_1Q && op.kind != TOP_CX) return false;
   RegTile t;
@@ -3841,20 +3846,22 @@ int small_circuit_ops(int n, const dm_op *ops, int nops, const double *params, i
 // The register-resident program of a small circuit; *fits false (and no
 // error) if it holds operations that form does not take.  FP64: memory noise
 // and single-qubit maps between two CX gates on a qubit become one map.
-// FP32: every operation on its own and in order, as the LDS kernel rounds.
+// FP32: every operation on its own and in order, as the LDS kernel rounds; on
+// fewer than 7 qubits that many redistributions cost more than the LDS
+// kernel's passes (49 circuits of 6 qubits and 40-150 gates, memory noise
+// after each: 1109 us against 604; 7 qubits 1454 against 1749).
 template <typename T>
 int small_circuit_plan(int n, const dm_op *ops, int nops, const double *params, int64_t nparams, int ci, bool *fits,
                        RegPlan *rp) {
+  *fits = false;
+  if (sizeof(T) == 4 && n < kRegTile) return DM_OK;
   std::vector<TileOp> tops;
   std::vector<double> vals;
   if (int rc = small_circuit_ops(n, ops, nops, params, nparams, ci, &tops, &vals)) return rc;
   std::vector<TileOp> flat;
   flat.reserve(tops.size() * 2);
   for (const TileOp &op : tops) {
-    if (op.kind == TOP_2Q) {
-      *fits = false;
-      return DM_OK;
-    }
+    if (op.kind == TOP_2Q) return DM_OK;
     if (op.kind != TOP_ALLQ) {
       flat.push_back(op);
       continue;
@@ -3967,16 +3974,21 @@ int enqueue_batch(dm_batch *b) {
                        rc + b->nreg6, rrecs, rvals, b->d_probs, b->d_stamps + 2 * (size_t)b->nreg6);
     if (int rc2 = last_launch("k_circuit_reg")) return rc2;
   }
-  if (b->nreg6) {
-    hipLaunchKernelGGL((k_circuit_reg<T, 6, SEQ>), dim3(b->nreg6), dim3(RegCircShape<6>::threads), 0, b->side, rc,
-                       rrecs, rvals, b->d_probs, b->d_stamps);
-    if (int rc2 = last_launch("k_circuit_reg")) return rc2;
+  if constexpr (!SEQ) {
+    if (b->nreg6) {
+      hipLaunchKernelGGL((k_circuit_reg<T, 6, SEQ>), dim3(b->nreg6), dim3(RegCircShape<6>::threads), 0, b->side, rc,
+                         rrecs, rvals, b->d_probs, b->d_stamps);
+      if (int rc2 = last_launch("k_circuit_reg")) return rc2;
+    }
   }
   const int reg = b->nreg6 + b->nreg7;
-  for (int w = 1; w <= 7; ++w) {
+  // the widest first, in turn on the two streams: a width's circuits rarely
+  // fill the chip and run beside the next width's
+  for (int w = 7; w >= 1; --w) {
     const int lo = b->small_width_start[w], hi = b->small_width_start[w + 1];
     if (hi <= lo) continue;
-    hipLaunchKernelGGL((k_circuit_lds<T>), dim3(hi - lo), dim3(b->lds_threads), lds_bytes(w, b->dtype), b->side,
+    hipLaunchKernelGGL((k_circuit_lds<T>), dim3(hi - lo), dim3(b->lds_threads), lds_bytes(w, b->dtype),
+                       (w & 1) ? b->side2 : b->side,
                        static_cast<const BatchCirc *>(b->d_circs) + (lo - reg), static_cast<const TileOp *>(b->d_tops),
                        static_cast<const T *>(b->d_vals), b->d_probs, b->d_stamps + 2 * (size_t)lo);
     if (int rc = last_launch("k_circuit_lds")) return rc;
@@ -4180,7 +4192,9 @@ static int batch_create_t(dm_batch *b, const int64_t *op_start, const dm_op *ops
   std::vector<double> qvals;
   std::vector<std::vector<int>> chain;  // pass-table indices of each HBM circuit, in order
   std::vector<double> work;             // per HBM circuit: bytes moved (ticket order)
-  uint64_t arena = 0;
+  uint64_t arena = 0, tiles = 0;
+  for (int c = 0; c < b->ncirc; ++c)
+    if (b->nq[c] > lds_max_qubits && b->nq[c] >= kRegTile) tiles += pow4(b->nq[c] - kRegTile);
   for (int c = 0; c < b->ncirc; ++c) {
     if (b->nq[c] <= lds_max_qubits) continue;
     const int j = (int)b->large.size();
@@ -4189,7 +4203,7 @@ static int batch_create_t(dm_batch *b, const int64_t *op_start, const dm_op *ops
     probe.n = b->nq[c];
     probe.dtype = b->dtype;
     probe.N = pow4(probe.n);
-    probe.batched = true;
+    probe.batched = tiles >= (uint64_t)cu;
     BatchPass bp;
     memset(&bp, 0, sizeof(bp));
     bp.circ = j;

@@ -1,7 +1,7 @@
 """Register-resident fused passes against the oracle.
 
-Passes of many single-qubit maps and CX gates on a few qubits take the
-register-resident kernel from 7 qubits up (always from 12).  The cases cover
+Passes of single-qubit maps and CX gates take the register-resident kernel
+from 12 qubits up, and FP64 passes of many operations from 7.  The cases cover
 every place of the operands in the tile (load and store layouts, the digits
 that lie across lanes, tiles of 5-7 digits completed to 7), unital, general
 and diagonal maps, plain CX and CX with separable and general pair scales,
@@ -133,7 +133,8 @@ def with_identity(sub, qubits):
     return sub + [(native.SUB_2Q, list(qubits[:2]), np.eye(16))]
 
 
-@pytest.mark.parametrize('n,m,qubits', [(8, 7, [0, 2, 3, 7]), (9, 6, [0, 1, 4]), (12, 7, [0, 1, 10, 11])])
+@pytest.mark.parametrize('n,m,qubits', [(8, 7, [0, 2, 3, 7]), (9, 6, [0, 1, 4]), (12, 7, [0, 1, 10, 11]),
+                                        (12, 6, [6, 7, 8]), (12, 7, [2, 4, 8, 10]), (12, 7, [8, 9, 10, 11])])
 def test_fp32_passes_equal_the_lds_form_bit_for_bit(n, m, qubits):
     """FP32 keeps the order of operations: the state is the same whichever
     form ran."""
