@@ -2996,6 +2996,17 @@ std::vector<FusedPass> fuse_plain_run(const dm_state *h, const PlainRun &run, co
   std::vector<FusedPass> out;
   const int n = h->n;
   if (run.ops.size() < 2 || n > 18) return out;
+  // kernels of the run one by one
+  double kernels = 0.0;
+  int last = -1;
+  for (int i : run.src) {
+    if (i == last) continue;
+    last = i;
+    const double *pv = params + ops[i].param;
+    const bool feed = ops[i].kind == DM_OP_MEMORY_NOISE && (1 - pv[2]) * (2 * pv[1] - 1) != 0.0;
+    kernels += !feed ? 1 : n >= 12 ? 1 + (n - 4) / 4 : 1 + (n - 4) / 3;
+  }
+  if (kernels < 2) return out;  // (a run that is one memory-noise operation)
   if (n <= 6) {
     RegPlan rp;
     reg_plan(reg_items(run.ops, run.vals, 6), 6, false, false, &rp);
@@ -3015,16 +3026,6 @@ std::vector<FusedPass> fuse_plain_run(const dm_state *h, const PlainRun &run, co
     fp.vals = std::move(rp.vals);
     out.push_back(std::move(fp));
     return out;
-  }
-  // kernels of the run one by one
-  double kernels = 0.0;
-  int last = -1;
-  for (int i : run.src) {
-    if (i == last) continue;
-    last = i;
-    const double *pv = params + ops[i].param;
-    const bool feed = ops[i].kind == DM_OP_MEMORY_NOISE && (1 - pv[2]) * (2 * pv[1] - 1) != 0.0;
-    kernels += !feed ? 1 : n >= 12 ? 1 + (n - 4) / 4 : 1 + (n - 4) / 3;
   }
   const std::vector<std::vector<int>> blocks = plain_blocks(n, run);
   if (blocks.size() * (n < 12 ? 2.0 : 1.4) >= kernels) return out;
