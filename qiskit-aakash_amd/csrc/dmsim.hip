@@ -2895,7 +2895,8 @@ bool plan_reg(const dm_state *h, FusedPass *fp) {
 
 // Runs of single-qubit, CX and memory-noise operations of a program on an
 // FP64 state as fused passes (an FP32 state keeps one kernel per operation:
-// its kernels round differently).
+// its kernels round differently).  Up to 6 qubits, where one kernel takes the
+// whole run, the program's own fused passes join it.
 struct PlainRun {
   std::vector<TileOp> ops;      // digits are positions
   std::vector<double> vals;
@@ -3004,9 +3005,13 @@ std::vector<FusedPass> fuse_plain_run(const dm_state *h, const PlainRun &run, co
     last = i;
     const double *pv = params + ops[i].param;
     const bool feed = ops[i].kind == DM_OP_MEMORY_NOISE && (1 - pv[2]) * (2 * pv[1] - 1) != 0.0;
-    kernels += !feed ? 1 : n >= 12 ? 1 + (n - 4) / 4 : 1 + (n - 4) / 3;
+    kernels += ops[i].kind == DM_OP_FUSED ? 3 : !feed ? 1 : n >= 12 ? 1 + (n - 4) / 4 : 1 + (n - 4) / 3;
   }
-  if (kernels < 2) return out;  // (a run that is one memory-noise operation)
+  // one launch for runs of six kernels or more (5 qubits, 80 gates in dense
+  // blocks with short runs between them: 293 us one by one, 302 with every
+  // run of two and more as one launch; 6 qubits, 80 gates in fused passes:
+  // 176 us one by one, 90 as one launch)
+  if (n <= 6 && kernels < 6) return out;
   if (n <= 6) {
     RegPlan rp;
     reg_plan(reg_items(run.ops, run.vals, 6), 6, false, false, &rp);
@@ -3058,7 +3063,10 @@ std::vector<FusedPass> fuse_plain_run(const dm_state *h, const PlainRun &run, co
   return out;
 }
 
-int parse_fused(const dm_state *h, const double *p, int64_t avail, int opi, FusedPass *fp, bool allow_reg = false) {
+// With `run`, a record of single-qubit and CX operations joins it instead and
+// leaves *fp without operations.
+int parse_fused(const dm_state *h, const double *p, int64_t avail, int opi, FusedPass *fp, bool allow_reg = false,
+                PlainRun *run = nullptr) {
   int64_t at = 0;
   auto next = [&](double *out) -> bool {
     if (at >= avail) return false;
@@ -3153,6 +3161,20 @@ int parse_fused(const dm_state *h, const double *p, int64_t avail, int opi, Fuse
     }
     at += nv;
     fp->ops.push_back(op);
+  }
+  if (run) {
+    for (const TileOp &op : fp->ops)
+      if (op.kind != TOP_1Q && op.kind != TOP_CX) return DM_OK;
+    const int32_t base = (int32_t)run->vals.size();
+    run->vals.insert(run->vals.end(), fp->vals.begin(), fp->vals.end());
+    for (TileOp op : fp->ops) {
+      for (int x = 0; x < (op.kind == TOP_CX ? 2 : 1); ++x) op.d[x] = fp->geo.tpos[op.d[x]];
+      op.param += base;
+      run->ops.push_back(op);
+      run->src.push_back(opi);
+    }
+    fp->ops.clear();
+    return DM_OK;
   }
   if (allow_reg && plan_reg(h, fp)) return DM_OK;
   // LDS layout.  The 64 banks (4 bytes each) are LDS index bits 0-5, tile
@@ -3483,18 +3505,25 @@ int stage_program(dm_state *h, const dm_op *ops, int nops, const double *params,
     pp->fused_of.push_back((int)pp->fused.size());
     pp->fused.push_back(std::move(fp));
   };
+  int one_by_one = 0;  // operations before this one have been found not to gain as a run
   for (int i = 0; i < nops; ++i) {
-    if (ops[i].kind == DM_OP_FUSED) {
-      if (ops[i].param < 0 || ops[i].param >= nparams) return fail(DM_ERR_ARG, "op %d: bad parameter offset", i);
-      FusedPass fp;
-      if (int rc = parse_fused(h, params + ops[i].param, nparams - ops[i].param, i, &fp, true)) return rc;
-      add_fused(ops[i], std::move(fp));
-      continue;
-    }
-    if (sizeof(T) == 8 && fuse_plain && plain_op(ops[i])) {
+    auto fused_args = [&](int j) {
+      return ops[j].param < 0 || ops[j].param >= nparams ? fail(DM_ERR_ARG, "op %d: bad parameter offset", j) : DM_OK;
+    };
+    if (sizeof(T) == 8 && fuse_plain && i >= one_by_one) {
       PlainRun run;
       int e = i;
-      for (; e < nops && plain_op(ops[e]); ++e) add_plain(h->n, ops[e], params, e, &run);
+      for (; e < nops; ++e) {
+        if (plain_op(ops[e])) {
+          add_plain(h->n, ops[e], params, e, &run);
+          continue;
+        }
+        if (h->n > 6 || ops[e].kind != DM_OP_FUSED) break;
+        FusedPass fp;
+        if (int rc = fused_args(e)) return rc;
+        if (int rc = parse_fused(h, params + ops[e].param, nparams - ops[e].param, e, &fp, false, &run)) return rc;
+        if (!fp.ops.empty()) break;
+      }
       std::vector<FusedPass> fps = fuse_plain_run<T>(h, run, ops, params);
       dm_op synth;
       memset(&synth, 0, sizeof(synth));
@@ -3507,11 +3536,17 @@ int stage_program(dm_state *h, const dm_op *ops, int nops, const double *params,
         pp->ops.push_back(ops[fp.plain]);
         pp->fused_of.push_back(-1);
       }
-      for (int j = i; fps.empty() && j < e; ++j) {
-        pp->ops.push_back(ops[j]);
-        pp->fused_of.push_back(-1);
+      if (!fps.empty()) {
+        i = e - 1;
+        continue;
       }
-      i = e - 1;
+      one_by_one = e;
+    }
+    if (ops[i].kind == DM_OP_FUSED) {
+      if (int rc = fused_args(i)) return rc;
+      FusedPass fp;
+      if (int rc = parse_fused(h, params + ops[i].param, nparams - ops[i].param, i, &fp, true)) return rc;
+      add_fused(ops[i], std::move(fp));
       continue;
     }
     if (ops[i].kind == DM_OP_BLOCK) pool += (size_t)1 << (4 * ops[i].k);
