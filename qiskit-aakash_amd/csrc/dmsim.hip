@@ -2844,10 +2844,15 @@ void set_reg(FusedPass *fp, RegPlan &&rp, const RegTile &t) {
 // operations in a tile that holds the positions 0-2 (64 consecutive
 // coefficients per access).  The grid is one workgroup of 256 threads per
 // tile, so 18 qubits are the most that fit the 2^32 work items of a launch.
-// From 12 qubits on it is faster for any pass (16 qubits, one / 8 / 16 pairs
-// of a single-qubit map and a CX on three digits: FP32 6.0 / 6.5 / 7.1 ms
-// against 6.7 / 7.7 / 14.3 with the tile in LDS, FP64 12.0 / 12.6 / 16.4
-// against 13.1 / 15.5 / 24.8).  Below, a launch is a few workgroups per CU
+// From 12 qubits on it is faster for FP64 passes (16 qubits, one / 8 / 16
+// pairs of a single-qubit map and a CX on three digits: 12.0 / 12.6 / 16.4 ms
+// against 13.1 / 15.5 / 24.8) and for FP32 passes inside the last-level cache
+// (13 qubits, 7-32 members: 93-171 us against 107-197).  Above it an FP32
+// pass of few members is bound by HBM in either form, and the persistent
+// tile-in-LDS kernel walks the state at least as well (16 qubits, 33 passes
+// of 3-11 members: 6.59 ms each in LDS against 6.60; single ones on positions
+// 8-12 up to 1.6 ms less); passes of 12 members and more take 6.78 ms in
+// registers against 7.99.  Below 12 qubits, a launch is a few workgroups per CU
 // and its latency counts: the tile-in-LDS kernel's 6-digit tiles fill more
 // CUs, and in FP32 the operations in order need too many redistributions (300
 // gates on 9 / 11 qubits, matching, learned: 437 / 494 us in LDS against 463 /
@@ -2861,6 +2866,7 @@ void set_reg(FusedPass *fp, RegPlan &&rp, const RegTile &t) {
 bool plan_reg(const dm_state *h, FusedPass *fp) {
   if (h->n < kRegTile || h->n > 18) return false;
   const bool few = h->n < 12 && !h->batched;
+  const bool light = h->dtype == DM_FP32 && h->N * 4 > (256ull << 20);
   if (few && (h->dtype == DM_FP32 || fp->ops.size() < 12 || (fp->m < 7 && h->n < 11))) return false;
   for (const TileOp &op : fp->ops)
     if (op.kind != TOP_1Q && op.kind != TOP_CX) return false;
@@ -2889,6 +2895,7 @@ bool plan_reg(const dm_state *h, FusedPass *fp) {
   RegPlan rp;
   reg_plan(ordered ? reg_items_in_order(ops, vals) : reg_items(ops, vals, kRegTile), kRegTile, true, ordered, &rp);
   if (few && ops.size() < 4 * (size_t)rp.ns) return false;
+  if (light && rp.vals.size() / kRegVals - 1 < 12) return false;
   set_reg(fp, std::move(rp), t);
   return true;
 }
