@@ -4313,15 +4313,15 @@ static int batch_create_t(dm_batch *b, const int64_t *op_start, const dm_op *ops
     std::vector<int> order(chain.size());
     for (size_t j = 0; j < order.size(); ++j) order[j] = (int)j;
     std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return work[x] > work[y]; });
-    constexpr uint64_t kCacheBytes = 200ull << 20;
+    constexpr uint64_t kCacheBytes = 200ull << 20, kOneGroup = 300ull << 20;
     uint64_t total = 0, largest = 1;
     for (const auto &ids : chain) {
       const uint64_t bytes = pow4(passes[ids[0]].n) * sizeof(T);
       total += bytes;
       largest = std::max(largest, bytes);
     }
-    const int chains = total <= kCacheBytes ? 1 : largest * 3 <= kCacheBytes ? 3 : 2;
-    const uint64_t group_bytes = kCacheBytes / chains;
+    const int chains = total <= kOneGroup ? 1 : largest * 3 <= kCacheBytes ? 3 : 2;
+    const uint64_t group_bytes = chains == 1 ? kOneGroup : kCacheBytes / chains;
     std::vector<double> load(chains, 0.0);
     for (size_t g0 = 0; g0 < order.size();) {
       size_t g1 = g0;

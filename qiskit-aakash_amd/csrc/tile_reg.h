@@ -685,6 +685,11 @@ inline void reg_plan(const std::vector<RegItem> &items, int m, bool io, bool ord
     for (int b = a + 1; b < m; ++b)
       for (int c = b + 1; c < m; ++c) triples[nt++] = (1u << a) | (1u << b) | (1u << c);
   std::vector<char> done(items.size(), 0);
+  // pending items inside each triple: no more than these can be taken, so a
+  // triple is looked at only if it may beat the best one so far
+  int inside[35] = {0};
+  for (const RegItem &it : items)
+    for (uint32_t t = 0; t < nt; ++t) inside[t] += (it.mask & ~triples[t]) == 0;
   std::vector<uint32_t> stage;
   std::vector<std::vector<int>> members;
   size_t first = 0, left = items.size();
@@ -695,6 +700,7 @@ inline void reg_plan(const std::vector<RegItem> &items, int m, bool io, bool ord
       if (!stage.empty() && !(triples[t] & stage.back())) continue;  // a redistribution keeps one digit
       // in order, the first pending item comes first
       if (ordered && left && !(io && stage.empty()) && (items[first].mask & ~triples[t])) continue;
+      if (inside[t] <= most) continue;
       const int n = reg_absorb(items, done, first, triples[t], ordered, nullptr);
       if (n > most) {
         most = n;
@@ -703,7 +709,10 @@ inline void reg_plan(const std::vector<RegItem> &items, int m, bool io, bool ord
     }
     std::vector<int> take;
     reg_absorb(items, done, first, triples[best], ordered, &take);
-    for (int i : take) done[i] = 1;
+    for (int i : take) {
+      done[i] = 1;
+      for (uint32_t t = 0; t < nt; ++t) inside[t] -= (items[i].mask & ~triples[t]) == 0;
+    }
     left -= take.size();
     while (first < items.size() && done[first]) ++first;
     stage.push_back(triples[best]);
