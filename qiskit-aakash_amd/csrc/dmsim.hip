@@ -2847,11 +2847,11 @@ void set_reg(FusedPass *fp, RegPlan &&rp, const RegTile &t) {
 // From 12 qubits on it is faster for FP64 passes (16 qubits, one / 8 / 16
 // pairs of a single-qubit map and a CX on three digits: 12.0 / 12.6 / 16.4 ms
 // against 13.1 / 15.5 / 24.8) and for FP32 passes inside the last-level cache
-// (13 qubits, 7-32 members: 93-171 us against 107-197).  Above it an FP32
-// pass of few members is bound by HBM in either form, and the persistent
+// (13 qubits, 7-32 maps, CX and scales: 93-171 us against 107-197).  Above it an FP32
+// pass of few operations is bound by HBM in either form, and the persistent
 // tile-in-LDS kernel walks the state at least as well (16 qubits, 33 passes
-// of 3-11 members: 6.59 ms each in LDS against 6.60; single ones on positions
-// 8-12 up to 1.6 ms less); passes of 12 members and more take 6.78 ms in
+// of 3-11 maps, CX and scales: 6.59 ms each in LDS against 6.60; single ones on positions
+// 8-12 up to 1.6 ms less); passes of 12 and more take 6.77 ms in
 // registers against 7.99.  Below 12 qubits, a launch is a few workgroups per CU
 // and its latency counts: the tile-in-LDS kernel's 6-digit tiles fill more
 // CUs, and in FP32 the operations in order need too many redistributions (300
@@ -2892,10 +2892,11 @@ bool plan_reg(const dm_state *h, FusedPass *fp) {
   }
   for (TileOp &op : ops)
     for (int x = 0; x < (op.kind == TOP_CX ? 2 : 1); ++x) op.d[x] = t.digit[fp->geo.tpos[op.d[x]]];
+  const std::vector<RegItem> reg_ops = ordered ? reg_items_in_order(ops, vals) : reg_items(ops, vals, kRegTile);
+  if (light && reg_ops.size() < 12) return false;
   RegPlan rp;
-  reg_plan(ordered ? reg_items_in_order(ops, vals) : reg_items(ops, vals, kRegTile), kRegTile, true, ordered, &rp);
+  reg_plan(reg_ops, kRegTile, true, ordered, &rp);
   if (few && ops.size() < 4 * (size_t)rp.ns) return false;
-  if (light && rp.vals.size() / kRegVals - 1 < 12) return false;
   set_reg(fp, std::move(rp), t);
   return true;
 }

@@ -19,6 +19,7 @@ enum {
   RM_CX = 6,    // + pair: CX, no values; pairs (control, target) (0,1) (1,0) (0,2) (2,0) (1,2) (2,1)
   RM_D1 = 12,   // + slot: scale components X, Y, Z by 3 values
   RM_D2 = 15,   // + pair of slots (0,1) (0,2) (1,2): 16 scales, index 4 i_first + i_second
+  RM_CXD = 18,  // + pair as RM_CX: CX, then 16 scales, index 4 i_control + i_target
 };
 
 struct RegStage {
@@ -131,6 +132,35 @@ __device__ __forceinline__ void reg_cx(T (&v)[64]) {
   }
 }
 
+// The same followed by the pair's scales; the two signs go into their scales
+// (the product has the same bits).  A pair that swaps is two products and a
+// copy, against a swap, two products and a separate member (13 qubits FP32:
+// 2.86 -> 2.70 ms, 16 qubits FP32 504 -> 498 ms).
+template <typename T, int C, int TG>
+__device__ __forceinline__ void reg_cxd(T (&v)[64], const T (&pv)[kRegVals]) {
+  constexpr int SC = 1 << (2 * C), ST = 1 << (2 * TG), SO = 1 << (2 * (3 - C - TG));
+  T d[16];
+#pragma unroll
+  for (int i = 1; i < 16; ++i) d[i] = pv[i];
+  d[7] = -d[7];
+  d[10] = -d[10];
+#pragma unroll
+  for (int o = 0; o < 4; ++o) {
+    auto X = [&](int i) -> T & { return v[o * SO + (i >> 2) * SC + (i & 3) * ST]; };
+    constexpr int pairs[6][2] = {{2, 14}, {3, 15}, {4, 5}, {6, 11}, {8, 9}, {7, 10}};
+#pragma unroll
+    for (int p = 0; p < 6; ++p) {
+      const int i = pairs[p][0], j = pairs[p][1];
+      const T t = d[i] * X(j);
+      X(j) = d[j] * X(i);
+      X(i) = t;
+    }
+    X(1) *= d[1];
+    X(12) *= d[12];
+    X(13) *= d[13];
+  }
+}
+
 template <typename T, int SLOT>
 __device__ __forceinline__ void reg_d1(T (&v)[64], const T (&pv)[kRegVals]) {
   constexpr int S = 1 << (2 * SLOT);
@@ -197,7 +227,13 @@ __device__ __forceinline__ void reg_members(T (&v)[64], const uint32_t *__restri
       case RM_D1 + 2: reg_d1<T, 2>(v, pv); break;
       case RM_D2 + 0: reg_d2<T, 0, 1>(v, pv); break;
       case RM_D2 + 1: reg_d2<T, 0, 2>(v, pv); break;
-      default: reg_d2<T, 1, 2>(v, pv); break;
+      case RM_D2 + 2: reg_d2<T, 1, 2>(v, pv); break;
+      case RM_CXD + 0: reg_cxd<T, 0, 1>(v, pv); break;
+      case RM_CXD + 1: reg_cxd<T, 1, 0>(v, pv); break;
+      case RM_CXD + 2: reg_cxd<T, 0, 2>(v, pv); break;
+      case RM_CXD + 3: reg_cxd<T, 2, 0>(v, pv); break;
+      case RM_CXD + 4: reg_cxd<T, 1, 2>(v, pv); break;
+      default: reg_cxd<T, 2, 1>(v, pv); break;
     }
   }
 }
@@ -803,8 +839,8 @@ inline void reg_plan(const std::vector<RegItem> &items, int m, bool io, bool ord
     memset(&sg, 0, sizeof(sg));
     sg.mem = (uint32_t)kinds.size();
     auto slot = [&](int d) { return lay[k].r[0] == d ? 0 : lay[k].r[1] == d ? 1 : 2; };
-    for (int i : members[k]) {
-      const RegItem &it = items[i];
+    for (size_t x = 0; x < members[k].size(); ++x) {
+      const RegItem &it = items[members[k][x]];
       double v[kRegVals] = {0.0};
       uint32_t kind;
       if (it.kind == 0) {
@@ -819,7 +855,16 @@ inline void reg_plan(const std::vector<RegItem> &items, int m, bool io, bool ord
         const int s0 = slot(it.d0), s1 = slot(it.d1);
         const int lo = std::min(s0, s1), hi = std::max(s0, s1);
         const int pair = lo == 0 ? hi - 1 : 2;  // (0,1) (0,2) (1,2)
-        if (it.kind == 1) {
+        const RegItem *scale = nullptr;  // the scale of this CX, if it comes next
+        if (it.kind == 1 && x + 1 < members[k].size()) {
+          scale = &items[members[k][x + 1]];
+          if (scale->kind != 2 || scale->d0 != it.d0 || scale->d1 != it.d1) scale = nullptr;
+        }
+        if (scale) {
+          kind = RM_CXD + 2 * pair + (s0 > s1 ? 1 : 0);
+          memcpy(v, scale->v, 16 * sizeof(double));
+          ++x;
+        } else if (it.kind == 1) {
           kind = RM_CX + 2 * pair + (s0 > s1 ? 1 : 0);
         } else {
           kind = RM_D2 + pair;
