@@ -231,9 +231,9 @@ int dm_mlp_train(float *params, int n_features, int hidden, const float *X, cons
  * 6-digit tile pass (DM_OP_FUSED with tile size 6, DM_OP_1Q, DM_OP_CX[_SCALED],
  * DM_OP_2Q, DM_OP_MEMORY_NOISE; memory noise as 1-qubit channels, 6 qubits
  * per pass; in FP32 also DM_OP_FUSED with tile size 7 holding single-qubit
- * and CX operations).  The circuits run in groups: one group while all
- * states fit the last-level cache together, else groups that do, in two or
- * three chains side by side.  Round r of a group holds pass r of its
+ * and CX operations).  The circuits run in groups: one group up to 300 MiB
+ * of states, else groups that fit the last-level cache, in two or three
+ * chains side by side.  Round r of a group holds pass r of its
  * circuits, plus the |0..0> initialisation first and the probabilities last:
  * its initialisation and probability work (split into at most items_per_pass
  * items per pass) is one grid-stride launch, and its passes of 6-digit and of

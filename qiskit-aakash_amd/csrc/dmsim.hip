@@ -3301,10 +3301,12 @@ int launch_fused(dm_state *h, const FusedPass &fp, const uint32_t *d_recs, const
   if (fp.reg) {
     const RegStage *st = reinterpret_cast<const RegStage *>(d_recs);
     const uint32_t *mem = reinterpret_cast<const uint32_t *>(st + fp.reg_stages);
-    if (fp.whole) {
-      hipLaunchKernelGGL((k_state_reg<T>), dim3(1), dim3(64), 0, h->stream, static_cast<T *>(h->d_a), fp.reg_whole, st,
-                         mem, d_vals);
-      return last_launch("k_state_reg");
+    if constexpr (sizeof(T) == 8) {
+      if (fp.whole) {  // (FP64 programs only)
+        hipLaunchKernelGGL((k_state_reg<T>), dim3(1), dim3(64), 0, h->stream, static_cast<T *>(h->d_a), fp.reg_whole,
+                           st, mem, d_vals);
+        return last_launch("k_state_reg");
+      }
     }
     // states above the 256 MB of the last-level cache stream with
     // nontemporal accesses (16 qubits, FP32: 6.0 against 6.4 ms a pass), the
@@ -4300,8 +4302,10 @@ static int batch_create_t(dm_batch *b, const int64_t *op_start, const dm_op *ops
   b->npasses = (int64_t)passes.size();
 
   // Items in round order: round r of a group holds pass r of every circuit
-  // of the group that has one.  Batches whose states fit the 256 MB
-  // last-level cache together are one group.  Larger ones form groups, most
+  // of the group that has one.  Batches of up to 300 MiB of states are one
+  // group, the 256 MB last-level cache holds most of it (152 FP32 circuits of
+  // 8-10 qubits, 273 MB: 2.4 ms, in groups 3.4; 20 of 11 qubits, 335 MB, one
+  // group 2.49, groups 2.32).  Larger ones form groups, most
   // work first, that run one after another in two or three chains (a stream
   // each): all but a state's first pass then read what the pass before left
   // in the cache, and the chains fill each other's launch gaps and tails.

@@ -4,14 +4,14 @@ Each circuit follows the reference's semantics for a circuit with a barrier
 after every gate: the gate, then memory noise on every qubit (one level per
 gate, dm_simulator.py:1172-1177), and finally an ensemble Z measurement of
 all qubits with polarisation retention ``depolarization_factor``.  Small
-registers (<= ``lds_max_qubits``) run whole inside one workgroup's LDS; the
-others keep their state in one HBM arena and run as fused 6-digit tile
+registers (<= ``lds_max_qubits``) run whole inside one workgroup, in
+registers or in LDS; the others keep their state in one HBM arena and run as fused 6-digit tile
 passes (7-digit in FP32 where 6 digits would leave contiguous runs of 4^2
-or 4^3 coefficients that 7 digits lengthen), in groups whose states stay
-in the last-level cache; round r of a group (pass r of its circuits) is up
-to three launches: the initialisation and probability work, split into at
-most ``items_per_pass`` work items per pass, and one launch per tile size
-with a workgroup per tile; the batch is captured once into a hipGraph and
+or 4^3 coefficients that 7 digits lengthen), in one group up to 300 MiB of
+states and in groups that stay in the last-level cache above; round r of a
+group (pass r of its circuits) is up to four launches: the initialisation
+and probability work, split into at most ``items_per_pass`` work items per
+pass, and one launch per tile form with a workgroup per tile; the batch is captured once into a hipGraph and
 replayed (``dm_batch_*`` in dmsim.h).
 
 ``autotune`` picks the LDS cutoff width, the LDS workgroup size and the
