@@ -3499,9 +3499,13 @@ struct Prepared {
   size_t image_bytes() const { return vals_at + values.size(); }
 };
 
+// `in_registers` false: no runs of single operations and no register-resident
+// passes, whose image is larger where passes have few operations (one map on
+// position 0, FP64: three stage records and a spare member, 504 bytes against
+// 168).
 template <typename T>
 int stage_program(dm_state *h, const dm_op *ops, int nops, const double *params, int64_t nparams, Prepared *pp,
-                  bool fuse_plain = true) {
+                  bool in_registers = true) {
   pp->params.assign(params, params + (nparams > 0 ? nparams : 0));
   pp->ops.clear();
   pp->fused.clear();
@@ -3520,7 +3524,7 @@ int stage_program(dm_state *h, const dm_op *ops, int nops, const double *params,
     auto fused_args = [&](int j) {
       return ops[j].param < 0 || ops[j].param >= nparams ? fail(DM_ERR_ARG, "op %d: bad parameter offset", j) : DM_OK;
     };
-    if (sizeof(T) == 8 && fuse_plain && i >= one_by_one) {
+    if (sizeof(T) == 8 && in_registers && i >= one_by_one) {
       PlainRun run;
       int e = i;
       for (; e < nops; ++e) {
@@ -3555,7 +3559,7 @@ int stage_program(dm_state *h, const dm_op *ops, int nops, const double *params,
     if (ops[i].kind == DM_OP_FUSED) {
       if (int rc = fused_args(i)) return rc;
       FusedPass fp;
-      if (int rc = parse_fused(h, params + ops[i].param, nparams - ops[i].param, i, &fp, true)) return rc;
+      if (int rc = parse_fused(h, params + ops[i].param, nparams - ops[i].param, i, &fp, in_registers)) return rc;
       add_fused(ops[i], std::move(fp));
       continue;
     }
@@ -3740,7 +3744,7 @@ template <typename T>
 int run_program_noalloc(dm_state *h, const dm_op *ops, int nops, const double *params, int64_t nparams) {
   Prepared pp;
   if (int rc = stage_program<T>(h, ops, nops, params, nparams, &pp)) return rc;
-  // the image of fused runs is not what a program of single operations may
+  // a larger image of the register-resident forms is not what a program may
   // be refused for
   if (pp.image_bytes() > kNoAllocScratchBytes)
     if (int rc = stage_program<T>(h, ops, nops, params, nparams, &pp, false)) return rc;

@@ -75,3 +75,21 @@ def test_noalloc_refuses_an_image_above_its_scratch():
     assert 'exceeds' in native.last_error()
     assert np.array_equal(st.download(), before)
     st.close()
+
+
+@pytest.mark.parametrize('precision', ['fp64', 'fp32'])
+def test_noalloc_takes_passes_whose_register_form_exceeds_the_scratch(precision):
+    """25,001 passes of one X gate on the last qubit: with the tile in LDS a
+    pass is two 36-byte records and 12 values, 4.2 MB (FP64) or 3.0 MB in
+    all; the register-resident form's three 80-byte stages, member and spare
+    make 12.6 or 9.4 MB.  X only negates, so the result is exact."""
+    n = 12
+    prog = Program(n)
+    R = ptm.rows3(np.diag([1.0, 1.0, -1.0, -1.0]))
+    for _ in range(25001):
+        prog.fused(6, [n - 1], [(native.SUB_1Q, [n - 1], R)])
+    got = run(prog, n, precision, 'dm_run_program_noalloc')
+    st = native.DeviceState(n, precision)
+    st.init_product(np.array([1.0, 0.0, 0.0, 1.0] * (n - 1) + [1.0, 0.0, 0.0, -1.0]), 0.5 ** n)
+    assert np.array_equal(got, st.download())
+    st.close()
