@@ -21,6 +21,7 @@
 #include <vector>
 
 #include "dmsim.h"
+#include "reg_plan.h"
 
 namespace {
 
@@ -633,22 +634,8 @@ __global__ __launch_bounds__(kBlock) void k_block_mfma(T *__restrict__ a, const 
 // other operation of a pass into a stage member (group_stages), marks the
 // single-qubit members whose PTM is unital (first column (0, 0, 0): no term
 // in the identity component) as TOP_1QU, and gives every CX member its 16
-// scales (ones for a plain CX).
+// scales (ones for a plain CX).  TileOp and the kinds: reg_plan.h.
 // ---------------------------------------------------------------------------
-
-enum { TOP_1Q = 1, TOP_CX = 2, TOP_2Q = 3, TOP_DENSE = 4, TOP_STAGE = 6, TOP_1QU = 7 };
-
-struct TileOp {
-  int32_t kind, k, d[4], param;
-  // Swizzled passes: the order in which a thread's group index g enumerates
-  // the tile digits the operation leaves free (3 bits per digit, first digit
-  // in bits 0-2); the first ones cover distinct bank fields (lds_swz).
-  int32_t lanes;
-  // FP32 stages on digits >= 1 with 8-byte LDS accesses along digit 0: the
-  // order of the free digits other than digit 0, the first two covering the
-  // bank fields of LDS index bits 2-3 and 4-5.
-  int32_t qlanes;
-};
 
 struct TileGeom {
   int m;                  // tile digits (== template M)
@@ -2899,102 +2886,6 @@ bool plan_reg(const dm_state *h, FusedPass *fp) {
   if (few && ops.size() < 4 * (size_t)rp.ns) return false;
   set_reg(fp, std::move(rp), t);
   return true;
-}
-
-// Runs of single-qubit, CX and memory-noise operations of a program on an
-// FP64 state as fused passes (an FP32 state keeps one kernel per operation:
-// its kernels round differently).  Up to 6 qubits, where one kernel takes the
-// whole run, the program's own fused passes join it.
-struct PlainRun {
-  std::vector<TileOp> ops;      // digits are positions
-  std::vector<double> vals;
-  std::vector<int> src;         // program operation of each
-};
-
-bool plain_op(const dm_op &op) {
-  return op.kind == DM_OP_1Q || op.kind == DM_OP_CX || op.kind == DM_OP_CX_SCALED || op.kind == DM_OP_MEMORY_NOISE;
-}
-
-void add_plain(int n, const dm_op &op, const double *params, int src, PlainRun *run) {
-  TileOp t;
-  memset(&t, 0, sizeof(t));
-  t.param = (int32_t)run->vals.size();
-  auto put = [&](const double *v, int nv) { run->vals.insert(run->vals.end(), v, v + nv); };
-  const double *pv = params + op.param;
-  if (op.kind == DM_OP_MEMORY_NOISE) {
-    const double f = pv[0], p = pv[1], g = pv[2];
-    if (f == 1.0 && g == 1.0) return;
-    const double od = sqrt(g) * f, dd = (1 - g) * (2 * p - 1);
-    const double R[12] = {0, od, 0, 0, 0, 0, od, 0, dd, 0, 0, g};
-    put(R, 12);
-    t.kind = TOP_1Q;
-    t.k = 1;
-    for (int d = 0; d < n; ++d) {
-      t.d[0] = d;
-      run->ops.push_back(t);
-      run->src.push_back(src);
-    }
-    return;
-  }
-  t.d[0] = n - 1 - op.qubits[0];
-  if (op.kind == DM_OP_1Q) {
-    t.kind = TOP_1Q;
-    t.k = 1;
-    put(pv, 12);
-  } else {
-    t.kind = TOP_CX;
-    t.d[1] = n - 1 - op.qubits[1];
-    t.k = op.kind == DM_OP_CX_SCALED ? 1 : 0;
-    if (t.k) put(pv, 16);
-  }
-  run->ops.push_back(t);
-  run->src.push_back(src);
-}
-
-// Blocks of the run: the operations that the tile of the positions 0-2 and
-// up to four others takes (an operation joins unless it, or an earlier one
-// left out that shares a position with it, reaches outside), the others
-// chosen by growth from the first pending operation, with and without one
-// position forced in, whichever takes the most operations.
-std::vector<std::vector<int>> plain_blocks(int n, const PlainRun &run) {
-  const int no = (int)run.ops.size();
-  std::vector<uint32_t> mask(no);
-  for (int i = 0; i < no; ++i) {
-    mask[i] = 1u << run.ops[i].d[0];
-    if (run.ops[i].kind == TOP_CX) mask[i] |= 1u << run.ops[i].d[1];
-  }
-  const uint32_t low = 7u, full = (1u << n) - 1u;
-  const int most_high = std::min(4, n - 3);
-  std::vector<char> done(no, 0);
-  std::vector<std::vector<int>> out;
-  int first = 0, left = no;
-  std::vector<int> cur, best;
-  while (left) {
-    while (done[first]) ++first;
-    best.clear();
-    for (int force = -1; force < n; ++force) {
-      if (force >= 0 && force < 3) continue;
-      uint32_t T = force < 0 ? 0 : 1u << force, blocked = 0;
-      cur.clear();
-      for (int i = first; i < no; ++i) {
-        if (done[i]) continue;
-        const uint32_t m = mask[i], t2 = T | (m & ~low);
-        if ((m & blocked) || __builtin_popcount(t2) > most_high) {
-          blocked |= m;
-          const uint32_t open = __builtin_popcount(T) < most_high ? full : T | low;
-          if (!(open & ~blocked)) break;
-        } else {
-          T = t2;
-          cur.push_back(i);
-        }
-      }
-      if (cur.size() > best.size()) best = cur;
-    }
-    for (int i : best) done[i] = 1;
-    left -= (int)best.size();
-    out.push_back(best);
-  }
-  return out;
 }
 
 // The passes that replace the run, or none if one kernel per operation is

@@ -8,32 +8,7 @@
 // digits without touching LDS; between stages the tile is redistributed
 // through LDS once so that the next three digits are in registers.
 
-constexpr int kRegTile = 7;
 constexpr int kRegThreads = 256;
-constexpr int kRegVals = 16;  // values of one member (unused ones zero)
-
-// Members of a stage.  A slot is a register digit (0, 1, 2).
-enum {
-  RM_U1 = 0,    // + slot: unital single-qubit map, 9 values (3x3, rows X Y Z)
-  RM_A1 = 3,    // + slot: general single-qubit map, 12 values (rows X Y Z, columns I X Y Z)
-  RM_CX = 6,    // + pair: CX, no values; pairs (control, target) (0,1) (1,0) (0,2) (2,0) (1,2) (2,1)
-  RM_D1 = 12,   // + slot: scale components X, Y, Z by 3 values
-  RM_D2 = 15,   // + pair of slots (0,1) (0,2) (1,2): 16 scales, index 4 i_first + i_second
-  RM_CXD = 18,  // + pair as RM_CX: CX, then 16 scales, index 4 i_control + i_target
-};
-
-struct RegStage {
-  uint32_t nm, mem;       // members: count, first one
-  // redistribution into this stage (unused in the first): the slot whose
-  // digit is a register digit before and after (it orders the phases), and
-  // the LDS offset (coefficients) of one unit of each other digit, for the
-  // writer's layout (the previous stage) and the reader's (this stage); a
-  // coefficient's offset is the XOR of its digits times their offsets
-  uint32_t slot;
-  uint32_t wr[3], wl[3], ww;
-  uint32_t rr[3], rl[3], rw;
-  uint32_t pad[3];
-};
 
 struct RegGeom {
   int nr;
@@ -501,421 +476,6 @@ __global__ __launch_bounds__(64, 2) void k_state_reg(T *__restrict__ a, RegWhole
       if (in) a[o] = v[i];
     }
   }
-}
-
-// ---------------------------------------------------------------------------
-// Host: the register program of a fused pass.
-// ---------------------------------------------------------------------------
-
-struct RegItem {
-  uint32_t mask;       // tile digits
-  int kind;            // 0: single-qubit map, 1: CX, 2: pair scale
-  bool scaled;         // CX with 16 pair scales
-  bool exact;          // rounds nothing (a CX permutation)
-  int d0, d1;
-  double v[16];        // rows X, Y, Z (12 values), or 16 pair scales
-};
-
-// Kind and values of a single-qubit map: identity (no member), diagonal,
-// unital or general.
-inline int reg_1q_kind(const double *r) {
-  bool unital = true, diag = true, ident = true;
-  for (int i = 0; i < 3; ++i) {
-    if (r[4 * i] != 0.0) unital = false;
-    for (int j = 0; j < 3; ++j) {
-      const double x = r[4 * i + 1 + j];
-      if (i != j && x != 0.0) diag = false;
-      if (x != (i == j ? 1.0 : 0.0)) ident = false;
-    }
-  }
-  if (!unital) return RM_A1;
-  return ident ? -1 : diag ? RM_D1 : RM_U1;
-}
-
-// The operations of a pass in their given order, one item each (two for a
-// scaled CX: the permutation and the scale).
-inline std::vector<RegItem> reg_items_in_order(const std::vector<TileOp> &ops, const std::vector<double> &vals) {
-  std::vector<RegItem> out;
-  out.reserve(2 * ops.size());
-  for (const TileOp &op : ops) {
-    const double *v = vals.data() + op.param;
-    RegItem it;
-    it.scaled = false;
-    it.d0 = op.d[0];
-    if (op.kind == TOP_1Q || op.kind == TOP_1QU) {
-      it.kind = 0;
-      it.d1 = op.d[0];
-      it.mask = 1u << op.d[0];
-      it.exact = false;
-      memcpy(it.v, v, 12 * sizeof(double));
-      out.push_back(it);
-      continue;
-    }
-    it.kind = 1;
-    it.d1 = op.d[1];
-    it.mask = (1u << it.d0) | (1u << it.d1);
-    it.exact = true;
-    out.push_back(it);
-    bool scaled = false;
-    for (int i = 1; op.k && i < 16; ++i) scaled = scaled || v[i] != 1.0;
-    if (scaled) {
-      it.kind = 2;
-      it.exact = false;
-      memcpy(it.v, v, 16 * sizeof(double));
-      out.push_back(it);
-    }
-  }
-  return out;
-}
-
-// The pass's operations as register-stage items, free to be reordered where
-// they commute: runs of single-qubit maps on one digit become one map, and
-// the separable scale of a CX (a depolarising channel on each of its qubits)
-// goes into the next map on either digit where one follows before another
-// CX, so that the CX itself only permutes registers; what is left stays as a
-// scale of its own.
-inline std::vector<RegItem> reg_items(const std::vector<TileOp> &ops, const std::vector<double> &vals, int m) {
-  std::vector<RegItem> out;
-  out.reserve(2 * ops.size());
-  int pend[8];  // item index of the single-qubit map a digit's next one joins, or -1
-  for (int d = 0; d < m; ++d) pend[d] = -1;
-  for (const TileOp &op : ops) {
-    const double *v = vals.data() + op.param;
-    if (op.kind == TOP_1Q) {
-      const int d = op.d[0];
-      if (pend[d] < 0) {
-        RegItem it;
-        it.mask = 1u << d;
-        it.kind = 0;
-        it.scaled = it.exact = false;
-        it.d0 = it.d1 = d;
-        memcpy(it.v, v, 12 * sizeof(double));
-        pend[d] = (int)out.size();
-        out.push_back(it);
-      } else {
-        // (I, X, Y, Z) -> rows of the later map applied to the earlier one
-        double *e = out[pend[d]].v, w[12];
-        for (int i = 0; i < 3; ++i)
-          for (int j = 0; j < 4; ++j) {
-            double acc = j == 0 ? v[4 * i] : 0.0;
-            for (int k = 0; k < 3; ++k) acc += v[4 * i + 1 + k] * e[4 * k + j];
-            w[4 * i + j] = acc;
-          }
-        memcpy(e, w, sizeof(w));
-      }
-    } else {
-      RegItem it;
-      it.d0 = op.d[0];
-      it.d1 = op.d[1];
-      it.mask = (1u << it.d0) | (1u << it.d1);
-      it.kind = 1;
-      it.scaled = op.k != 0;
-      it.exact = false;
-      if (op.k) memcpy(it.v, v, 16 * sizeof(double));
-      out.push_back(it);
-      pend[it.d0] = pend[it.d1] = -1;
-    }
-  }
-  // scales
-  std::vector<RegItem> res;
-  res.reserve(out.size() + 8);
-  for (size_t i = 0; i < out.size(); ++i) {
-    const RegItem it = out[i];
-    if (it.kind != 1 || !it.scaled) {
-      res.push_back(it);
-      continue;
-    }
-    bool scaled = false, separable = it.v[0] == 1.0;
-    for (int c = 0; c < 4; ++c)
-      for (int t = 0; t < 4; ++t) {
-        const double s = it.v[4 * c + t];
-        if (s != 1.0 && (c | t)) scaled = true;
-        if (!(fabs(s - it.v[4 * c] * it.v[t]) <= 4e-16 * fabs(s))) separable = false;
-      }
-    RegItem cx = it;
-    cx.scaled = false;
-    res.push_back(cx);
-    if (!scaled) continue;
-    RegItem *next[2] = {nullptr, nullptr};
-    if (separable)
-      for (int s = 0; s < 2; ++s) {
-        const uint32_t bit = 1u << (s ? it.d1 : it.d0);
-        for (size_t j = i + 1; j < out.size(); ++j)
-          if (out[j].mask & bit) {
-            if (out[j].kind == 0) next[s] = &out[j];
-            break;
-          }
-      }
-    for (int s = 0; s < 2; ++s)
-      if (next[s])
-        for (int r = 0; r < 3; ++r)
-          for (int c = 1; c < 4; ++c) next[s]->v[4 * r + c] *= s ? it.v[c] : it.v[4 * c];
-    if (next[0] && next[1]) continue;
-    RegItem d = it;
-    if (!next[0] && !next[1]) {
-      d.kind = 2;
-    } else {
-      const int s = next[0] ? 1 : 0;
-      d.kind = 0;
-      d.d0 = d.d1 = s ? it.d1 : it.d0;
-      d.mask = 1u << d.d0;
-      for (int r = 0; r < 3; ++r)
-        for (int c = 0; c < 4; ++c) d.v[4 * r + c] = c == r + 1 ? (s ? it.v[c] : it.v[4 * c]) : 0.0;
-    }
-    res.push_back(d);
-  }
-  return res;
-}
-
-// Items (of those with done[i] == 0) that a stage on the digits of `triple`
-// takes: an item joins unless it, or an earlier one left out that it does
-// not commute with, reaches outside the triple.  Items on different digits
-// commute; with `ordered` (results bit for bit those of the given order)
-// only if one of them rounds nothing.
-inline int reg_absorb(const std::vector<RegItem> &items, const std::vector<char> &done, size_t first, uint32_t triple,
-                      bool ordered, std::vector<int> *take) {
-  uint32_t blocked = 0;
-  bool rounded = false;  // an item that rounds was left out
-  int n = 0;
-  for (size_t i = first; i < items.size(); ++i) {
-    if (done[i]) continue;
-    const uint32_t m = items[i].mask;
-    if ((m & blocked) || (m & ~triple) || (ordered && rounded && !items[i].exact)) {
-      blocked |= m;
-      rounded = rounded || !items[i].exact;
-      if (!(triple & ~blocked)) break;
-    } else {
-      ++n;
-      if (take) take->push_back((int)i);
-    }
-  }
-  return n;
-}
-
-struct RegLay {
-  int r[3], l[3], w, slot;  // register, lane and wave digits, slot that orders the phases
-};
-
-struct RegPlan {
-  int ns = 0;
-  RegLay first, last;           // layouts of the first and the last stage
-  std::vector<uint32_t> words;  // RegStage records, then the members' kinds and one spare
-  std::vector<double> vals;     // kRegVals values a member, and one spare block
-};
-
-// Stages: the first one on a layout that loads HBM directly (register digits
-// among 3-6, lanes on digits 0-2: 64 consecutive coefficients per access),
-// each further one on the three digits that take the most pending items (at
-// least one: an item's digits and one kept from the stage before), and
-// a last, possibly empty one on a layout that stores directly.  With
-// `ordered` the operations keep their order (see reg_absorb).
-// `io`: a tile of a state; otherwise (a whole circuit) any layout may come
-// first and last.  m digits (6: no wave digit).
-inline void reg_plan(const std::vector<RegItem> &items, int m, bool io, bool ordered, RegPlan *out) {
-  uint32_t triples[35], nt = 0;
-  for (int a = 3; a < m; ++a)  // the 4 load / store layouts of 7 digits first
-    for (int b = a + 1; b < m; ++b)
-      for (int c = b + 1; c < m; ++c) triples[nt++] = (1u << a) | (1u << b) | (1u << c);
-  const uint32_t nio = nt;
-  for (int a = 0; a < 3; ++a)
-    for (int b = a + 1; b < m; ++b)
-      for (int c = b + 1; c < m; ++c) triples[nt++] = (1u << a) | (1u << b) | (1u << c);
-  std::vector<char> done(items.size(), 0);
-  // pending items inside each triple: no more than these can be taken, so a
-  // triple is looked at only if it may beat the best one so far
-  int inside[35] = {0};
-  for (const RegItem &it : items)
-    for (uint32_t t = 0; t < nt; ++t) inside[t] += (it.mask & ~triples[t]) == 0;
-  std::vector<uint32_t> stage;
-  std::vector<std::vector<int>> members;
-  size_t first = 0, left = items.size();
-  while (left || stage.empty()) {
-    uint32_t best = 0;
-    int most = -1;
-    for (uint32_t t = 0; t < (io && stage.empty() ? nio : nt); ++t) {
-      if (!stage.empty() && !(triples[t] & stage.back())) continue;  // a redistribution keeps one digit
-      // in order, the first pending item comes first
-      if (ordered && left && !(io && stage.empty()) && (items[first].mask & ~triples[t])) continue;
-      if (inside[t] <= most) continue;
-      const int n = reg_absorb(items, done, first, triples[t], ordered, nullptr);
-      if (n > most) {
-        most = n;
-        best = t;
-      }
-    }
-    std::vector<int> take;
-    reg_absorb(items, done, first, triples[best], ordered, &take);
-    for (int i : take) {
-      done[i] = 1;
-      for (uint32_t t = 0; t < nt; ++t) inside[t] -= (items[i].mask & ~triples[t]) == 0;
-    }
-    left -= take.size();
-    while (first < items.size() && done[first]) ++first;
-    stage.push_back(triples[best]);
-    members.push_back(std::move(take));
-  }
-  if (io && (stage.back() & 7u)) {  // an empty stage that stores directly
-    const uint32_t last = stage.back();
-    uint32_t best = nio;
-    for (uint32_t t = 0; t < nio; ++t)
-      if ((triples[t] & last) && (best == nio || __builtin_popcount(triples[t] & last) >
-                                                     __builtin_popcount(triples[best] & last)))
-        best = t;
-    if (best == nio) {  // digits 0-2 in registers: one stage in between
-      stage.push_back((1u << 2) | (1u << 3) | (1u << 4));
-      members.emplace_back();
-      best = 0;  // digits 3, 4, 5
-    }
-    stage.push_back(triples[best]);
-    members.emplace_back();
-  }
-  const int ns = (int)stage.size();
-  std::vector<RegLay> lay(ns);
-  for (int k = 0; k < ns; ++k) {
-    RegLay &y = lay[k];
-    int reg[3], nreg = 0, rest[4], nrest = 0;
-    for (int d = 0; d < m; ++d) {
-      if ((stage[k] >> d) & 1) reg[nreg++] = d;
-      else rest[nrest++] = d;
-    }
-    // register digits: those kept from the previous stage stay in their
-    // slots, the first such slot orders the phases
-    for (int j = 0; j < 3; ++j) y.r[j] = -1;
-    y.slot = 0;
-    if (k) {
-      y.slot = -1;
-      for (int j = 0; j < 3; ++j)
-        if ((stage[k] >> lay[k - 1].r[j]) & 1) {
-          y.r[j] = lay[k - 1].r[j];
-          y.slot = j;  // the last one
-        }
-    }
-    for (int x = 0; x < 3; ++x) {
-      bool held = false;
-      for (int j = 0; j < 3; ++j) held = held || y.r[j] == reg[x];
-      for (int j = 0; j < 3 && !held; ++j)
-        if (y.r[j] < 0) {
-          y.r[j] = reg[x];
-          held = true;
-        }
-    }
-    // lane digits: digits 0-2 at the lane index of the load / store layouts,
-    // digits that were lanes before at their index; the wave digit is the
-    // highest of the others
-    for (int j = 0; j < 3; ++j) y.l[j] = -1;
-    bool used[8] = {false};
-    for (int x = 0; x < nrest; ++x)
-      if (rest[x] < 3) {
-        y.l[rest[x]] = rest[x];
-        used[rest[x]] = true;
-      }
-    if (k)
-      for (int j = 0; j < 3; ++j) {
-        const int d = lay[k - 1].l[j];
-        if (d >= 3 && y.l[j] < 0 && !((stage[k] >> d) & 1)) {
-          y.l[j] = d;
-          used[d] = true;
-        }
-      }
-    int x = 0;
-    for (int j = 0; j < 3; ++j)
-      if (y.l[j] < 0) {
-        while (used[rest[x]]) ++x;
-        y.l[j] = rest[x];
-        used[rest[x]] = true;
-      }
-    y.w = m;  // (no wave digit)
-    for (int q = 0; q < nrest; ++q)
-      if (!used[rest[q]]) y.w = rest[q];
-  }
-  out->first = lay[0];
-  out->last = lay[ns - 1];
-  out->ns = ns;
-  out->words.clear();
-  out->vals.clear();
-  std::vector<uint32_t> kinds;
-  for (int k = 0; k < ns; ++k) {
-    RegStage sg;
-    memset(&sg, 0, sizeof(sg));
-    sg.mem = (uint32_t)kinds.size();
-    auto slot = [&](int d) { return lay[k].r[0] == d ? 0 : lay[k].r[1] == d ? 1 : 2; };
-    for (size_t x = 0; x < members[k].size(); ++x) {
-      const RegItem &it = items[members[k][x]];
-      double v[kRegVals] = {0.0};
-      uint32_t kind;
-      if (it.kind == 0) {
-        const int k1 = reg_1q_kind(it.v);
-        if (k1 < 0) continue;
-        kind = k1 + slot(it.d0);
-        int at = 0;
-        for (int r = 0; r < 3; ++r)
-          for (int c = 0; c < 4; ++c)
-            if (k1 == RM_A1 || (k1 == RM_U1 && c > 0) || (k1 == RM_D1 && c == r + 1)) v[at++] = it.v[4 * r + c];
-      } else {
-        const int s0 = slot(it.d0), s1 = slot(it.d1);
-        const int lo = std::min(s0, s1), hi = std::max(s0, s1);
-        const int pair = lo == 0 ? hi - 1 : 2;  // (0,1) (0,2) (1,2)
-        const RegItem *scale = nullptr;  // the scale of this CX, if it comes next
-        if (it.kind == 1 && x + 1 < members[k].size()) {
-          scale = &items[members[k][x + 1]];
-          if (scale->kind != 2 || scale->d0 != it.d0 || scale->d1 != it.d1) scale = nullptr;
-        }
-        if (scale) {
-          kind = RM_CXD + 2 * pair + (s0 > s1 ? 1 : 0);
-          memcpy(v, scale->v, 16 * sizeof(double));
-          ++x;
-        } else if (it.kind == 1) {
-          kind = RM_CX + 2 * pair + (s0 > s1 ? 1 : 0);
-        } else {
-          kind = RM_D2 + pair;
-          for (int a = 0; a < 4; ++a)
-            for (int b = 0; b < 4; ++b) v[4 * a + b] = it.v[s0 < s1 ? 4 * a + b : 4 * b + a];
-        }
-      }
-      kinds.push_back(kind);
-      out->vals.insert(out->vals.end(), v, v + kRegVals);
-    }
-    sg.nm = (uint32_t)kinds.size() - sg.mem;
-    if (k) {
-      // LDS offsets of the digits.  The banks are the lowest three base-4
-      // digits of the coefficient index: the writer's lane digits sit there,
-      // and a lane digit of the reader that is none of them is added (XOR)
-      // to the place of one that is no lane of the reader, so that the lanes of a wave fall on
-      // distinct banks on both sides.  Every digit but the writer's lanes
-      // and the phase digit also has a place of its own above them.
-      const RegLay &w = lay[k - 1], &y = lay[k];
-      uint32_t co[8] = {0};
-      for (int j = 0; j < 3; ++j) co[w.l[j]] = 1u << (2 * j);
-      int high = 3;
-      for (int d = 0; d < m; ++d)
-        if (!co[d] && d != y.r[y.slot]) co[d] = 1u << (2 * high++);
-      bool place[3];  // places of writer lanes that are no reader lanes
-      for (int j = 0; j < 3; ++j) place[j] = w.l[j] != y.l[0] && w.l[j] != y.l[1] && w.l[j] != y.l[2];
-      for (int j = 0; j < 3; ++j) {
-        if (y.l[j] == w.l[0] || y.l[j] == w.l[1] || y.l[j] == w.l[2]) continue;
-        int at = j;
-        while (!place[at]) at = (at + 1) % 3;
-        place[at] = false;
-        co[y.l[j]] |= 1u << (2 * at);
-      }
-      sg.slot = (uint32_t)y.slot;
-      for (int j = 0; j < 3; ++j) {
-        sg.wr[j] = co[w.r[j]];
-        sg.wl[j] = co[w.l[j]];
-        sg.rr[j] = co[y.r[j]];
-        sg.rl[j] = co[y.l[j]];
-      }
-      sg.ww = co[w.w];
-      sg.rw = co[y.w];
-    }
-    uint32_t w[sizeof(RegStage) / 4];
-    memcpy(w, &sg, sizeof(sg));
-    out->words.insert(out->words.end(), w, w + sizeof(RegStage) / 4);
-  }
-  // the spare member that the last one's prefetch reads
-  kinds.push_back(0);
-  out->words.insert(out->words.end(), kinds.begin(), kinds.end());
-  out->vals.resize(out->vals.size() + kRegVals, 0.0);
 }
 
 // HBM strides of a tile's load and store layouts.
