@@ -2892,20 +2892,11 @@ bool plan_reg(const dm_state *h, FusedPass *fp) {
 // expected to be as fast.  Kernels of 3-5 us below 12 qubits, the passes
 // 9-20; from 12 qubits on a pass takes 1.0-1.4 times the kernels' time.
 template <typename T>
-std::vector<FusedPass> fuse_plain_run(const dm_state *h, const PlainRun &run, const dm_op *ops, const double *params) {
+std::vector<FusedPass> fuse_plain_run(const dm_state *h, const PlainRun &run, const dm_op *ops) {
   std::vector<FusedPass> out;
   const int n = h->n;
-  if (run.ops.size() < 2 || n > 18) return out;
-  // kernels of the run one by one
-  double kernels = 0.0;
-  int last = -1;
-  for (int i : run.src) {
-    if (i == last) continue;
-    last = i;
-    const double *pv = params + ops[i].param;
-    const bool feed = ops[i].kind == DM_OP_MEMORY_NOISE && (1 - pv[2]) * (2 * pv[1] - 1) != 0.0;
-    kernels += ops[i].kind == DM_OP_FUSED ? 3 : !feed ? 1 : n >= 12 ? 1 + (n - 4) / 4 : 1 + (n - 4) / 3;
-  }
+  if (run.total < 2 || n > 18) return out;
+  const double kernels = run.kernels;
   // one launch for runs of six kernels or more (5 qubits, 80 gates in dense
   // blocks with short runs between them: 293 us one by one, 302 with every
   // run of two and more as one launch; 6 qubits, 80 gates in fused passes:
@@ -2935,7 +2926,7 @@ std::vector<FusedPass> fuse_plain_run(const dm_state *h, const PlainRun &run, co
   if (blocks.size() * (n < 12 ? 2.0 : 1.4) >= kernels) return out;
   for (const std::vector<int> &b : blocks) {
     FusedPass fp;
-    if (b.size() == 1 && ops[run.src[b[0]]].kind != DM_OP_MEMORY_NOISE) {
+    if (b.size() == 1 && run.count[b[0]] == 1 && ops[run.src[b[0]]].kind != DM_OP_MEMORY_NOISE) {
       fp.plain = run.src[b[0]];  // its own kernel
       out.push_back(std::move(fp));
       continue;
@@ -3064,13 +3055,9 @@ int parse_fused(const dm_state *h, const double *p, int64_t avail, int opi, Fuse
   if (run) {
     for (const TileOp &op : fp->ops)
       if (op.kind != TOP_1Q && op.kind != TOP_CX) return DM_OK;
-    const int32_t base = (int32_t)run->vals.size();
-    run->vals.insert(run->vals.end(), fp->vals.begin(), fp->vals.end());
     for (TileOp op : fp->ops) {
       for (int x = 0; x < (op.kind == TOP_CX ? 2 : 1); ++x) op.d[x] = fp->geo.tpos[op.d[x]];
-      op.param += base;
-      run->ops.push_back(op);
-      run->src.push_back(opi);
+      push_plain(op, fp->vals.data() + op.param, op.kind == TOP_1Q ? 12 : op.k ? 16 : 0, opi, run);
     }
     fp->ops.clear();
     return DM_OK;
@@ -3425,11 +3412,13 @@ int stage_program(dm_state *h, const dm_op *ops, int nops, const double *params,
         }
         if (h->n > 6 || ops[e].kind != DM_OP_FUSED) break;
         FusedPass fp;
+        const int before = run.total;
         if (int rc = fused_args(e)) return rc;
         if (int rc = parse_fused(h, params + ops[e].param, nparams - ops[e].param, e, &fp, false, &run)) return rc;
         if (!fp.ops.empty()) break;
+        if (run.total > before) run.kernels += 3;
       }
-      std::vector<FusedPass> fps = fuse_plain_run<T>(h, run, ops, params);
+      std::vector<FusedPass> fps = fuse_plain_run<T>(h, run, ops);
       dm_op synth;
       memset(&synth, 0, sizeof(synth));
       synth.kind = DM_OP_FUSED;

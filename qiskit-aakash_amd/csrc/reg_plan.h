@@ -116,6 +116,18 @@ inline std::vector<RegItem> reg_items_in_order(const std::vector<TileOp> &ops, c
   return out;
 }
 
+// The map v after e, both rows X, Y, Z of (I, X, Y, Z), into e.
+inline void compose_1q(const double *v, double *e) {
+  double w[12];
+  for (int i = 0; i < 3; ++i)
+    for (int j = 0; j < 4; ++j) {
+      double acc = j == 0 ? v[4 * i] : 0.0;
+      for (int k = 0; k < 3; ++k) acc += v[4 * i + 1 + k] * e[4 * k + j];
+      w[4 * i + j] = acc;
+    }
+  memcpy(e, w, sizeof(w));
+}
+
 // The pass's operations as register-stage items, free to be reordered where
 // they commute: runs of single-qubit maps on one digit become one map, and
 // the separable scale of a CX (a depolarising channel on each of its qubits)
@@ -141,15 +153,7 @@ inline std::vector<RegItem> reg_items(const std::vector<TileOp> &ops, const std:
         pend[d] = (int)out.size();
         out.push_back(it);
       } else {
-        // (I, X, Y, Z) -> rows of the later map applied to the earlier one
-        double *e = out[pend[d]].v, w[12];
-        for (int i = 0; i < 3; ++i)
-          for (int j = 0; j < 4; ++j) {
-            double acc = j == 0 ? v[4 * i] : 0.0;
-            for (int k = 0; k < 3; ++k) acc += v[4 * i + 1 + k] * e[4 * k + j];
-            w[4 * i + j] = acc;
-          }
-        memcpy(e, w, sizeof(w));
+        compose_1q(v, out[pend[d]].v);
       }
     } else {
       RegItem it;
@@ -215,30 +219,99 @@ inline std::vector<RegItem> reg_items(const std::vector<TileOp> &ops, const std:
   return res;
 }
 
-// Items (of those with done[i] == 0) that a stage on the digits of `triple`
-// takes: an item joins unless it, or an earlier one left out that it does
-// not commute with, reaches outside the triple.  Items on different digits
-// commute; with `ordered` (results bit for bit those of the given order)
-// only if one of them rounds nothing.
-inline int reg_absorb(const std::vector<RegItem> &items, const std::vector<char> &done, size_t first, uint32_t triple,
-                      bool ordered, std::vector<int> *take) {
-  uint32_t blocked = 0;
-  bool rounded = false;  // an item that rounds was left out
-  int n = 0;
-  for (size_t i = first; i < items.size(); ++i) {
-    if (done[i]) continue;
-    const uint32_t m = items[i].mask;
-    if ((m & blocked) || (m & ~triple) || (ordered && rounded && !items[i].exact)) {
-      blocked |= m;
-      rounded = rounded || !items[i].exact;
-      if (!(triple & ~blocked)) break;
-    } else {
+// The pending items of a pass or run: each digit has the list of the items
+// that touch it, in program order, and so have the items that round
+// something.  A stage's items are found by walking the lists of its digits,
+// so that planning takes time in proportion to the items taken and not to
+// those still pending.
+class RegQueue {
+ public:
+  static constexpr int kEnd = INT32_MAX;
+
+  explicit RegQueue(const std::vector<RegItem> &items) : items_(items), link_(3 * items.size()) {
+    for (int &h : head_) h = kEnd;
+    for (size_t i = items.size(); i-- > 0;)
+      for (int s = 0; s < 3; ++s) {
+        const int l = list(items[i], s);
+        if (l < 0) continue;
+        link_[3 * i + s] = {head_[l], kEnd};
+        if (head_[l] != kEnd) back(head_[l], l) = (int)i;
+        head_[l] = (int)i;
+      }
+    for (const RegItem &it : items) ++count_[it.mask];
+  }
+
+  // Pending items inside the triple of digits d.
+  int inside(const int (&d)[3]) const {
+    int n = 0;
+    for (int a = 0; a < 3; ++a) n += count_[1u << d[a]] + count_[(1u << d[a]) | (1u << d[(a + 1) % 3])];
+    return n;
+  }
+
+  // The digits of the first pending item.
+  uint32_t first_mask() const {
+    int i = kEnd;
+    for (int d = 0; d < kRounding; ++d) i = std::min(i, head_[d]);
+    return i == kEnd ? 0u : items_[i].mask;
+  }
+
+  // Items that a stage on the digits d takes: an item joins unless it, or an
+  // earlier one left out that it does not commute with, reaches outside the
+  // triple.  Items on different digits commute; with `ordered` (results bit
+  // for bit those of the given order) only if one of them rounds nothing: an
+  // item that rounds joins only as the first pending one of those.
+  int absorb(const int (&d)[3], bool ordered, std::vector<int> *take) const {
+    uint32_t blocked = 0;
+    const uint32_t triple = (1u << d[0]) | (1u << d[1]) | (1u << d[2]);
+    int at[3] = {head_[d[0]], head_[d[1]], head_[d[2]]}, rounding = head_[kRounding], n = 0;
+    for (;;) {
+      const int i = std::min(at[0], std::min(at[1], at[2]));
+      if (i == kEnd) return n;
+      const RegItem &it = items_[i];
+      if ((it.mask & blocked) || (it.mask & ~triple) || (ordered && !it.exact && i != rounding)) {
+        blocked |= it.mask;
+        for (int s = 0; s < 3; ++s)
+          if ((it.mask >> d[s]) & 1) at[s] = kEnd;
+        continue;
+      }
       ++n;
-      if (take) take->push_back((int)i);
+      if (take) take->push_back(i);
+      if (ordered && !it.exact) rounding = link_[3 * (size_t)i + 2].next;
+      for (int s = 0; s < 3; ++s)
+        if (at[s] == i) at[s] = link_[3 * (size_t)i + (it.d0 == d[s] ? 0 : 1)].next;
     }
   }
-  return n;
-}
+
+  void remove(int i) {
+    --count_[items_[i].mask];
+    for (int s = 0; s < 3; ++s) {
+      const int l = list(items_[i], s);
+      if (l < 0) continue;
+      const Link k = link_[3 * (size_t)i + s];
+      if (k.prev == kEnd) head_[l] = k.next;
+      else next(k.prev, l) = k.next;
+      if (k.next != kEnd) back(k.next, l) = k.prev;
+    }
+  }
+
+ private:
+  static constexpr int kRounding = 8;  // the list of the items that round
+  struct Link {
+    int next, prev;
+  };
+  // list of an item's link: its first digit's, its second digit's, the rounding items'; -1: none
+  static int list(const RegItem &it, int s) {
+    return s == 0 ? it.d0 : s == 1 ? (it.d1 != it.d0 ? it.d1 : -1) : it.exact ? -1 : kRounding;
+  }
+  size_t slot(int i, int l) const { return 3 * (size_t)i + (l == kRounding ? 2 : items_[i].d0 == l ? 0 : 1); }
+  int &next(int i, int l) { return link_[slot(i, l)].next; }
+  int &back(int i, int l) { return link_[slot(i, l)].prev; }
+
+  const std::vector<RegItem> &items_;
+  std::vector<Link> link_;
+  int head_[9];
+  int count_[256] = {0};  // pending items by digits
+};
 
 struct RegLay {
   int r[3], l[3], w, slot;  // register, lane and wave digits, slot that orders the phases
@@ -256,49 +329,49 @@ struct RegPlan {
 // each further one on the three digits that take the most pending items (at
 // least one: an item's digits and one kept from the stage before), and
 // a last, possibly empty one on a layout that stores directly.  With
-// `ordered` the operations keep their order (see reg_absorb).
+// `ordered` the operations keep their order (see RegQueue::absorb).
 // `io`: a tile of a state; otherwise (a whole circuit) any layout may come
 // first and last.  m digits (6: no wave digit).
 inline void reg_plan(const std::vector<RegItem> &items, int m, bool io, bool ordered, RegPlan *out) {
+  int digits[35][3];
   uint32_t triples[35], nt = 0;
+  auto add = [&](int a, int b, int c) {
+    digits[nt][0] = a;
+    digits[nt][1] = b;
+    digits[nt][2] = c;
+    triples[nt++] = (1u << a) | (1u << b) | (1u << c);
+  };
   for (int a = 3; a < m; ++a)  // the 4 load / store layouts of 7 digits first
     for (int b = a + 1; b < m; ++b)
-      for (int c = b + 1; c < m; ++c) triples[nt++] = (1u << a) | (1u << b) | (1u << c);
+      for (int c = b + 1; c < m; ++c) add(a, b, c);
   const uint32_t nio = nt;
   for (int a = 0; a < 3; ++a)
     for (int b = a + 1; b < m; ++b)
-      for (int c = b + 1; c < m; ++c) triples[nt++] = (1u << a) | (1u << b) | (1u << c);
-  std::vector<char> done(items.size(), 0);
-  // pending items inside each triple: no more than these can be taken, so a
-  // triple is looked at only if it may beat the best one so far
-  int inside[35] = {0};
-  for (const RegItem &it : items)
-    for (uint32_t t = 0; t < nt; ++t) inside[t] += (it.mask & ~triples[t]) == 0;
+      for (int c = b + 1; c < m; ++c) add(a, b, c);
+  RegQueue queue(items);
   std::vector<uint32_t> stage;
   std::vector<std::vector<int>> members;
-  size_t first = 0, left = items.size();
+  size_t left = items.size();
   while (left || stage.empty()) {
+    const bool load = io && stage.empty();
+    const uint32_t first = ordered && !load ? queue.first_mask() : 0u;
     uint32_t best = 0;
     int most = -1;
-    for (uint32_t t = 0; t < (io && stage.empty() ? nio : nt); ++t) {
+    for (uint32_t t = 0; t < (load ? nio : nt); ++t) {
       if (!stage.empty() && !(triples[t] & stage.back())) continue;  // a redistribution keeps one digit
-      // in order, the first pending item comes first
-      if (ordered && left && !(io && stage.empty()) && (items[first].mask & ~triples[t])) continue;
-      if (inside[t] <= most) continue;
-      const int n = reg_absorb(items, done, first, triples[t], ordered, nullptr);
+      if (first & ~triples[t]) continue;                   // in order, the first pending item comes first
+      if (queue.inside(digits[t]) <= most) continue;       // no more than these can be taken
+      const int n = queue.absorb(digits[t], ordered, nullptr);
       if (n > most) {
         most = n;
         best = t;
       }
     }
     std::vector<int> take;
-    reg_absorb(items, done, first, triples[best], ordered, &take);
-    for (int i : take) {
-      done[i] = 1;
-      for (uint32_t t = 0; t < nt; ++t) inside[t] -= (items[i].mask & ~triples[t]) == 0;
-    }
+    take.reserve(most);
+    queue.absorb(digits[best], ordered, &take);
+    for (int i : take) queue.remove(i);
     left -= take.size();
-    while (first < items.size() && done[first]) ++first;
     stage.push_back(triples[best]);
     members.push_back(std::move(take));
   }
@@ -470,11 +543,41 @@ inline void reg_plan(const std::vector<RegItem> &items, int m, bool io, bool ord
 // FP64 state as fused passes (an FP32 state keeps one kernel per operation:
 // its kernels round differently).  Up to 6 qubits, where one kernel takes the
 // whole run, the program's own fused passes join it.
+// Single-qubit maps of a position with no CX between them are one map.
 struct PlainRun {
   std::vector<TileOp> ops;      // digits are positions
   std::vector<double> vals;
-  std::vector<int> src;         // program operation of each
+  std::vector<int> src;         // program operation of each (the first one)
+  std::vector<int> count;       // operations in each (memory noise: one a position)
+  int pend[32];                 // the map that a position's next one joins, or -1
+  int total = 0;                // sum of count
+  double kernels = 0.0;         // the kernels that run the operations one by one
+
+  PlainRun() {
+    for (int &p : pend) p = -1;
+  }
 };
+
+// One operation (digits are positions) with its nv values; program operation src.
+inline void push_plain(TileOp t, const double *v, int nv, int src, PlainRun *run) {
+  ++run->total;
+  if (t.kind == TOP_1Q) {
+    int &p = run->pend[t.d[0]];
+    if (p >= 0) {
+      compose_1q(v, &run->vals[run->ops[p].param]);
+      ++run->count[p];
+      return;
+    }
+    p = (int)run->ops.size();
+  } else {
+    run->pend[t.d[0]] = run->pend[t.d[1]] = -1;
+  }
+  t.param = (int32_t)run->vals.size();
+  run->vals.insert(run->vals.end(), v, v + nv);
+  run->ops.push_back(t);
+  run->src.push_back(src);
+  run->count.push_back(1);
+}
 
 inline bool plain_op(const dm_op &op) {
   return op.kind == DM_OP_1Q || op.kind == DM_OP_CX || op.kind == DM_OP_CX_SCALED || op.kind == DM_OP_MEMORY_NOISE;
@@ -483,37 +586,34 @@ inline bool plain_op(const dm_op &op) {
 inline void add_plain(int n, const dm_op &op, const double *params, int src, PlainRun *run) {
   TileOp t;
   memset(&t, 0, sizeof(t));
-  t.param = (int32_t)run->vals.size();
-  auto put = [&](const double *v, int nv) { run->vals.insert(run->vals.end(), v, v + nv); };
   const double *pv = params + op.param;
   if (op.kind == DM_OP_MEMORY_NOISE) {
     const double f = pv[0], p = pv[1], g = pv[2];
     if (f == 1.0 && g == 1.0) return;
     const double od = sqrt(g) * f, dd = (1 - g) * (2 * p - 1);
     const double R[12] = {0, od, 0, 0, 0, 0, od, 0, dd, 0, 0, g};
-    put(R, 12);
     t.kind = TOP_1Q;
     t.k = 1;
     for (int d = 0; d < n; ++d) {
       t.d[0] = d;
-      run->ops.push_back(t);
-      run->src.push_back(src);
+      push_plain(t, R, 12, src, run);
     }
+    // a diagonal kernel, or with a thermal feed tile passes
+    run->kernels += dd == 0.0 ? 1 : n >= 12 ? 1 + (n - 4) / 4 : 1 + (n - 4) / 3;
     return;
   }
+  run->kernels += 1;
   t.d[0] = n - 1 - op.qubits[0];
   if (op.kind == DM_OP_1Q) {
     t.kind = TOP_1Q;
     t.k = 1;
-    put(pv, 12);
+    push_plain(t, pv, 12, src, run);
   } else {
     t.kind = TOP_CX;
     t.d[1] = n - 1 - op.qubits[1];
     t.k = op.kind == DM_OP_CX_SCALED ? 1 : 0;
-    if (t.k) put(pv, 16);
+    push_plain(t, pv, t.k ? 16 : 0, src, run);
   }
-  run->ops.push_back(t);
-  run->src.push_back(src);
 }
 
 // Blocks of the run: the operations that the tile of the positions 0-2 and
@@ -521,41 +621,72 @@ inline void add_plain(int n, const dm_op &op, const double *params, int src, Pla
 // left out that shares a position with it, reaches outside), the others
 // chosen by growth from the first pending operation, with and without one
 // position forced in, whichever takes the most operations.
+// Each position has the list of its pending operations, and a block is found
+// by walking the lists of the positions still open to it: the time goes with
+// the operations taken and not with those left pending.
 inline std::vector<std::vector<int>> plain_blocks(int n, const PlainRun &run) {
+  constexpr int kEnd = INT32_MAX;
+  struct Link {
+    int next, prev;
+  };
   const int no = (int)run.ops.size();
   std::vector<uint32_t> mask(no);
-  for (int i = 0; i < no; ++i) {
-    mask[i] = 1u << run.ops[i].d[0];
-    if (run.ops[i].kind == TOP_CX) mask[i] |= 1u << run.ops[i].d[1];
-  }
+  std::vector<Link> link(2 * (size_t)no);
+  int head[32];
+  for (int &h : head) h = kEnd;
+  auto at = [&](int i, int p) -> Link & { return link[2 * (size_t)i + (run.ops[i].d[0] == p ? 0 : 1)]; };
+  for (int i = no - 1; i >= 0; --i)
+    for (int x = 0; x < (run.ops[i].kind == TOP_CX ? 2 : 1); ++x) {
+      const int p = run.ops[i].d[x];
+      mask[i] |= 1u << p;
+      at(i, p) = {head[p], kEnd};
+      if (head[p] != kEnd) at(head[p], p).prev = i;
+      head[p] = i;
+    }
   const uint32_t low = 7u, full = (1u << n) - 1u;
   const int most_high = std::min(4, n - 3);
-  std::vector<char> done(no, 0);
   std::vector<std::vector<int>> out;
-  int first = 0, left = no;
   std::vector<int> cur, best;
-  while (left) {
-    while (done[first]) ++first;
+  for (int left = no; left;) {
     best.clear();
+    int most = 0;
     for (int force = -1; force < n; ++force) {
       if (force >= 0 && force < 3) continue;
       uint32_t T = force < 0 ? 0 : 1u << force, blocked = 0;
+      int walk[32], ops = 0;
+      memcpy(walk, head, sizeof(walk));
       cur.clear();
-      for (int i = first; i < no; ++i) {
-        if (done[i]) continue;
+      for (;;) {
+        const uint32_t open = (__builtin_popcount(T) < most_high ? full : T | low) & ~blocked;
+        int i = kEnd;
+        for (uint32_t s = open; s; s &= s - 1) i = std::min(i, walk[__builtin_ctz(s)]);
+        if (i == kEnd) break;
         const uint32_t m = mask[i], t2 = T | (m & ~low);
         if ((m & blocked) || __builtin_popcount(t2) > most_high) {
           blocked |= m;
-          const uint32_t open = __builtin_popcount(T) < most_high ? full : T | low;
-          if (!(open & ~blocked)) break;
-        } else {
-          T = t2;
-          cur.push_back(i);
+          continue;
+        }
+        T = t2;
+        cur.push_back(i);
+        ops += run.count[i];
+        for (uint32_t s = m; s; s &= s - 1) {
+          const int p = __builtin_ctz(s);
+          walk[p] = at(i, p).next;
         }
       }
-      if (cur.size() > best.size()) best = cur;
+      if (ops > most) {
+        most = ops;
+        best.swap(cur);
+      }
     }
-    for (int i : best) done[i] = 1;
+    for (int i : best)
+      for (uint32_t s = mask[i]; s; s &= s - 1) {
+        const int p = __builtin_ctz(s);
+        const Link k = at(i, p);
+        if (k.prev == kEnd) head[p] = k.next;
+        else at(k.prev, p).next = k.next;
+        if (k.next != kEnd) at(k.next, p).prev = k.prev;
+      }
     left -= (int)best.size();
     out.push_back(best);
   }
