@@ -1997,6 +1997,13 @@ struct ProfPending {
   int fam;
 };
 
+// A program image from pinned host memory (see enqueue_image).
+__global__ __launch_bounds__(kBlock) void k_image(uint4 *__restrict__ dst, const uint4 *__restrict__ src,
+                                                  uint32_t packs) {
+  const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+  if (i < packs) dst[i] = src[i];
+}
+
 // A fused pass parsed from its parameter record (see DM_OP_FUSED in dmsim.h).
 struct FusedPass {
   int m = 0;
@@ -2035,9 +2042,13 @@ struct dm_state {
   size_t red_cap = 0;           // doubles
   void *d_mat = nullptr;        // program image: tile-operation records, block matrices (storage dtype)
   size_t mat_cap = 0;           // bytes
-  void *h_img = nullptr;        // pinned copy of the image on its way to d_mat
+  // the image on its way to d_mat: small ones and the first larger ones in
+  // pageable memory, then in pinned memory
+  std::vector<char> page_img;
+  void *h_img = nullptr;
   size_t img_cap = 0;           // bytes
-  hipEvent_t img_ev = nullptr;  // that copy's end
+  int large_images = 0;         // larger ones without the pinned buffer
+  hipEvent_t img_ev = nullptr;  // that upload's end
   bool img_busy = false;
   double *d_aux = nullptr;      // gathered vectors / overlap operand
   size_t aux_cap = 0;           // bytes
@@ -3494,16 +3505,38 @@ int upload_image(dm_state *h, Prepared *pp, void *dev) {
   return DM_OK;
 }
 
-// The same into the handle's own buffer, in stream order through a pinned
-// copy: nothing waits for the device unless the previous image is still on
-// its way.
+// The same into the handle's own buffer, in stream order from a host copy that
+// the handle keeps until the upload has ended: nothing waits for the device
+// unless the previous image is still on its way.  Passes walk their records
+// one after another, so what counts is where the image lies afterwards: a
+// kernel's copy is in the caches, a copy engine's is not (a dependent walk:
+// 126-199 ns a 64-byte line against 372; a pass of 300 operations on 6 qubits,
+// FP32, 162 us against 197).
+// - Up to kSmallImage the runtime copies with a kernel, also from pageable
+//   memory (2.7-8 us a call; pinning a buffer costs 17-110 us with its first
+//   touch, and as much again when it is freed).
+// - Larger ones up to kKernelImage go in pieces of that size while a handle
+//   has had only a few of them (8 us a piece), as pinning would cost a program
+//   that runs once more than it saves; then k_image copies them from a pinned
+//   buffer (64 KB: 13.5 us against the engine's 10.5; 1 MB: 37 against 28).
+// - Above, the engine; the first few wait for the stream.
+constexpr size_t kSmallImage = 16 << 10, kKernelImage = 256 << 10;
+constexpr int kUnpinnedImages = 3;
+
 int enqueue_image(dm_state *h, Prepared *pp) {
   const size_t bytes = pp->image_bytes();
+  bool pinned = bytes > kSmallImage;
+  if (pinned && h->large_images < kUnpinnedImages) {
+    ++h->large_images;
+    if (bytes > kKernelImage) return upload_image(h, pp, h->d_mat);
+    pinned = false;
+  }
   if (h->img_busy) {
     HIP_TRY(hipEventSynchronize(h->img_ev));
     h->img_busy = false;
   }
-  if (h->img_cap < bytes) {
+  if (!h->img_ev) HIP_TRY(hipEventCreateWithFlags(&h->img_ev, hipEventDisableTiming));
+  if (pinned && h->img_cap < bytes) {
     if (h->h_img) hipHostFree(h->h_img);
     h->h_img = nullptr;
     h->img_cap = 0;
@@ -3515,11 +3548,21 @@ int enqueue_image(dm_state *h, Prepared *pp) {
     }
     h->img_cap = cap;
   }
-  if (!h->img_ev) HIP_TRY(hipEventCreateWithFlags(&h->img_ev, hipEventDisableTiming));
-  char *img = static_cast<char *>(h->h_img);
+  if (!pinned && h->page_img.size() < bytes) h->page_img.resize(bytes);
+  char *img = pinned ? static_cast<char *>(h->h_img) : h->page_img.data();
   if (!pp->tops.empty()) memcpy(img, pp->tops.data(), pp->tops.size() * 4);
   if (!pp->values.empty()) memcpy(img + pp->vals_at, pp->values.data(), pp->values.size());
-  HIP_TRY(hipMemcpyAsync(h->d_mat, img, bytes, hipMemcpyHostToDevice, h->stream));
+  if (pinned && bytes <= kKernelImage) {
+    const size_t packs = (bytes + 15) / 16;  // (both buffers hold a multiple of 16)
+    hipLaunchKernelGGL(k_image, dim3((unsigned)((packs + kBlock - 1) / kBlock)), dim3(kBlock), 0, h->stream,
+                       static_cast<uint4 *>(h->d_mat), reinterpret_cast<const uint4 *>(img), (uint32_t)packs);
+    if (int rc = last_launch("k_image")) return rc;
+  } else {
+    const size_t piece = pinned ? bytes : kSmallImage;
+    for (size_t at = 0; at < bytes; at += piece)
+      HIP_TRY(hipMemcpyAsync(static_cast<char *>(h->d_mat) + at, img + at, std::min(piece, bytes - at),
+                             hipMemcpyHostToDevice, h->stream));
+  }
   HIP_TRY(hipEventRecord(h->img_ev, h->stream));
   h->img_busy = true;
   pp->d_ops = h->d_mat;
@@ -3532,8 +3575,9 @@ template <typename T>
 int prepare_program(dm_state *h, const dm_op *ops, int nops, const double *params, int64_t nparams, Prepared *pp) {
   if (int rc = stage_program<T>(h, ops, nops, params, nparams, pp)) return rc;
   if (pp->tops.empty() && pp->values.empty()) return DM_OK;
-  if (h->mat_cap < pp->image_bytes()) HIP_TRY(hipStreamSynchronize(h->stream));  // the old buffer may be in use
-  if (int rc = ensure(&h->d_mat, &h->mat_cap, pp->image_bytes())) return rc;
+  const size_t bytes = (pp->image_bytes() + 15) & ~(size_t)15;  // (k_image copies 16 at a time)
+  if (h->mat_cap < bytes) HIP_TRY(hipStreamSynchronize(h->stream));  // the old buffer may be in use
+  if (int rc = ensure(&h->d_mat, &h->mat_cap, bytes)) return rc;
   return enqueue_image(h, pp);
 }
 

@@ -327,3 +327,38 @@ def test_fp64_fused_passes_join_the_run_of_a_small_register(n, m, dense):
     st.close()
     assert got[0] == 2.0 ** -n
     assert np.abs(got - want).max() <= members * 8 * EPS['fp64'] * top
+
+
+@pytest.mark.parametrize('precision', ['fp64', 'fp32'])
+def test_program_images_of_every_size_and_in_turn(precision):
+    """Images of a few hundred bytes to above 256 KiB, one program after the
+    other on one handle without a wait between them, often enough for the
+    uploads from pageable and from pinned memory, against the same programs
+    each on a handle of its own: the same bit for bit."""
+    n = 7
+    rng = np.random.default_rng(8)
+    progs = []
+    for passes in (1, 4, 40, 700, 3, 41):  # about 0.4 KB a pass and more
+        prog = Program(n)
+        for _ in range(passes):
+            c, t = (int(x) for x in rng.choice(n, 2, replace=False))
+            prog.fused(7, [c, t], [(native.SUB_1Q, [c], ptm.rows3(random_map(rng, 'general'))),
+                                   (native.SUB_CX, [c, t], random_scale(rng, 'general')),
+                                   (native.SUB_1Q, [t], ptm.rows3(random_map(rng, 'unital')))])
+        progs.append(prog)
+    a = rng.normal(size=4 ** n) * 2.0 ** -n
+    kept = native.DeviceState(n, precision)
+    kept.upload(a)
+    for _ in range(6):
+        for prog in progs:
+            prog.run(kept)
+    got = kept.download()
+    kept.close()
+    for _ in range(6):
+        for prog in progs:
+            st = native.DeviceState(n, precision)
+            st.upload(a)
+            prog.run(st)
+            a = st.download()
+            st.close()
+    assert np.array_equal(got, a)
