@@ -2900,19 +2900,13 @@ bool plan_reg(const dm_state *h, FusedPass *fp) {
 }
 
 // The passes that replace the run, or none if one kernel per operation is
-// expected to be as fast.  Kernels of 3-5 us below 12 qubits, the passes
-// 9-20; from 12 qubits on a pass takes 1.0-1.4 times the kernels' time.
+// expected to be as fast (plain_pass_cost).
 template <typename T>
 std::vector<FusedPass> fuse_plain_run(const dm_state *h, const PlainRun &run, const dm_op *ops) {
   std::vector<FusedPass> out;
   const int n = h->n;
-  if (run.total < 2 || n > 18) return out;
-  const double kernels = run.kernels;
-  // one launch for runs of six kernels or more (5 qubits, 80 gates in dense
-  // blocks with short runs between them: 293 us one by one, 302 with every
-  // run of two and more as one launch; 6 qubits, 80 gates in fused passes:
-  // 176 us one by one, 90 as one launch)
-  if (n <= 6 && kernels < 6) return out;
+  if (run.total < 2) return out;
+  if (plain_pass_cost(n, 1) >= run.kernels) return out;
   if (n <= 6) {
     RegPlan rp;
     reg_plan(reg_items(run.ops, run.vals, 6), 6, false, false, &rp);
@@ -2934,7 +2928,7 @@ std::vector<FusedPass> fuse_plain_run(const dm_state *h, const PlainRun &run, co
     return out;
   }
   const std::vector<std::vector<int>> blocks = plain_blocks(n, run);
-  if (blocks.size() * (n < 12 ? 2.0 : 1.4) >= kernels) return out;
+  if (plain_pass_cost(n, blocks.size()) >= run.kernels) return out;
   for (const std::vector<int> &b : blocks) {
     FusedPass fp;
     if (b.size() == 1 && run.count[b[0]] == 1 && ops[run.src[b[0]]].kind != DM_OP_MEMORY_NOISE) {
@@ -3375,7 +3369,7 @@ int launch_memory_noise_tiles(dm_state *h, double f, double p, double g) {
 // values starting at a 256-byte boundary.
 struct Prepared {
   std::vector<dm_op> ops;
-  std::vector<double> params;
+  const double *params = nullptr;      // the caller's (a Prepared lives for one call)
   std::vector<FusedPass> fused;
   std::vector<int> fused_of;
   std::vector<size_t> offs, top_off;
@@ -3395,7 +3389,7 @@ struct Prepared {
 template <typename T>
 int stage_program(dm_state *h, const dm_op *ops, int nops, const double *params, int64_t nparams, Prepared *pp,
                   bool in_registers = true) {
-  pp->params.assign(params, params + (nparams > 0 ? nparams : 0));
+  pp->params = nparams > 0 ? params : nullptr;
   pp->ops.clear();
   pp->fused.clear();
   pp->fused_of.clear();
@@ -3408,12 +3402,25 @@ int stage_program(dm_state *h, const dm_op *ops, int nops, const double *params,
     pp->fused_of.push_back((int)pp->fused.size());
     pp->fused.push_back(std::move(fp));
   };
+  const bool runs = sizeof(T) == 8 && in_registers && h->n <= 18;
   int one_by_one = 0;  // operations before this one have been found not to gain as a run
+  int counted = 0;     // operations before this one have been counted
   for (int i = 0; i < nops; ++i) {
     auto fused_args = [&](int j) {
       return ops[j].param < 0 || ops[j].param >= nparams ? fail(DM_ERR_ARG, "op %d: bad parameter offset", j) : DM_OK;
     };
-    if (sizeof(T) == 8 && in_registers && i >= one_by_one) {
+    if (runs && i >= counted) {
+      // operations that may form runs; too few of them are not even collected
+      double most = 0.0;
+      uint32_t used = 0;
+      for (counted = i; counted < nops && (plain_op(ops[counted]) || (h->n <= 6 && ops[counted].kind == DM_OP_FUSED));
+           ++counted) {
+        most += plain_kernels(h->n, ops[counted], params);
+        used |= plain_positions(h->n, ops[counted]);
+      }
+      if (plain_pass_cost(h->n, least_blocks(used)) >= most) one_by_one = counted;
+    }
+    if (runs && i >= one_by_one) {
       PlainRun run;
       int e = i;
       for (; e < nops; ++e) {
@@ -3427,7 +3434,7 @@ int stage_program(dm_state *h, const dm_op *ops, int nops, const double *params,
         if (int rc = fused_args(e)) return rc;
         if (int rc = parse_fused(h, params + ops[e].param, nparams - ops[e].param, e, &fp, false, &run)) return rc;
         if (!fp.ops.empty()) break;
-        if (run.total > before) run.kernels += 3;
+        if (run.total > before) run.kernels += plain_kernels(h->n, ops[e], params);
       }
       std::vector<FusedPass> fps = fuse_plain_run<T>(h, run, ops);
       dm_op synth;
@@ -3467,11 +3474,12 @@ int stage_program(dm_state *h, const dm_op *ops, int nops, const double *params,
   // has parameter values (noiseless CX only): the kernels read them from
   // the records.
   pp->tops.clear();
-  std::vector<T> staging(pool);
+  pp->values.resize(pool * sizeof(T));
+  T *staging = reinterpret_cast<T *>(pp->values.data());
   size_t off = 0;
   for (int i = 0; i < nops; ++i) {
     if (ops[i].kind == DM_OP_BLOCK) {
-      prep_block_matrix<T>(h->n, ops[i].qubits, ops[i].k, params + ops[i].param, staging.data() + off,
+      prep_block_matrix<T>(h->n, ops[i].qubits, ops[i].k, params + ops[i].param, staging + off,
                            &pp->pos[4 * (size_t)i]);
       pp->offs[i] = off;
       off += (size_t)1 << (4 * ops[i].k);
@@ -3484,8 +3492,6 @@ int stage_program(dm_state *h, const dm_op *ops, int nops, const double *params,
     }
   }
   pp->vals_at = (pp->tops.size() * 4 + 255) & ~(size_t)255;
-  pp->values.resize(staging.size() * sizeof(T));
-  if (!staging.empty()) memcpy(pp->values.data(), staging.data(), pp->values.size());
   return DM_OK;
 }
 
@@ -3584,10 +3590,9 @@ int prepare_program(dm_state *h, const dm_op *ops, int nops, const double *param
 template <typename T>
 int launch_program(dm_state *h, const Prepared &pp) {
   const T *dmat = static_cast<const T *>(pp.d_mat);
-  const double *params = pp.params.data();
   for (size_t i = 0; i < pp.ops.size(); ++i) {
     const dm_op &op = pp.ops[i];
-    const double *pv = pp.params.empty() ? nullptr : params + op.param;
+    const double *pv = pp.params ? pp.params + op.param : nullptr;
     int rc = DM_OK;
     switch (op.kind) {
       case DM_OP_1Q: rc = launch_1q<T>(h, op.qubits[0], pv); break;

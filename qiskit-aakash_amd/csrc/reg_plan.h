@@ -228,17 +228,25 @@ class RegQueue {
  public:
   static constexpr int kEnd = INT32_MAX;
 
-  explicit RegQueue(const std::vector<RegItem> &items) : items_(items), link_(3 * items.size()) {
+  explicit RegQueue(const std::vector<RegItem> &items) : node_(items.size()) {
     for (int &h : head_) h = kEnd;
-    for (size_t i = items.size(); i-- > 0;)
+    for (size_t i = items.size(); i-- > 0;) {
+      const RegItem &it = items[i];
+      Node &e = node_[i];
+      e.mask = it.mask;
+      e.list[0] = (int8_t)it.d0;
+      e.list[1] = (int8_t)(it.d1 != it.d0 ? it.d1 : -1);
+      e.list[2] = (int8_t)(it.exact ? -1 : kRounding);
+      ++count_[it.mask];
       for (int s = 0; s < 3; ++s) {
-        const int l = list(items[i], s);
+        const int l = e.list[s];
         if (l < 0) continue;
-        link_[3 * i + s] = {head_[l], kEnd};
-        if (head_[l] != kEnd) back(head_[l], l) = (int)i;
+        e.next[s] = head_[l];
+        e.prev[s] = kEnd;
+        if (head_[l] != kEnd) node_[head_[l]].prev[slot(head_[l], l)] = (int)i;
         head_[l] = (int)i;
       }
-    for (const RegItem &it : items) ++count_[it.mask];
+    }
   }
 
   // Pending items inside the triple of digits d.
@@ -252,7 +260,7 @@ class RegQueue {
   uint32_t first_mask() const {
     int i = kEnd;
     for (int d = 0; d < kRounding; ++d) i = std::min(i, head_[d]);
-    return i == kEnd ? 0u : items_[i].mask;
+    return i == kEnd ? 0u : node_[i].mask;
   }
 
   // Items that a stage on the digits d takes: an item joins unless it, or an
@@ -267,48 +275,46 @@ class RegQueue {
     for (;;) {
       const int i = std::min(at[0], std::min(at[1], at[2]));
       if (i == kEnd) return n;
-      const RegItem &it = items_[i];
-      if ((it.mask & blocked) || (it.mask & ~triple) || (ordered && !it.exact && i != rounding)) {
-        blocked |= it.mask;
+      const Node &e = node_[i];
+      const bool rounds = e.list[2] >= 0;
+      if ((e.mask & (blocked | ~triple)) || (ordered && rounds && i != rounding)) {
+        blocked |= e.mask;
         for (int s = 0; s < 3; ++s)
-          if ((it.mask >> d[s]) & 1) at[s] = kEnd;
+          if ((e.mask >> d[s]) & 1) at[s] = kEnd;
         continue;
       }
       ++n;
       if (take) take->push_back(i);
-      if (ordered && !it.exact) rounding = link_[3 * (size_t)i + 2].next;
+      if (ordered && rounds) rounding = e.next[2];
       for (int s = 0; s < 3; ++s)
-        if (at[s] == i) at[s] = link_[3 * (size_t)i + (it.d0 == d[s] ? 0 : 1)].next;
+        if (at[s] == i) at[s] = e.next[e.list[0] == d[s] ? 0 : 1];
     }
   }
 
   void remove(int i) {
-    --count_[items_[i].mask];
+    const Node &e = node_[i];
+    --count_[e.mask];
     for (int s = 0; s < 3; ++s) {
-      const int l = list(items_[i], s);
+      const int l = e.list[s];
       if (l < 0) continue;
-      const Link k = link_[3 * (size_t)i + s];
-      if (k.prev == kEnd) head_[l] = k.next;
-      else next(k.prev, l) = k.next;
-      if (k.next != kEnd) back(k.next, l) = k.prev;
+      if (e.prev[s] == kEnd) head_[l] = e.next[s];
+      else node_[e.prev[s]].next[slot(e.prev[s], l)] = e.next[s];
+      if (e.next[s] != kEnd) node_[e.next[s]].prev[slot(e.next[s], l)] = e.prev[s];
     }
   }
 
  private:
   static constexpr int kRounding = 8;  // the list of the items that round
-  struct Link {
-    int next, prev;
+  // An item's lists: its first digit's, its second digit's, the rounding
+  // items' (-1: none), and its neighbours in each.
+  struct Node {
+    uint32_t mask;
+    int8_t list[3];
+    int next[3], prev[3];
   };
-  // list of an item's link: its first digit's, its second digit's, the rounding items'; -1: none
-  static int list(const RegItem &it, int s) {
-    return s == 0 ? it.d0 : s == 1 ? (it.d1 != it.d0 ? it.d1 : -1) : it.exact ? -1 : kRounding;
-  }
-  size_t slot(int i, int l) const { return 3 * (size_t)i + (l == kRounding ? 2 : items_[i].d0 == l ? 0 : 1); }
-  int &next(int i, int l) { return link_[slot(i, l)].next; }
-  int &back(int i, int l) { return link_[slot(i, l)].prev; }
+  int slot(int i, int l) const { return l == kRounding ? 2 : node_[i].list[0] == l ? 0 : 1; }
 
-  const std::vector<RegItem> &items_;
-  std::vector<Link> link_;
+  std::vector<Node> node_;
   int head_[9];
   int count_[256] = {0};  // pending items by digits
 };
@@ -583,26 +589,79 @@ inline bool plain_op(const dm_op &op) {
   return op.kind == DM_OP_1Q || op.kind == DM_OP_CX || op.kind == DM_OP_CX_SCALED || op.kind == DM_OP_MEMORY_NOISE;
 }
 
+// Thermal feed of a memory noise (f, p, g): what its Z component takes from I.
+inline double noise_feed(const double *v) { return (1 - v[2]) * (2 * v[1] - 1); }
+
+// The kernels that run one operation by itself, in units of a short launch
+// (3-5 us below 12 qubits); a fused pass of a register of up to 6 qubits
+// counts 3.  Memory noise is a diagonal kernel or, with a thermal feed, tile
+// passes, which at 7-9 qubits take two short launches each (7 qubits, one map
+// and one such level: 26 us; two maps 18).
+inline double plain_kernels(int n, const dm_op &op, const double *params) {
+  if (op.kind == DM_OP_FUSED) return 3;
+  if (op.kind != DM_OP_MEMORY_NOISE) return 1;
+  const double *v = params + op.param;
+  if (v[0] == 1.0 && v[2] == 1.0) return 0;
+  if (noise_feed(v) == 0.0) return 1;
+  return n >= 12 ? 1 + (n - 4) / 4 : (1 + (n - 4) / 3) * (n >= 7 && n <= 9 ? 2 : 1);
+}
+
+// The positions of an operation (a fused pass of a register of up to 6 qubits:
+// all), and the fewest blocks of operations on the positions `used`: a block
+// takes the positions 0-2 and four others.
+inline uint32_t plain_positions(int n, const dm_op &op) {
+  if (op.kind == DM_OP_1Q) return 1u << (n - 1 - op.qubits[0]);
+  if (op.kind == DM_OP_CX || op.kind == DM_OP_CX_SCALED)
+    return (1u << (n - 1 - op.qubits[0])) | (1u << (n - 1 - op.qubits[1]));
+  return (1u << n) - 1u;
+}
+inline size_t least_blocks(uint32_t used) { return std::max(1, (__builtin_popcount(used & ~7u) + 3) / 4); }
+
+// What `blocks` passes instead of the run's own kernels cost, in the same
+// units, staging and upload of their image included; the run is fused where
+// its kernels cost more.  FP64, one call, us, kernels against passes:
+// - up to 6 qubits one launch takes the run: six kernels (5 qubits, 4 maps and
+//   4 noise levels 41 against 31; 80 gates in dense blocks with short runs
+//   between them 293, and 302 with every run of two and more as one launch);
+// - 7-9 qubits: kernels of 4.5 us beside passes of 12-14 and 20 of fixed cost
+//   (9 qubits, 4 gates 27 against 34, 8 gates 43 against 35, 4 gates and 4
+//   levels, two passes, 42 against 46, 8 and 8 64 against 48);
+// - 10 and 11 qubits: kernels of 7-13 us (10 qubits, 4 gates 39 against 35, 4
+//   gates and 4 levels 54 against 53);
+// - from 12 qubits on a pass takes 1.0-1.4 times a kernel (12 qubits, two
+//   gates, one pass, 104 against 58; 13 qubits, 4 gates 700 against 226).
+inline double plain_pass_cost(int n, size_t blocks) {
+  return n <= 6 ? 5.5 : n <= 9 ? 3.0 * blocks + 3.0 : n <= 11 ? 2.0 * blocks : 1.4 * blocks;
+}
+
 inline void add_plain(int n, const dm_op &op, const double *params, int src, PlainRun *run) {
   TileOp t;
   memset(&t, 0, sizeof(t));
   const double *pv = params + op.param;
+  run->kernels += plain_kernels(n, op, params);
   if (op.kind == DM_OP_MEMORY_NOISE) {
-    const double f = pv[0], p = pv[1], g = pv[2];
+    const double f = pv[0], g = pv[2];
     if (f == 1.0 && g == 1.0) return;
-    const double od = sqrt(g) * f, dd = (1 - g) * (2 * p - 1);
+    const double od = sqrt(g) * f, dd = noise_feed(pv);
     const double R[12] = {0, od, 0, 0, 0, 0, od, 0, dd, 0, 0, g};
     t.kind = TOP_1Q;
     t.k = 1;
     for (int d = 0; d < n; ++d) {
+      const int p = run->pend[d];
+      if (p >= 0) {  // compose_1q without its products with zero
+        double *e = &run->vals[run->ops[p].param];
+        for (int j = 0; j < 8; ++j) e[j] *= od;
+        for (int j = 8; j < 12; ++j) e[j] *= g;
+        e[8] += dd;
+        ++run->count[p];
+        ++run->total;
+        continue;
+      }
       t.d[0] = d;
       push_plain(t, R, 12, src, run);
     }
-    // a diagonal kernel, or with a thermal feed tile passes
-    run->kernels += dd == 0.0 ? 1 : n >= 12 ? 1 + (n - 4) / 4 : 1 + (n - 4) / 3;
     return;
   }
-  run->kernels += 1;
   t.d[0] = n - 1 - op.qubits[0];
   if (op.kind == DM_OP_1Q) {
     t.kind = TOP_1Q;
@@ -650,8 +709,9 @@ inline std::vector<std::vector<int>> plain_blocks(int n, const PlainRun &run) {
   for (int left = no; left;) {
     best.clear();
     int most = 0;
+    uint32_t grown = 0;  // the positions of the growth without a forced one: with one of them forced it is the same
     for (int force = -1; force < n; ++force) {
-      if (force >= 0 && force < 3) continue;
+      if (force >= 0 && (((low | grown) >> force) & 1)) continue;
       uint32_t T = force < 0 ? 0 : 1u << force, blocked = 0;
       int walk[32], ops = 0;
       memcpy(walk, head, sizeof(walk));
@@ -674,6 +734,7 @@ inline std::vector<std::vector<int>> plain_blocks(int n, const PlainRun &run) {
           walk[p] = at(i, p).next;
         }
       }
+      if (force < 0) grown = T;
       if (ops > most) {
         most = ops;
         best.swap(cur);

@@ -9,7 +9,9 @@ reg_plan.h is plain C++ and is compiled here with g++ into two drivers:
 * programs of 400,000 gates whose last digit is never used, or only by the
   last gate: planning time goes with the length of the program.  A planner
   that looks at what is still pending at every stage needs 1e10 steps and
-  more (over a minute); the limit of 20 s is some 40 times what it takes.
+  more (over a minute); the limit of 20 s is some 40 times what it takes;
+* the choice between one kernel an operation and fused passes, at sizes where
+  both were timed.
 """
 import os
 import shutil
@@ -240,6 +242,51 @@ int main() {
 '''
 
 
+CHOICE = COMMON + r'''
+// Whether a run of `gates` single-qubit and CX gates on the qubits 0-3, each
+// followed by a memory-noise level if noise is not null, becomes passes.
+static bool fuses(int n, int gates, const double *noise) {
+  std::vector<double> prm(kMap, kMap + 12);
+  if (noise) prm.insert(prm.end(), noise, noise + 3);
+  PlainRun run;
+  uint32_t used = 0;
+  for (int i = 0; i < gates; ++i)
+    for (int level = 0; level < (noise ? 2 : 1); ++level) {
+      dm_op op;
+      memset(&op, 0, sizeof(op));
+      op.kind = level ? DM_OP_MEMORY_NOISE : i % 8 < 4 ? DM_OP_1Q : DM_OP_CX;
+      op.param = level ? 12 : 0;
+      op.qubits[0] = i % 4;
+      op.qubits[1] = (i + 1) % 4;
+      add_plain(n, op, prm.data(), i, &run);
+      used |= plain_positions(n, op);
+    }
+  const size_t blocks = n <= 6 ? 1 : plain_blocks(n, run).size();
+  if (least_blocks(used) > blocks) abort();
+  return plain_pass_cost(n, blocks) < run.kernels;
+}
+
+int main() {
+  const double dephasing[3] = {0.998, 1.0, 1.0}, thermal[3] = {0.998, 1.0, 0.999};
+  struct {
+    int n, gates;
+    const double *noise;
+    double kernels, passes;  // us a call, measured
+  } rows[] = {{5, 4, thermal, 63, 33},   {5, 8, nullptr, 41, 33},   {7, 4, nullptr, 24, 32}, {7, 2, dephasing, 23, 32},
+              {7, 1, thermal, 26, 33},   {7, 2, thermal, 39, 33},   {9, 4, nullptr, 27, 34}, {9, 8, nullptr, 43, 35},
+              {9, 4, dephasing, 42, 46}, {9, 8, dephasing, 64, 48}, {10, 4, nullptr, 39, 35}, {11, 4, nullptr, 65, 38},
+              {12, 2, nullptr, 104, 58}, {13, 4, thermal, 3800, 606}};
+  int bad = 0;
+  for (const auto &r : rows)
+    if (fuses(r.n, r.gates, r.noise) != (r.passes < r.kernels)) {
+      printf("%d qubits, %d gates: the slower choice\n", r.n, r.gates);
+      ++bad;
+    }
+  return bad;
+}
+'''
+
+
 def run_driver(tmp_path, source, limit):
     if shutil.which('g++') is None:
         pytest.skip('no g++')
@@ -259,3 +306,7 @@ def test_stages_and_blocks_follow_their_definition(tmp_path):
 
 def test_planning_time_goes_with_the_program(tmp_path):
     assert len(run_driver(tmp_path, LONG, 20).splitlines()) == 12
+
+
+def test_runs_are_fused_where_that_was_measured_faster(tmp_path):
+    run_driver(tmp_path, CHOICE, 20)
