@@ -225,8 +225,8 @@ int dm_mlp_train(float *params, int n_features, int hidden, const float *X, cons
  * Circuits of at most lds_max_qubits (5..7) qubits run whole inside one
  * workgroup: in registers when they hold single-qubit maps, CX and memory
  * noise only (FP64: one launch for up to 6 qubits, one for 7; FP32: 7
- * qubits), else in LDS (one launch per width, lds_threads threads per
- * workgroup).
+ * qubits), else in LDS (one launch up to 6 qubits and one of 7, lds_threads
+ * threads per workgroup).
  * The others keep their state in one HBM arena: each operation becomes a
  * 6-digit tile pass (DM_OP_FUSED with tile size 6, DM_OP_1Q, DM_OP_CX[_SCALED],
  * DM_OP_2Q, DM_OP_MEMORY_NOISE; memory noise as 1-qubit channels, 6 qubits
@@ -239,8 +239,8 @@ int dm_mlp_train(float *params, int n_features, int hidden, const float *X, cons
  * items per pass) is one grid-stride launch, and its passes of 6-digit and of
  * 7-digit records one launch each with a workgroup per tile (a further one
  * for 7-digit tiles that do not hold the three lowest positions).  A run is
- * at most 9 launches of whole circuits plus these per round (the longest circuit's
- * passes + 2 rounds a group); dm_batch_run with use_graph != 0
+ * at most 4 launches of whole circuits plus these per round (the longest
+ * circuit's passes + 2 rounds a group); dm_batch_run with use_graph != 0
  * captures them into one hipGraph on first use and replays it.  Per-circuit
  * times (circuit_us) are GPU clock stamps from a circuit's initialisation to
  * its probabilities; circuits run concurrently.  dm_batch_info reports the

@@ -3698,16 +3698,14 @@ struct dm_batch {
   std::vector<int64_t> prob_off;
   int64_t nprobs = 0;
   std::vector<double> err;
-  // LDS tier: circuits held entirely in one workgroup's LDS, grouped by width
+  // circuits held entirely in one workgroup, in the order: in registers up to 6
+  // qubits and 7 qubits, in LDS up to 6 qubits (of at most lds6_width) and 7
   std::vector<int> small;
-  std::vector<int> small_width_start;  // per width 1..7: first index into small-ordered arrays
-  // in the order: register-resident circuits of up to 6 qubits, of 7 qubits,
-  // then the others by width (small_width_start)
-  int nreg6 = 0, nreg7 = 0;
+  int nreg6 = 0, nreg7 = 0, nlds6 = 0, nlds7 = 0, lds6_width = 0;
   void *d_rcircs = nullptr, *d_rrecs = nullptr, *d_rvals = nullptr;
   void *d_circs = nullptr, *d_tops = nullptr, *d_vals = nullptr;
   int lds_threads = 256;
-  hipStream_t side2 = nullptr;
+  hipStream_t side2 = nullptr;  // (only with circuits of 7 qubits)
   hipEvent_t join2 = nullptr;
   // HBM tier: the states in one arena, the pass table, the items in round
   // order (round r: pass r of every circuit), and the tile operations and
@@ -3941,37 +3939,37 @@ template <typename T>
 int enqueue_batch(dm_batch *b) {
   HIP_TRY(hipEventRecord(b->fork, b->master));
   HIP_TRY(hipStreamWaitEvent(b->side, b->fork, 0));
-  // LDS tier on the side streams: the register-resident circuits, then one
-  // launch per width for the others
-  HIP_TRY(hipStreamWaitEvent(b->side2, b->fork, 0));
+  // whole circuits on the side streams, those of 7 qubits on one of their own:
+  // either kind rarely fills the chip
   constexpr bool SEQ = sizeof(T) == 4;
-  const RegCirc *rc = static_cast<const RegCirc *>(b->d_rcircs);
-  const uint32_t *rrecs = static_cast<const uint32_t *>(b->d_rrecs);
-  const T *rvals = static_cast<const T *>(b->d_rvals);
-  if (b->nreg7) {
-    hipLaunchKernelGGL((k_circuit_reg<T, 7, SEQ>), dim3(b->nreg7), dim3(RegCircShape<7>::threads), 0, b->side2,
-                       rc + b->nreg6, rrecs, rvals, b->d_probs, b->d_stamps + 2 * (size_t)b->nreg6);
-    if (int rc2 = last_launch("k_circuit_reg")) return rc2;
+  if (b->side2) {
+    HIP_TRY(hipStreamWaitEvent(b->side2, b->fork, 0));
+    if (b->nreg7) {
+      hipLaunchKernelGGL((k_circuit_reg<T, 7, SEQ>), dim3(b->nreg7), dim3(RegCircShape<7>::threads), 0, b->side2,
+                         static_cast<const RegCirc *>(b->d_rcircs) + b->nreg6,
+                         static_cast<const uint32_t *>(b->d_rrecs), static_cast<const T *>(b->d_rvals), b->d_probs,
+                         b->d_stamps + 2 * (size_t)b->nreg6);
+      if (int rc = last_launch("k_circuit_reg")) return rc;
+    }
   }
   if constexpr (!SEQ) {
     if (b->nreg6) {
-      hipLaunchKernelGGL((k_circuit_reg<T, 6, SEQ>), dim3(b->nreg6), dim3(RegCircShape<6>::threads), 0, b->side, rc,
-                         rrecs, rvals, b->d_probs, b->d_stamps);
-      if (int rc2 = last_launch("k_circuit_reg")) return rc2;
+      hipLaunchKernelGGL((k_circuit_reg<T, 6, SEQ>), dim3(b->nreg6), dim3(RegCircShape<6>::threads), 0, b->side,
+                         static_cast<const RegCirc *>(b->d_rcircs), static_cast<const uint32_t *>(b->d_rrecs),
+                         static_cast<const T *>(b->d_rvals), b->d_probs, b->d_stamps);
+      if (int rc = last_launch("k_circuit_reg")) return rc;
     }
   }
   const int reg = b->nreg6 + b->nreg7;
-  // the widest first, in turn on the two streams: a width's circuits rarely
-  // fill the chip and run beside the next width's
-  for (int w = 7; w >= 1; --w) {
-    const int lo = b->small_width_start[w], hi = b->small_width_start[w + 1];
-    if (hi <= lo) continue;
-    hipLaunchKernelGGL((k_circuit_lds<T>), dim3(hi - lo), dim3(b->lds_threads), lds_bytes(w, b->dtype),
-                       (w & 1) ? b->side2 : b->side,
-                       static_cast<const BatchCirc *>(b->d_circs) + (lo - reg), static_cast<const TileOp *>(b->d_tops),
-                       static_cast<const T *>(b->d_vals), b->d_probs, b->d_stamps + 2 * (size_t)lo);
-    if (int rc = last_launch("k_circuit_lds")) return rc;
-  }
+  auto in_lds = [&](int first, int count, int width, hipStream_t st) -> int {
+    if (!count) return DM_OK;
+    hipLaunchKernelGGL((k_circuit_lds<T>), dim3(count), dim3(b->lds_threads), lds_bytes(width, b->dtype), st,
+                       static_cast<const BatchCirc *>(b->d_circs) + first, static_cast<const TileOp *>(b->d_tops),
+                       static_cast<const T *>(b->d_vals), b->d_probs, b->d_stamps + 2 * (size_t)(reg + first));
+    return last_launch("k_circuit_lds");
+  };
+  if (int rc = in_lds(0, b->nlds6, b->lds6_width, b->side)) return rc;
+  if (int rc = in_lds(b->nlds6, b->nlds7, 7, b->side2)) return rc;
   // HBM tier: the rounds in order on the master stream.  A round's INIT /
   // PROBS items (master), 6-digit tile items (side6) and 7-digit tile items
   // (side7, FP32) belong to distinct circuits: the three launches run side
@@ -4052,8 +4050,10 @@ int enqueue_batch(dm_batch *b) {
   }
   HIP_TRY(hipEventRecord(b->join, b->side));
   HIP_TRY(hipStreamWaitEvent(b->master, b->join, 0));
-  HIP_TRY(hipEventRecord(b->join2, b->side2));
-  HIP_TRY(hipStreamWaitEvent(b->master, b->join2, 0));
+  if (b->side2) {
+    HIP_TRY(hipEventRecord(b->join2, b->side2));
+    HIP_TRY(hipStreamWaitEvent(b->master, b->join2, 0));
+  }
   return DM_OK;
 }
 
@@ -4092,7 +4092,7 @@ static int batch_create_t(dm_batch *b, const int64_t *op_start, const dm_op *ops
   // the longest first
   std::vector<RegCirc> rcircs;
   std::vector<uint32_t> rrecs;
-  std::vector<double> rvals;
+  std::vector<T> rvals;
   std::vector<char> in_reg(b->ncirc, 0);
   {
     struct Planned {
@@ -4142,12 +4142,15 @@ static int batch_create_t(dm_batch *b, const int64_t *op_start, const dm_op *ops
       }
     b->launches += (b->nreg6 > 0) + (b->nreg7 > 0);
   }
-  b->small_width_start.assign(9, 0);
-  for (int w = 1; w <= 7; ++w) {
-    b->small_width_start[w] = (int)b->small.size();
+  // in LDS: 7 qubits last, the others widest first in one launch (with one a
+  // width, on two streams in turn, a graph of small circuits took 280 us more
+  // to set up)
+  for (int w : {6, 5, 4, 3, 2, 1, 7}) {
     if (w > lds_max_qubits) continue;
     for (int c = 0; c < b->ncirc; ++c) {
       if (b->nq[c] != w || in_reg[c]) continue;
+      ++(w == 7 ? b->nlds7 : b->nlds6);
+      if (w < 7) b->lds6_width = std::max(b->lds6_width, w);
       BatchCirc bc;
       bc.n = w;
       bc.op_off = (int64_t)tops.size();
@@ -4161,14 +4164,13 @@ static int batch_create_t(dm_batch *b, const int64_t *op_start, const dm_op *ops
       b->small.push_back(c);
     }
   }
-  b->small_width_start[8] = (int)b->small.size();
-  for (int w = 1; w <= 7; ++w) b->launches += b->small_width_start[w + 1] > b->small_width_start[w] ? 1 : 0;
+  b->launches += (b->nlds6 > 0) + (b->nlds7 > 0);
 
   // HBM tier: every circuit as INIT, its tile passes, PROBS; states in one arena
   std::vector<BatchPass> passes;
   std::vector<TileOp> qtops;
   std::vector<uint32_t> recs;           // register-resident passes
-  std::vector<double> qvals;
+  std::vector<T> qvals;
   std::vector<std::vector<int>> chain;  // pass-table indices of each HBM circuit, in order
   std::vector<double> work;             // per HBM circuit: bytes moved (ticket order)
   uint64_t arena = 0, tiles = 0;
@@ -4319,8 +4321,10 @@ static int batch_create_t(dm_batch *b, const int64_t *op_start, const dm_op *ops
   HIP_TRY(hipStreamCreateWithFlags(&b->side, hipStreamNonBlocking));
   HIP_TRY(hipEventCreateWithFlags(&b->fork, hipEventDisableTiming));
   HIP_TRY(hipEventCreateWithFlags(&b->join, hipEventDisableTiming));
-  HIP_TRY(hipStreamCreateWithFlags(&b->side2, hipStreamNonBlocking));
-  HIP_TRY(hipEventCreateWithFlags(&b->join2, hipEventDisableTiming));
+  if (b->nreg7 || b->nlds7) {
+    HIP_TRY(hipStreamCreateWithFlags(&b->side2, hipStreamNonBlocking));
+    HIP_TRY(hipEventCreateWithFlags(&b->join2, hipEventDisableTiming));
+  }
   HIP_TRY(hipStreamCreateWithFlags(&b->side6, hipStreamNonBlocking));
   HIP_TRY(hipStreamCreateWithFlags(&b->side7, hipStreamNonBlocking));
   HIP_TRY(hipEventCreateWithFlags(&b->forkr, hipEventDisableTiming));
@@ -4334,10 +4338,9 @@ static int batch_create_t(dm_batch *b, const int64_t *op_start, const dm_op *ops
     return DM_OK;
   };
   if (!rcircs.empty()) {
-    std::vector<T> tv(rvals.begin(), rvals.end());
     if (int rc = upload(&b->d_rcircs, rcircs.data(), rcircs.size() * sizeof(RegCirc))) return rc;
     if (int rc = upload(&b->d_rrecs, rrecs.data(), rrecs.size() * 4)) return rc;
-    if (int rc = upload(&b->d_rvals, tv.data(), tv.size() * sizeof(T))) return rc;
+    if (int rc = upload(&b->d_rvals, rvals.data(), rvals.size() * sizeof(T))) return rc;
   }
   if (!circs.empty()) {
     std::vector<T> tv(vals.begin(), vals.end());
@@ -4350,12 +4353,11 @@ static int batch_create_t(dm_batch *b, const int64_t *op_start, const dm_op *ops
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)need));
   }
   if (b->nitems) {
-    std::vector<T> tv(qvals.begin(), qvals.end());
     HIP_TRY(hipMalloc(&b->d_arena, arena * sizeof(T)));
     if (int rc = upload(&b->d_passes, passes.data(), passes.size() * sizeof(BatchPass))) return rc;
     if (int rc = upload(&b->d_items, items.data(), items.size() * sizeof(BatchItem))) return rc;
     if (int rc = upload(&b->d_qtops, qtops.data(), qtops.size() * sizeof(TileOp))) return rc;
-    if (int rc = upload(&b->d_qvals, tv.data(), tv.size() * sizeof(T))) return rc;
+    if (int rc = upload(&b->d_qvals, qvals.data(), qvals.size() * sizeof(T))) return rc;
     if (int rc = upload(&b->d_recs, recs.data(), recs.size() * 4)) return rc;
     int per_cu = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_batch_round<T>, kQueueThreads, 0) != hipSuccess ||

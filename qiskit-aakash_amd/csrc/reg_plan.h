@@ -269,26 +269,8 @@ class RegQueue {
   // for bit those of the given order) only if one of them rounds nothing: an
   // item that rounds joins only as the first pending one of those.
   int absorb(const int (&d)[3], bool ordered, std::vector<int> *take) const {
-    uint32_t blocked = 0;
-    const uint32_t triple = (1u << d[0]) | (1u << d[1]) | (1u << d[2]);
-    int at[3] = {head_[d[0]], head_[d[1]], head_[d[2]]}, rounding = head_[kRounding], n = 0;
-    for (;;) {
-      const int i = std::min(at[0], std::min(at[1], at[2]));
-      if (i == kEnd) return n;
-      const Node &e = node_[i];
-      const bool rounds = e.list[2] >= 0;
-      if ((e.mask & (blocked | ~triple)) || (ordered && rounds && i != rounding)) {
-        blocked |= e.mask;
-        for (int s = 0; s < 3; ++s)
-          if ((e.mask >> d[s]) & 1) at[s] = kEnd;
-        continue;
-      }
-      ++n;
-      if (take) take->push_back(i);
-      if (ordered && rounds) rounding = e.next[2];
-      for (int s = 0; s < 3; ++s)
-        if (at[s] == i) at[s] = e.next[e.list[0] == d[s] ? 0 : 1];
-    }
+    return take ? (ordered ? walk<true, true>(d, take) : walk<false, true>(d, take))
+                : (ordered ? walk<true, false>(d, take) : walk<false, false>(d, take));
   }
 
   void remove(int i) {
@@ -304,6 +286,33 @@ class RegQueue {
   }
 
  private:
+  template <bool ORDERED, bool TAKE>
+  int walk(const int (&d)[3], std::vector<int> *take) const {
+    const uint32_t triple = (1u << d[0]) | (1u << d[1]) | (1u << d[2]);
+    int a = head_[d[0]], b = head_[d[1]], c = head_[d[2]], n = 0;  // next item of each digit, kEnd: blocked or none
+    int rounding = ORDERED ? head_[kRounding] : 0;
+    uint32_t outside = ~triple;  // and the digits of items left out
+    for (;;) {
+      const int i = std::min(a, std::min(b, c));
+      if (i == kEnd) return n;
+      const Node &e = node_[i];
+      const bool rounds = ORDERED && e.list[2] >= 0;
+      if ((e.mask & outside) || (rounds && i != rounding)) {
+        outside |= e.mask;
+        if (a == i) a = kEnd;
+        if (b == i) b = kEnd;
+        if (c == i) c = kEnd;
+        continue;
+      }
+      ++n;
+      if (TAKE) take->push_back(i);
+      if (rounds) rounding = e.next[2];
+      if (a == i) a = e.next[e.list[0] == d[0] ? 0 : 1];
+      if (b == i) b = e.next[e.list[0] == d[1] ? 0 : 1];
+      if (c == i) c = e.next[e.list[0] == d[2] ? 0 : 1];
+    }
+  }
+
   static constexpr int kRounding = 8;  // the list of the items that round
   // An item's lists: its first digit's, its second digit's, the rounding
   // items' (-1: none), and its neighbours in each.
@@ -356,7 +365,9 @@ inline void reg_plan(const std::vector<RegItem> &items, int m, bool io, bool ord
       for (int c = b + 1; c < m; ++c) add(a, b, c);
   RegQueue queue(items);
   std::vector<uint32_t> stage;
-  std::vector<std::vector<int>> members;
+  std::vector<int> order;     // items in the order in which the stages take them
+  std::vector<size_t> taken;  // end of each stage's items in `order`
+  order.reserve(items.size());
   size_t left = items.size();
   while (left || stage.empty()) {
     const bool load = io && stage.empty();
@@ -373,13 +384,12 @@ inline void reg_plan(const std::vector<RegItem> &items, int m, bool io, bool ord
         best = t;
       }
     }
-    std::vector<int> take;
-    take.reserve(most);
-    queue.absorb(digits[best], ordered, &take);
-    for (int i : take) queue.remove(i);
-    left -= take.size();
+    const size_t from = order.size();
+    queue.absorb(digits[best], ordered, &order);
+    for (size_t x = from; x < order.size(); ++x) queue.remove(order[x]);
+    left -= order.size() - from;
     stage.push_back(triples[best]);
-    members.push_back(std::move(take));
+    taken.push_back(order.size());
   }
   if (io && (stage.back() & 7u)) {  // an empty stage that stores directly
     const uint32_t last = stage.back();
@@ -390,11 +400,11 @@ inline void reg_plan(const std::vector<RegItem> &items, int m, bool io, bool ord
         best = t;
     if (best == nio) {  // digits 0-2 in registers: one stage in between
       stage.push_back((1u << 2) | (1u << 3) | (1u << 4));
-      members.emplace_back();
+      taken.push_back(order.size());
       best = 0;  // digits 3, 4, 5
     }
     stage.push_back(triples[best]);
-    members.emplace_back();
+    taken.push_back(order.size());
   }
   const int ns = (int)stage.size();
   std::vector<RegLay> lay(ns);
@@ -459,15 +469,18 @@ inline void reg_plan(const std::vector<RegItem> &items, int m, bool io, bool ord
   out->last = lay[ns - 1];
   out->ns = ns;
   out->words.clear();
+  out->words.reserve(ns * (sizeof(RegStage) / 4) + items.size() + 1);
   out->vals.clear();
+  out->vals.reserve((items.size() + 1) * kRegVals);
   std::vector<uint32_t> kinds;
+  kinds.reserve(items.size() + 1);
   for (int k = 0; k < ns; ++k) {
     RegStage sg;
     memset(&sg, 0, sizeof(sg));
     sg.mem = (uint32_t)kinds.size();
     auto slot = [&](int d) { return lay[k].r[0] == d ? 0 : lay[k].r[1] == d ? 1 : 2; };
-    for (size_t x = 0; x < members[k].size(); ++x) {
-      const RegItem &it = items[members[k][x]];
+    for (size_t x = k ? taken[k - 1] : 0; x < taken[k]; ++x) {
+      const RegItem &it = items[order[x]];
       double v[kRegVals] = {0.0};
       uint32_t kind;
       if (it.kind == 0) {
@@ -483,8 +496,8 @@ inline void reg_plan(const std::vector<RegItem> &items, int m, bool io, bool ord
         const int lo = std::min(s0, s1), hi = std::max(s0, s1);
         const int pair = lo == 0 ? hi - 1 : 2;  // (0,1) (0,2) (1,2)
         const RegItem *scale = nullptr;  // the scale of this CX, if it comes next
-        if (it.kind == 1 && x + 1 < members[k].size()) {
-          scale = &items[members[k][x + 1]];
+        if (it.kind == 1 && x + 1 < taken[k]) {
+          scale = &items[order[x + 1]];
           if (scale->kind != 2 || scale->d0 != it.d0 || scale->d1 != it.d1) scale = nullptr;
         }
         if (scale) {

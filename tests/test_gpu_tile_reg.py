@@ -362,3 +362,26 @@ def test_program_images_of_every_size_and_in_turn(precision):
             a = st.download()
             st.close()
     assert np.array_equal(got, a)
+
+
+@pytest.mark.parametrize('precision', ['fp64', 'fp32'])
+def test_whole_circuits_in_lds_of_all_widths(precision):
+    """Circuits of 1-6 qubits that keep the LDS kernel (FP32; in FP64 those
+    with a two-qubit map) are one launch, those of 7 another (in FP32 the
+    register-resident one), each circuit as in a batch of its own."""
+    from dmsim import batch
+    rng = np.random.default_rng(5)
+    circuits = []
+    for n in (3, 1, 6, 7, 2, 5, 7, 4, 6):
+        prog, _ = small_circuit(rng, n, 12, (0.98, 0.8, 0.995))
+        if precision == 'fp64' and n > 1:
+            prog.two_qubit(0, 1, np.eye(16))
+        circuits.append((n, prog, 0.97))
+    b = batch.Batch(circuits, precision, lds_max_qubits=7, lds_threads=256)
+    assert b.info()['launches'] == (2 if precision == 'fp32' else 3)  # FP64: one qubit stays in registers
+    for graph in (False, True, True):
+        for circuit, got in zip(circuits, b.run(graph)[0]):
+            one = batch.Batch([circuit], precision, lds_max_qubits=7, lds_threads=256)
+            assert np.array_equal(one.run(False)[0][0], got)
+            one.close()
+    b.close()
