@@ -403,6 +403,8 @@ struct Tab4 {
 // consecutive coefficients of a chunk.  Bound by HBM writes.  |0..0>, FP32:
 // 16 qubits 8.4 ms with n multiplications a coefficient, 4.2 ms with chunks
 // of 4^5, 3.2 ms (5.4 TB/s) with 4^6; 13 qubits 148, 74 and 49 us.
+// Up to 10 qubits chunks are of 4^5, as building a larger table takes longer
+// than the few coefficients of a workgroup (8 qubits FP64, 4^6 7.4 us, 4^5 6.1).
 // NT: nontemporal accesses (states above the last-level cache).
 constexpr int kTabDigits = 6;
 
@@ -469,6 +471,30 @@ __global__ __launch_bounds__(kBlock) void k_diag_pow(T *__restrict__ a, uint64_t
       x.v[e] = x.v[e] * (s_h[nxy] * s_g[nz]);
     }
     stp(a + u * W, x);
+  }
+}
+
+// FP64 in place from 12 qubits on: a thread multiplies the n factors of its
+// two coefficients.  Bound by HBM, and the workgroups pass over the state in
+// the order of addresses, which streams better than chunks do (12 / 14 qubits
+// 43 / 702 us against 46 / 730).
+__global__ __launch_bounds__(kBlock) void k_diag_units(double *__restrict__ a, uint64_t units, int n, Tab4 tab,
+                                                       double scale) {
+  using P = Pack<double, 2>;
+  __shared__ double s_tab[kMaxQubits * 4];
+  for (int i = threadIdx.x; i < 4 * n; i += kBlock) s_tab[i] = tab.t[i];
+  __syncthreads();
+  const uint64_t step = (uint64_t)gridDim.x * kBlock;
+  for (uint64_t u = (uint64_t)blockIdx.x * kBlock + threadIdx.x; u < units; u += step) {
+    P x = ldp<P>(a + u * 2);
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const uint64_t i = u * 2 + e;
+      double f = scale;
+      for (int p = 0; p < n; ++p) f *= s_tab[4 * p + ((i >> (2 * p)) & 3)];
+      x.v[e] = x.v[e] * f;
+    }
+    stp(a + u * 2, x);
   }
 }
 
@@ -2321,7 +2347,13 @@ int launch_diag_tab(dm_state *h, const double *tab_by_pos, bool write_only, doub
   memset(&tab, 0, sizeof(tab));
   memcpy(tab.t, tab_by_pos, sizeof(double) * 4 * h->n);
   ProfScope ps(h, write_only ? 7 : 4);
-  const int low = std::min(h->n, kTabDigits);
+  if (sizeof(T) == 8 && !write_only && h->n >= 12) {
+    const uint64_t units = h->N / 2;
+    hipLaunchKernelGGL(k_diag_units, dim3(grid_for(h, units)), dim3(kBlock), 0, h->stream,
+                       static_cast<double *>(h->d_a), units, h->n, tab, scale);
+    return last_launch("k_diag_units");
+  }
+  const int low = std::min(h->n, h->n <= 10 ? kTabDigits - 1 : kTabDigits);
   const uint64_t chunks = h->N >> (2 * low);
   // several chunks a workgroup, so that the LDS table is a small part of it
   const dim3 grid((unsigned)std::min<uint64_t>(chunks, 8192));

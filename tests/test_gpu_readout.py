@@ -99,3 +99,11 @@ def test_sums(n, pa, pb):
     assert abs(c['dot'] - np.dot(a, b)) <= tol * np.sqrt(aa * bb)
     assert abs(c['norm2_self'] - aa) <= tol * aa and abs(c['norm2_other'] - bb) <= tol * bb
     assert abs(purity - aa * 2.0 ** n) <= tol * aa * 2.0 ** n and tr == a[0] * 2.0 ** n
+
+
+@pytest.mark.parametrize('precision', ['fp64', 'fp32'])
+@pytest.mark.parametrize('n', [10, 11, 12, 13])
+def test_product_states_and_diagonals_where_the_tables_change(n, precision):
+    """Tables of 4^5 coefficients up to 10 qubits, of 4^6 above, and FP64
+    diagonals without one from 12 (tolerances as above)."""
+    test_product_states_and_diagonals(n, precision)
