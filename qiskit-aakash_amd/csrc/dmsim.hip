@@ -1352,37 +1352,46 @@ __device__ __forceinline__ double block_sum(double v) {
   return t;
 }
 
-// Four consecutive coefficients as FP64 (16-byte loads).
-template <typename T>
-__device__ __forceinline__ void load4(const T *p, double (&x)[4]) {
-  const Pack<T, 4> q = ldq<T, true>(p);
+// W consecutive coefficients as FP64, streamed (nontemporal).
+template <int W, typename T>
+__device__ __forceinline__ void load_sum(const T *p, double (&x)[W]) {
+  constexpr int H = W * sizeof(T) > 16 ? 16 / sizeof(T) : W;
+  using V = T __attribute__((ext_vector_type(H)));
 #pragma unroll
-  for (int e = 0; e < 4; ++e) x[e] = (double)q.v[e];
+  for (int h = 0; h < W / H; ++h) {
+    const V v = __builtin_nontemporal_load(reinterpret_cast<const V *>(p + h * H));
+#pragma unroll
+    for (int e = 0; e < H; ++e) x[h * H + e] = (double)v[e];
+  }
 }
 
-// Sums over N coefficients, N a multiple of 4: each thread takes quads with
-// the stride of the grid, two in flight.  Bound by HBM (15 qubits, FP32: one
-// coefficient per load 1.15 ms, 3.7 TB/s; quads 0.70 ms).
+// Sums over N coefficients, N a multiple of 4: each thread takes packs of 16
+// bytes with the stride of the grid, two in flight.  Bound by HBM (14 qubits:
+// FP32, one coefficient per load 282 us, packs 170; FP64 355 and 311, with 32
+// bytes a thread 370; more than 1024 workgroups are slower).
+constexpr int kSumGrid = 1024;
+
 template <typename T>
-__global__ __launch_bounds__(kBlock) void k_sumsq(const T *__restrict__ a, uint64_t quads, double *part) {
+__global__ __launch_bounds__(kBlock) void k_sumsq(const T *__restrict__ a, uint64_t packs, double *part) {
+  constexpr int W = 16 / sizeof(T);
   double s0 = 0.0, s1 = 0.0;
   const uint64_t step = (uint64_t)gridDim.x * kBlock;
   uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
-  for (; i + step < quads; i += 2 * step) {
-    double x[4], y[4];
-    load4(a + 4 * i, x);
-    load4(a + 4 * (i + step), y);
+  for (; i + step < packs; i += 2 * step) {
+    double x[W], y[W];
+    load_sum<W>(a + W * i, x);
+    load_sum<W>(a + W * (i + step), y);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
+    for (int e = 0; e < W; ++e) {
       s0 += x[e] * x[e];
       s1 += y[e] * y[e];
     }
   }
-  if (i < quads) {
-    double x[4];
-    load4(a + 4 * i, x);
+  if (i < packs) {
+    double x[W];
+    load_sum<W>(a + W * i, x);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) s0 += x[e] * x[e];
+    for (int e = 0; e < W; ++e) s0 += x[e] * x[e];
   }
   const double s = block_sum(s0 + s1);
   if (threadIdx.x == 0) part[blockIdx.x] = s;
@@ -1399,18 +1408,28 @@ __global__ __launch_bounds__(kBlock) void k_dot(const T *__restrict__ a, const T
   if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
-// per block: max |a-b|, sum a*b, sum a*a, sum b*b (columns of gridDim.x)
+// per block: max |a-b|, sum a*b, sum a*a, sum b*b (columns of gridDim.x).
+// Coefficients per load: four, in FP64 against FP64 one (14 qubits: 594 us with
+// one and 2048 workgroups, 638 with two and 1024, 734 with four and 4096;
+// FP32 against FP32 341 with four, 535 with one).
 template <typename TA, typename TB>
-__global__ __launch_bounds__(kBlock) void k_diff(const TA *__restrict__ a, const TB *__restrict__ b, uint64_t quads,
+struct DiffShape {
+  static constexpr bool both64 = sizeof(TA) + sizeof(TB) == 16;
+  static constexpr int width = both64 ? 1 : 4, grid = both64 ? 2 * kSumGrid : kSumGrid;
+};
+
+template <typename TA, typename TB>
+__global__ __launch_bounds__(kBlock) void k_diff(const TA *__restrict__ a, const TB *__restrict__ b, uint64_t packs,
                                                  double *part) {
+  constexpr int W = DiffShape<TA, TB>::width;
   double mx = 0.0, ab = 0.0, aa = 0.0, bb = 0.0;
   const uint64_t step = (uint64_t)gridDim.x * kBlock;
-  for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < quads; i += step) {
-    double x[4], y[4];
-    load4(a + 4 * i, x);
-    load4(b + 4 * i, y);
+  for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < packs; i += step) {
+    double x[W], y[W];
+    load_sum<W>(a + W * i, x);
+    load_sum<W>(b + W * i, y);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
+    for (int e = 0; e < W; ++e) {
       mx = fmax(mx, fabs(x[e] - y[e]));
       ab += x[e] * y[e];
       aa += x[e] * x[e];
@@ -2451,12 +2470,12 @@ int reserve_red(dm_state *h, size_t doubles) {
 
 template <typename T>
 int do_sumsq(dm_state *h, double *out) {
-  const uint64_t quads = h->N / 4;
-  const int grid = std::min(grid_for(h, quads), 4096);
+  const uint64_t packs = h->N / (16 / sizeof(T));
+  const int grid = std::min(grid_for(h, packs), kSumGrid);
   int rc = reserve_red(h, (size_t)grid + 8);
   if (rc) return rc;
   ProfScope ps(h, 6);
-  hipLaunchKernelGGL((k_sumsq<T>), dim3(grid), dim3(kBlock), 0, h->stream, static_cast<const T *>(h->d_a), quads,
+  hipLaunchKernelGGL((k_sumsq<T>), dim3(grid), dim3(kBlock), 0, h->stream, static_cast<const T *>(h->d_a), packs,
                      h->d_red);
   hipLaunchKernelGGL(k_sum_parts, dim3(1), dim3(kBlock), 0, h->stream, h->d_red, grid, h->d_red + grid);
   rc = last_launch("k_sumsq");
@@ -4406,19 +4425,37 @@ static int batch_create_t(dm_batch *b, const int64_t *op_start, const dm_op *ops
   return DM_OK;
 }
 
+constexpr int kHostParts = 256;  // (FP64, 8 qubits: 25 us against 27)
+
 template <typename TA, typename TB>
 static int diff_t(dm_state *a, dm_state *b, double *out4) {
-  const uint64_t quads = a->N / 4;
-  const int grid = std::min(grid_for(a, quads), 4096);
+  using Shape = DiffShape<TA, TB>;
+  const uint64_t packs = a->N / Shape::width;
+  const int grid = std::min(grid_for(a, packs), Shape::grid);
   if (int rc = reserve_red(a, 4 * (size_t)grid + 8)) return rc;
   HIP_TRY(hipStreamSynchronize(b->stream));
   hipLaunchKernelGGL((k_diff<TA, TB>), dim3(grid), dim3(kBlock), 0, a->stream, static_cast<const TA *>(a->d_a),
-                     static_cast<const TB *>(b->d_a), quads, a->d_red);
-  double *res = a->d_red + 4 * (size_t)grid;
-  hipLaunchKernelGGL(k_diff_parts, dim3(4), dim3(kBlock), 0, a->stream, a->d_red, grid, res);
+                     static_cast<const TB *>(b->d_a), packs, a->d_red);
+  if (grid > kHostParts) {
+    double *res = a->d_red + 4 * (size_t)grid;
+    hipLaunchKernelGGL(k_diff_parts, dim3(4), dim3(kBlock), 0, a->stream, a->d_red, grid, res);
+    if (int rc = last_launch("k_diff")) return rc;
+    HIP_TRY(hipMemcpyAsync(out4, res, 4 * sizeof(double), hipMemcpyDeviceToHost, a->stream));
+    HIP_TRY(hipStreamSynchronize(a->stream));
+    return DM_OK;
+  }
+  // few partials: their sums are cheaper here than by a second launch
   if (int rc = last_launch("k_diff")) return rc;
-  HIP_TRY(hipMemcpyAsync(out4, res, 4 * sizeof(double), hipMemcpyDeviceToHost, a->stream));
+  double part[4 * kHostParts];
+  HIP_TRY(hipMemcpyAsync(part, a->d_red, 4 * (size_t)grid * sizeof(double), hipMemcpyDeviceToHost, a->stream));
   HIP_TRY(hipStreamSynchronize(a->stream));
+  for (int c = 0; c < 4; ++c) {
+    out4[c] = 0.0;
+    for (int i = 0; i < grid; ++i) {
+      const double p = part[c * grid + i];
+      out4[c] = c ? out4[c] + p : std::max(out4[c], p);
+    }
+  }
   return DM_OK;
 }
 

@@ -101,6 +101,15 @@ def test_sums(n, pa, pb):
     assert abs(purity - aa * 2.0 ** n) <= tol * aa * 2.0 ** n and tr == a[0] * 2.0 ** n
 
 
+@pytest.mark.parametrize('n,pa,pb', [(n, pa, pb) for n in (8, 9, 10) for pa in ('fp64', 'fp32') for pb in ('fp64', 'fp32')]
+                         + [(12, 'fp64', 'fp64'), (12, 'fp32', 'fp64')])
+def test_sums_where_the_partials_move_to_the_device(n, pa, pb):
+    """Up to 256 workgroups (8 qubits FP64 against FP64, 9 otherwise) the host
+    adds their partials, above a kernel; 12 qubits: more packs than the
+    workgroups take at once."""
+    test_sums(n, pa, pb)
+
+
 @pytest.mark.parametrize('precision', ['fp64', 'fp32'])
 @pytest.mark.parametrize('n', [10, 11, 12, 13])
 def test_product_states_and_diagonals_where_the_tables_change(n, precision):
