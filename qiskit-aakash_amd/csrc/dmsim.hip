@@ -854,6 +854,28 @@ __device__ __forceinline__ void member_cx(T (&v)[NG][4][4], const T *__restrict_
   for (int g = 0; g < NG; ++g) cx_map<T, T, LO, true>(v[g], sv);
 }
 
+// 16x16 PTM member, pair index 4 i_d0 + i_d1 (first row the identity's),
+// digit d0 a (lo) or b.
+template <typename T, int NG>
+__device__ __forceinline__ void member_2q(T (&v)[NG][4][4], const T *__restrict__ pv, bool lo) {
+#pragma unroll
+  for (int g = 0; g < NG; ++g) {
+    T w[16];
+#pragma unroll
+    for (int r = 1; r < 16; ++r) {
+      T acc = T(0);
+#pragma unroll
+      for (int c = 0; c < 16; ++c) acc = fmad(pv[16 * r + c], lo ? v[g][c >> 2][c & 3] : v[g][c & 3][c >> 2], acc);
+      w[r] = acc;
+    }
+#pragma unroll
+    for (int r = 1; r < 16; ++r) {
+      if (lo) v[g][r >> 2][r & 3] = w[r];
+      else v[g][r & 3][r >> 2] = w[r];
+    }
+  }
+}
+
 // The member operations of a stage on NG groups of 16 coefficients in
 // registers: v[g][x][y], x the component index along stage digit a (the
 // lower one), y along the other digit.
@@ -873,24 +895,13 @@ __device__ __forceinline__ void stage_apply(T (&v)[NG][4][4], int a, const TileO
     } else if (!GEN2Q || m.kind == TOP_CX) {
       if (lo) member_cx<T, NG, true>(v, pv);
       else member_cx<T, NG, false>(v, pv);
+    } else if (NG > 1) {
+      // (7-digit FP32 tiles; with one group the selects are faster than a
+      // second copy of the code and its scalar registers)
+      if (lo) member_2q<T, NG>(v, pv, true);
+      else member_2q<T, NG>(v, pv, false);
     } else {
-      // 16x16 PTM, pair index 4 i_d0 + i_d1 (first row the identity's)
-#pragma unroll
-      for (int g = 0; g < NG; ++g) {
-        T w[16];
-#pragma unroll
-        for (int r = 1; r < 16; ++r) {
-          T acc = T(0);
-#pragma unroll
-          for (int c = 0; c < 16; ++c) acc = fmad(pv[16 * r + c], lo ? v[g][c >> 2][c & 3] : v[g][c & 3][c >> 2], acc);
-          w[r] = acc;
-        }
-#pragma unroll
-        for (int r = 1; r < 16; ++r) {
-          if (lo) v[g][r >> 2][r & 3] = w[r];
-          else v[g][r & 3][r >> 2] = w[r];
-        }
-      }
+      member_2q<T, NG>(v, pv, lo);
     }
   }
 }
