@@ -3020,6 +3020,39 @@ std::vector<FusedPass> fuse_plain_run(const dm_state *h, const PlainRun &run, co
   return out;
 }
 
+// Geometry of a tile: the positions in it, its digits and the others.
+void tile_geometry(int n, int m, const bool *intile, FusedPass *fp, int *digit_of_pos) {
+  memset(&fp->geo, 0, sizeof(fp->geo));
+  fp->m = m;
+  fp->geo.m = m;
+  int j = 0;
+  for (int pos = 0; pos < n; ++pos)
+    if (intile[pos]) {
+      digit_of_pos[pos] = j;
+      fp->geo.tpos[j++] = pos;
+    } else {
+      fp->geo.rpos[fp->geo.nr++] = pos;
+    }
+  int w = 0;
+  while (w < m && fp->geo.tpos[w] == w) ++w;
+  fp->geo.w = w;
+  fp->geo.tiles = 1ull << (2 * fp->geo.nr);
+}
+
+// The lowest position outside joins the tile.
+void widen_tile(int n, FusedPass *fp) {
+  bool intile[kMaxQubits] = {false};
+  int pos[8], digit_of_pos[kMaxQubits];
+  for (int j = 0; j < fp->m; ++j) intile[pos[j] = fp->geo.tpos[j]] = true;
+  int low = 0;
+  while (intile[low]) ++low;
+  intile[low] = true;
+  tile_geometry(n, fp->m + 1, intile, fp, digit_of_pos);
+  for (TileOp &op : fp->ops)
+    for (int x = 0; x < (op.kind == TOP_1Q ? 1 : op.kind == TOP_DENSE ? op.k : 2); ++x)
+      op.d[x] = digit_of_pos[pos[op.d[x]]];
+}
+
 // With `run`, a record of single-qubit and CX operations joins it instead and
 // leaves *fp without operations.
 int parse_fused(const dm_state *h, const double *p, int64_t avail, int opi, FusedPass *fp, bool allow_reg = false,
@@ -3057,22 +3090,8 @@ int parse_fused(const dm_state *h, const double *p, int64_t avail, int opi, Fuse
       ++count;
     }
   if (!intile[0]) return fail(DM_ERR_ARG, "op %d: fused tile must hold the last qubit's position", opi);
-  memset(&fp->geo, 0, sizeof(fp->geo));
-  fp->m = m;
-  fp->geo.m = m;
   int digit_of_pos[kMaxQubits];
-  int j = 0;
-  for (int pos = 0; pos < h->n; ++pos)
-    if (intile[pos]) {
-      digit_of_pos[pos] = j;
-      fp->geo.tpos[j++] = pos;
-    } else {
-      fp->geo.rpos[fp->geo.nr++] = pos;
-    }
-  int w = 0;
-  while (w < m && fp->geo.tpos[w] == w) ++w;
-  fp->geo.w = w;
-  fp->geo.tiles = 1ull << (2 * fp->geo.nr);
+  tile_geometry(h->n, m, intile, fp, digit_of_pos);
   int nsub = 0;
   if (!next_int(&nsub) || nsub < 0) return fail(DM_ERR_ARG, "op %d: bad fused op count", opi);
   for (int i = 0; i < nsub; ++i) {
@@ -3130,6 +3149,19 @@ int parse_fused(const dm_state *h, const double *p, int64_t avail, int opi, Fuse
     return DM_OK;
   }
   if (allow_reg && plan_reg(h, fp)) return DM_OK;
+  // Tiles of short runs on states above the last-level cache: the workgroups
+  // of a small tile are so many, and ask HBM for so short pieces at once, that
+  // a larger tile is faster whatever its operations need.  Two passes each:
+  // 14 qubits FP64, 5 / 6 digits 5.8 / 2.5 ms; 16 qubits FP32, runs of 4^2 in
+  // 6 digits / 4^3 in 7 digits 19-21 / 13 ms.  (The matrix-core operations
+  // take 6 digits.)
+  if (fp->m == 5 && h->n >= 13) widen_tile(h->n, fp);
+  if (h->dtype == DM_FP32 && fp->m == 6 && h->n >= 14 && fp->geo.w < 3) {
+    bool dense = false;
+    for (const TileOp &op : fp->ops) dense = dense || op.kind == TOP_DENSE;
+    if (!dense) widen_tile(h->n, fp);
+  }
+  m = fp->m;
   // LDS layout.  The 64 banks (4 bytes each) are LDS index bits 0-5, tile
   // digits 0-2.  Stages on digits 3 and up, and stages on digit 0 and a
   // digit >= 3 (one quad access per component), fall on distinct banks in
@@ -3306,7 +3338,10 @@ int launch_fused(dm_state *h, const FusedPass &fp, const uint32_t *d_recs, const
   //  - otherwise (runs of 4^2, whose neighbouring tiles share HBM lines, or
   //    one resident workgroup per CU): persistent workgroups that prefetch
   //    their next tile, 8 (resp. 4) per resident slot, with consecutive
-  //    tiles kept on one XCD.
+  //    tiles kept on one XCD.  FP32 6-digit tiles at 13 qubits (256 MB) keep
+  //    to four workgroups a CU, where their registers allow five: four
+  //    16x16 maps 427 us a pair of passes with four, 453 with five (12
+  //    qubits, inside the cache, 4 % the other way).
   // FP32 tiles over runs of >= 4^3 load and store nontemporally (FP64
   // passes measured 1.3x slower with the hint).
   // Measured and rejected for FP32 7-digit tiles over runs of 4^3: the
@@ -3332,10 +3367,13 @@ int launch_fused(dm_state *h, const FusedPass &fp, const uint32_t *d_recs, const
       }                                                                                                          \
     }                                                                                                            \
     const bool full = long_runs && per_cu >= 2;                                                                  \
-    const uint64_t slots = (uint64_t)h->cu_count * per_cu * (per_cu >= 2 ? 8 : 4);                              \
+    /* FP32 6-digit tiles of short runs at 13 qubits: four workgroups a CU, held by 33 KB of LDS each */       \
+    const bool four = !full && sizeof(T) == 4 && MM == 6 && h->n >= 13 && per_cu > 4;                            \
+    const size_t pad = four ? (33 << 10) - (sizeof(T) << (2 * MM)) : 0;                                          \
+    const uint64_t slots = (uint64_t)h->cu_count * (four ? 4 : per_cu) * (per_cu >= 2 ? 8 : 4);                 \
     uint64_t g = full ? fp.geo.tiles : std::min<uint64_t>(fp.geo.tiles, slots);                                 \
     if (!full && g >= 8) g -= g % 8;                                                                             \
-    hipLaunchKernelGGL((k_tile_prog<T, MM, D, G, NTH, L>), dim3((unsigned)g), dim3(NTH), 0, h->stream, a,       \
+    hipLaunchKernelGGL((k_tile_prog<T, MM, D, G, NTH, L>), dim3((unsigned)g), dim3(NTH), pad, h->stream, a,     \
                        fp.geo, d_ops, nops, d_vals, (full ? 0 : 1) | (sizeof(T) == 4 && fp.geo.w >= 3 ? 2 : 0)); \
   } while (0)
 #define TILE_LAUNCH(MM, D, G, NTH)               \

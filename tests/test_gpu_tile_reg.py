@@ -385,3 +385,42 @@ def test_whole_circuits_in_lds_of_all_widths(precision):
             assert np.array_equal(one.run(False)[0][0], got)
             one.close()
     b.close()
+
+
+@pytest.mark.parametrize('n,m,qubits,precision', [
+    (13, 5, [0, 2, 3], 'fp64'), (13, 5, [0, 1, 2, 3], 'fp32'), (13, 5, [9, 12], 'fp64'), (13, 6, [1, 3, 5, 7], 'fp32'),
+    (14, 5, [0, 1, 2, 3], 'fp32'), (14, 6, [0, 1, 2, 3], 'fp32'), (14, 6, [4, 6, 7, 12], 'fp32'),
+    (14, 6, [3, 4, 5, 6], 'fp64'), (14, 5, [2, 13], 'fp64')])
+def test_small_tiles_of_large_states(n, m, qubits, precision):
+    """Passes whose tile is widened (5 digits from 13 qubits, FP32 6 digits of
+    short runs from 14) or kept to four workgroups a CU, with two-qubit maps,
+    against one kernel an operation.  Tolerance as above on either side."""
+    rng = np.random.default_rng(n + m)
+    vecs = np.concatenate([np.ones((n, 1)), rng.uniform(-0.5, 0.5, (n, 3))], axis=1)
+    fused, plain = native.DeviceState(n, precision), native.DeviceState(n, precision)
+    for st in (fused, plain):
+        st.init_product(vecs.reshape(-1), 2.0 ** -n)
+    sub, members = [], 9
+    for i in range(members):
+        c, t = (int(x) for x in rng.choice(qubits, 2, replace=False))
+        if i % 3 == 0:
+            R = random_map(rng, 'general')
+            sub.append((native.SUB_1Q, [c], ptm.rows3(R)))
+            plain.apply_1q(c, ptm.rows3(R))
+        elif i % 3 == 1:
+            s = random_scale(rng, 'general')
+            sub.append((native.SUB_CX, [c, t], s))
+            plain.apply_cx(c, t, s)
+        else:
+            R = ptm.cx_ptm((0.97, 0.02)) @ np.kron(random_map(rng, 'general'), random_map(rng, 'unital'))
+            sub.append((native.SUB_2Q, [c, t], R))
+            plain.apply_2q(c, t, R)
+    prog = Program(n)
+    prog.fused(m, qubits, sub)
+    prog.run(fused)
+    r = fused.compare(plain)
+    fused.close()
+    plain.close()
+    # a sum of at most 16 products a two-qubit member
+    assert r['max_abs_diff'] <= 2 * members * 32 * EPS[precision] * 2.0 ** -n
+    assert r['norm2_self'] > 0
