@@ -116,3 +116,29 @@ def test_product_states_and_diagonals_where_the_tables_change(n, precision):
     """Tables of 4^5 coefficients up to 10 qubits, of 4^6 above, and FP64
     diagonals without one from 12 (tolerances as above)."""
     test_product_states_and_diagonals(n, precision)
+
+
+@pytest.mark.parametrize('n,precision', [(14, 'fp64'), (15, 'fp32'), (16, 'fp32')])
+def test_probabilities_of_13_to_16_qubits(n, precision):
+    """More than 12 two-component digits: 1-4 leading ones are contracted in
+    registers.  A product state's probabilities are products of (1 +- err
+    b_q) / 2, b_q another one for each qubit, so that a wrong digit order or
+    column shows.  A coefficient has n + 1 factors, rounded to the storage
+    type, and a sum of 2^m of them at most prod (1 + err |b_q|) 2^-m."""
+    rng = np.random.default_rng(n)
+    eps = EPS if precision == 'fp64' else 2.0 ** -24
+    vecs = np.concatenate([np.ones((n, 1)), rng.uniform(0.1, 0.9, (n, 3)) * rng.choice([-1, 1], (n, 3))], axis=1)
+    st = native.DeviceState(n, precision)
+    st.init_product(vecs.reshape(-1), 2.0 ** -n)
+    for m in range(13, n + 1):
+        for basis, comp in (('X', 1), ('Z', 3)):
+            qubits = sorted(int(q) for q in rng.choice(n, m, replace=False))
+            want, top = np.ones(1), 1.0
+            for q in qubits:
+                b = 0.93 * vecs[q, comp]
+                want = np.kron(want, [(1 + b) / 2, (1 - b) / 2])
+                top *= (1 + abs(b)) / 2
+            got = st.probabilities(qubits, basis, 0.93)
+            assert got.shape == want.shape
+            assert np.abs(got - want).max() <= ((n + 2) * eps + 6 * m * EPS) * top, (m, basis)
+    st.close()

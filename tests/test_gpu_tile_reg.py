@@ -424,3 +424,102 @@ def test_small_tiles_of_large_states(n, m, qubits, precision):
     # a sum of at most 16 products a two-qubit member
     assert r['max_abs_diff'] <= 2 * members * 32 * EPS[precision] * 2.0 ** -n
     assert r['norm2_self'] > 0
+
+
+def random_members(rng, qubits, count):
+    sub = []
+    for _ in range(count):
+        if rng.random() < 0.4:
+            R = random_map(rng, rng.choice(['unital', 'general', 'diag']))
+            sub.append((native.SUB_1Q, [int(rng.choice(qubits))], ptm.rows3(R)))
+        else:
+            c, t = (int(x) for x in rng.choice(qubits, 2, replace=False))
+            sub.append((native.SUB_CX, [c, t], random_scale(rng, rng.choice(['none', 'separable', 'general']))))
+    return sub
+
+
+# FP32 passes in registers are those from 12 qubits (13: 256 MB, the largest
+# state with plain accesses; 14: nontemporal, passes of 12 members and more),
+# FP64 ones above the last-level cache from 13
+@pytest.mark.parametrize('n,precision', [(12, 'fp32'), (13, 'fp32'), (14, 'fp32'), (13, 'fp64'), (14, 'fp64')])
+def test_cx_passes_of_large_states_against_the_lds_form(n, precision):
+    """Passes of maps, CX and scales on low, high and scattered digits, each
+    state against the one that an identity two-qubit map in every pass keeps
+    in LDS: FP32 bit for bit, FP64 to 8 eps a member and side."""
+    rng = np.random.default_rng(60 + n)
+    vecs = np.concatenate([np.ones((n, 1)), rng.uniform(-0.9, 0.9, (n, 3))], axis=1)
+    reg, lds = Program(n), Program(n)
+    members = 0
+    for qubits in ([0, 1, 2, 3], [n - 4, n - 3, n - 2, n - 1], [0, 4, n - 5, n - 1], [n - 7, n - 6, n - 5, n - 4]):
+        sub = random_members(rng, qubits, 40)
+        members += len(sub)
+        reg.fused(7, qubits, sub)
+        lds.fused(7, qubits, with_identity(sub, qubits))
+    a, b = native.DeviceState(n, precision), native.DeviceState(n, precision)
+    for st, prog in ((a, reg), (b, lds)):
+        st.init_product(vecs.reshape(-1), 2.0 ** -n)
+        prog.run(st)
+    r = a.compare(b)
+    a.close()
+    b.close()
+    assert r['norm2_self'] > 4.0 ** -n
+    assert r['max_abs_diff'] <= (0.0 if precision == 'fp32' else 2 * members * 8 * EPS['fp64'] * 2.0 ** -n)
+
+
+def test_fp32_batch_passes_in_registers_equal_the_lds_form():
+    """Batches of as many tiles as CUs take the register form at every width
+    (8-10 qubits here), a state of that size by itself keeps the LDS form: the
+    same coefficients, so that the probabilities differ by FP64 roundings
+    only (an FP32 one would be 1e-10)."""
+    from dmsim import batch
+    rng = np.random.default_rng(9)
+    circuits = []
+    for n in (8, 9, 10, 10, 10, 10, 10):
+        prog = Program(n)
+        for _ in range(5):
+            qubits = sorted(int(q) for q in rng.choice(n, 4, replace=False))
+            prog.fused(6, qubits, random_members(rng, qubits, 16))
+        circuits.append((n, prog, 0.97))
+    b = batch.Batch(circuits, 'fp32', lds_max_qubits=6, lds_threads=256)
+    got = b.run(False)[0]
+    b.close()
+    for (n, prog, err), probs in zip(circuits, got):
+        st = native.DeviceState(n, 'fp32')
+        st.init_product(np.tile([1.0, 0.0, 0.0, 1.0], n), 2.0 ** -n)
+        prog.run(st)
+        assert np.abs(probs - st.probabilities(list(range(n)), 'Z', err)).max() <= 3 * n * 2.0 ** -53
+        st.close()
+
+
+@pytest.mark.parametrize('n', [13, 14])
+@pytest.mark.parametrize('noise', [None, (0.98, 0.8, 0.995)])
+def test_fp64_runs_of_single_operations_above_the_last_level_cache(n, noise):
+    """A program's run of single operations (fused passes, nontemporal, tiles
+    handed to the XCDs in runs) against one call an operation.  Tolerance as
+    for the smaller runs, on either side."""
+    rng = np.random.default_rng(80 + n)
+    vecs = np.concatenate([np.ones((n, 1)), rng.uniform(-0.5, 0.5, (n, 3))], axis=1)
+    run, single = native.DeviceState(n, 'fp64'), native.DeviceState(n, 'fp64')
+    for st in (run, single):
+        st.init_product(vecs.reshape(-1), 2.0 ** -n)
+    prog = Program(n)
+    ops = 24
+    for i in range(ops):
+        if i % 2 == 0:
+            q, R = int(rng.integers(n)), random_map(rng, 'general')
+            prog.one_qubit(q, R)
+            single.apply_1q(q, ptm.rows3(R))
+        else:
+            c, t = (int(x) for x in rng.choice(n, 2, replace=False))
+            s = random_scale(rng, rng.choice(['none', 'separable', 'general']))
+            prog.cx(c, t, s)
+            single.apply_cx(c, t, s)
+        if noise is not None and i % 8 == 7:
+            prog.memory_noise(*noise)
+            single.memory_noise(*noise)
+    prog.run(run)
+    r = run.compare(single)
+    run.close()
+    single.close()
+    assert r['norm2_self'] > 4.0 ** -n
+    assert r['max_abs_diff'] <= 2 * (ops + 3 * n) * 8 * EPS['fp64'] * 2.0 ** -n
