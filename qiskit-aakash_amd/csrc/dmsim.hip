@@ -2952,10 +2952,14 @@ bool plan_reg(const dm_state *h, FusedPass *fp) {
   }
   for (TileOp &op : ops)
     for (int x = 0; x < (op.kind == TOP_CX ? 2 : 1); ++x) op.d[x] = t.digit[fp->geo.tpos[op.d[x]]];
-  const std::vector<RegItem> reg_ops = ordered ? reg_items_in_order(ops, vals) : reg_items(ops, vals, kRegTile);
-  if (light && reg_ops.size() < 12) return false;
   RegPlan rp;
-  reg_plan(reg_ops, kRegTile, true, ordered, &rp);
+  if (ordered) {
+    const std::vector<RegItem<double>> items = reg_items_in_order(ops, vals);
+    if (light && items.size() < 12) return false;
+    reg_plan(items, kRegTile, true, true, &rp);
+  } else {
+    reg_plan(reg_items(ops, vals, kRegTile), kRegTile, true, false, &rp);
+  }
   if (few && ops.size() < 4 * (size_t)rp.ns) return false;
   set_reg(fp, std::move(rp), t);
   return true;
@@ -3536,6 +3540,7 @@ int stage_program(dm_state *h, const dm_op *ops, int nops, const double *params,
         if (!fp.ops.empty()) break;
         if (run.total > before) run.kernels += plain_kernels(h->n, ops[e], params);
       }
+      settle_all(h->n, &run);
       std::vector<FusedPass> fps = fuse_plain_run<T>(h, run, ops);
       dm_op synth;
       memset(&synth, 0, sizeof(synth));
@@ -3952,8 +3957,8 @@ int small_circuit_plan(int n, const dm_op *ops, int nops, const double *params, 
     }
   }
   const int m = n == 7 ? 7 : 6;
-  const bool ordered = sizeof(T) == 4;
-  reg_plan(ordered ? reg_items_in_order(flat, vals) : reg_items(flat, vals, m), m, false, ordered, rp);
+  if (sizeof(T) == 4) reg_plan(reg_items_in_order(flat, vals), m, false, true, rp);
+  else reg_plan(reg_items(flat, vals, m), m, false, false, rp);
   *fits = true;
   return DM_OK;
 }

@@ -10,6 +10,7 @@ reg_plan.h is plain C++ and is compiled here with g++ into two drivers:
   last gate: planning time goes with the length of the program.  A planner
   that looks at what is still pending at every stage needs 1e10 steps and
   more (over a minute); the limit of 20 s is some 40 times what it takes;
+* maps composed on the host are rounded once, against 113 bits;
 * the choice between one kernel an operation and fused passes, at sizes where
   both were timed.
 """
@@ -36,7 +37,8 @@ static const double kMap[12] = {0, .6, .8, 0, 0, -.8, .6, 0, .1, 0, 0, .9};
 '''
 
 DEFINITION = COMMON + r'''
-static std::vector<int> takes(const std::vector<RegItem> &items, const std::vector<char> &done, uint32_t triple,
+template <typename V>
+static std::vector<int> takes(const std::vector<RegItem<V>> &items, const std::vector<char> &done, uint32_t triple,
                               bool ordered) {
   std::vector<int> out;
   uint32_t blocked = 0;
@@ -52,6 +54,41 @@ static std::vector<int> takes(const std::vector<RegItem> &items, const std::vect
     }
   }
   return out;
+}
+
+// Stages on random digits until every item is taken.
+template <typename V>
+static int walk(const std::vector<RegItem<V>> &items, int m, bool ordered) {
+  int bad = 0;
+  std::vector<char> done(items.size(), 0);
+  RegQueue queue(items);
+  size_t left = items.size();
+  for (int step = 0; left && step < 10000; ++step) {
+    int d[3] = {uni(0, m - 1), 0, 0};
+    do d[1] = uni(0, m - 1);
+    while (d[1] == d[0]);
+    do d[2] = uni(0, m - 1);
+    while (d[2] == d[0] || d[2] == d[1]);
+    std::sort(d, d + 3);
+    const uint32_t triple = (1u << d[0]) | (1u << d[1]) | (1u << d[2]);
+    std::vector<int> got;
+    const int n = queue.absorb(d, ordered, &got);
+    const std::vector<int> want = takes(items, done, triple, ordered);
+    int inside = 0, first = -1;
+    for (size_t i = 0; i < items.size(); ++i)
+      if (!done[i]) {
+        inside += (items[i].mask & ~triple) == 0;
+        if (first < 0) first = (int)i;
+      }
+    if (got != want || n != (int)want.size() || queue.inside(d) != inside || queue.first_mask() != items[first].mask)
+      ++bad;
+    for (int i : want) {
+      done[i] = 1;
+      queue.remove(i);
+    }
+    left -= want.size();
+  }
+  return bad + (left != 0);
 }
 
 static int stages() {
@@ -78,37 +115,7 @@ static int stages() {
       }
       ops.push_back(op);
     }
-    const std::vector<RegItem> items = ordered ? reg_items_in_order(ops, vals) : reg_items(ops, vals, m);
-    std::vector<char> done(items.size(), 0);
-    RegQueue queue(items);
-    size_t left = items.size();
-    for (int step = 0; left && step < 10000; ++step) {
-      int d[3] = {uni(0, m - 1), 0, 0};
-      do d[1] = uni(0, m - 1);
-      while (d[1] == d[0]);
-      do d[2] = uni(0, m - 1);
-      while (d[2] == d[0] || d[2] == d[1]);
-      std::sort(d, d + 3);
-      const uint32_t triple = (1u << d[0]) | (1u << d[1]) | (1u << d[2]);
-      std::vector<int> got;
-      const int n = queue.absorb(d, ordered, &got);
-      const std::vector<int> want = takes(items, done, triple, ordered);
-      int inside = 0, first = -1;
-      for (size_t i = 0; i < items.size(); ++i)
-        if (!done[i]) {
-          inside += (items[i].mask & ~triple) == 0;
-          if (first < 0) first = (int)i;
-        }
-      if (got != want || n != (int)want.size() || queue.inside(d) != inside ||
-          queue.first_mask() != items[first].mask)
-        ++bad;
-      for (int i : want) {
-        done[i] = 1;
-        queue.remove(i);
-      }
-      left -= want.size();
-    }
-    if (left) ++bad;
+    bad += ordered ? walk(reg_items_in_order(ops, vals), m, true) : walk(reg_items(ops, vals, m), m, false);
   }
   return bad;
 }
@@ -172,6 +179,7 @@ static int blocks() {
       add_plain(n, op, prm.data(), i, &run);
       total += op.kind == DM_OP_MEMORY_NOISE ? n : 1;
     }
+    settle_all(n, &run);
     int counted = 0;
     for (int c : run.count) counted += c;
     if (counted != total || run.total != total) ++bad;
@@ -219,7 +227,8 @@ int main() {
         long_program(gates, 0, m - 2, late ? m - 1 : -1, &ops, &vals);
         const auto t0 = std::chrono::steady_clock::now();
         RegPlan rp;
-        reg_plan(ordered ? reg_items_in_order(ops, vals) : reg_items(ops, vals, m), m, false, ordered, &rp);
+        if (ordered) reg_plan(reg_items_in_order(ops, vals), m, false, true, &rp);
+        else reg_plan(reg_items(ops, vals, m), m, false, false, &rp);
         printf("digits %d late %d ordered %d: %.2f s, %d stages\n", m, late, ordered,
                std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count(), rp.ns);
         fflush(stdout);
@@ -261,6 +270,7 @@ static bool fuses(int n, int gates, const double *noise) {
       add_plain(n, op, prm.data(), i, &run);
       used |= plain_positions(n, op);
     }
+  settle_all(n, &run);
   const size_t blocks = n <= 6 ? 1 : plain_blocks(n, run).size();
   if (least_blocks(used) > blocks) abort();
   return plain_pass_cost(n, blocks) < run.kernels;
@@ -283,6 +293,82 @@ int main() {
       ++bad;
     }
   return bad;
+}
+'''
+
+
+COMPOSE = COMMON + r'''
+// Composed maps are rounded once: every value of a run of single-qubit maps
+// and noise levels on one position, and of the item made of it, against the
+// product in 113 bits.
+typedef __float128 Q;
+
+int main() {
+  int bad = 0;
+  double worst = 0.0;
+  for (int trial = 0; trial < 300; ++trial) {
+    const int n = 7, q = 3, nops = uni(2, 120);
+    Q e[12] = {0, 1, 0, 0, 0, 0, 1, 0, 0, 0, 0, 1};
+    PlainRun run;
+    std::vector<TileOp> ops;
+    std::vector<double> vals;
+    for (int i = 0; i < nops; ++i) {
+      double R[12] = {0};
+      dm_op op;
+      memset(&op, 0, sizeof(op));
+      std::vector<double> prm;
+      if (uni(0, 2)) {
+        op.kind = DM_OP_MEMORY_NOISE;
+        const double g = 0.9 + 0.099 * uni(0, 1000) / 1000.0, f = 0.9 + 0.0001 * uni(0, 1000), p = 0.001 * uni(0, 1000);
+        prm = {f, p, g};
+        R[1] = R[6] = sqrt(g) * f;
+        R[8] = (1 - g) * (2 * p - 1);
+        R[11] = g;
+      } else {
+        op.kind = DM_OP_1Q;
+        op.qubits[0] = q;
+        const double a = 0.01 * uni(0, 628), b = 0.01 * uni(0, 628), ca = cos(a), sa = sin(a), cb = cos(b), sb = sin(b);
+        const double U[9] = {ca, -sa * cb, sa * sb, sa, ca * cb, -ca * sb, 0, sb, cb};
+        for (int r = 0; r < 3; ++r)
+          for (int c = 0; c < 3; ++c) R[4 * r + 1 + c] = U[3 * r + c];
+        prm.assign(R, R + 12);
+      }
+      add_plain(n, op, prm.data(), i, &run);
+      TileOp t;
+      memset(&t, 0, sizeof(t));
+      t.kind = TOP_1Q;
+      t.k = 1;
+      t.param = (int32_t)vals.size();
+      ops.push_back(t);
+      vals.insert(vals.end(), R, R + 12);
+      Q w[12];
+      for (int r = 0; r < 3; ++r)
+        for (int c = 0; c < 4; ++c) {
+          w[4 * r + c] = c ? Q(0) : Q(R[4 * r]);
+          for (int k = 0; k < 3; ++k) w[4 * r + c] += Q(R[4 * r + 1 + k]) * e[4 * k + c];
+        }
+      for (int c = 0; c < 12; ++c) e[c] = w[c];
+    }
+    settle_all(n, &run);
+    int at = -1;
+    for (size_t i = 0; i < run.ops.size(); ++i)
+      if (run.ops[i].d[0] == n - 1 - q) at = run.ops[i].param;
+    const std::vector<RegItem<long double>> items = reg_items(ops, vals, 7);
+    if (items.size() != 1) ++bad;
+    for (int c = 0; c < 12 && at >= 0; ++c) {
+      const double v[2] = {(double)run.vals[at + c], (double)items[0].v[c]};
+      // half a unit in the last place, and the 64-bit roundings of the chain
+      const double tol = ldexp(fabs((double)e[c]), -53) + ldexp(4.0 * nops, -64);
+      for (double x : v) {
+        const double err = fabs((double)(Q(x) - e[c]));
+        worst = std::max(worst, err / tol);
+        if (!(err <= tol)) ++bad;
+      }
+    }
+    if (at < 0) ++bad;
+  }
+  printf("%d above, worst %.2f of the bound\n", bad, worst);
+  return bad != 0;
 }
 '''
 
@@ -310,3 +396,7 @@ def test_planning_time_goes_with_the_program(tmp_path):
 
 def test_runs_are_fused_where_that_was_measured_faster(tmp_path):
     run_driver(tmp_path, CHOICE, 20)
+
+
+def test_composed_maps_are_rounded_once(tmp_path):
+    run_driver(tmp_path, COMPOSE, 20)
