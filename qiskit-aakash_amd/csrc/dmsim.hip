@@ -3810,8 +3810,6 @@ struct dm_batch {
   void *d_rcircs = nullptr, *d_rrecs = nullptr, *d_rvals = nullptr;
   void *d_circs = nullptr, *d_tops = nullptr, *d_vals = nullptr;
   int lds_threads = 256;
-  hipStream_t side2 = nullptr;  // (only with circuits of 7 qubits)
-  hipEvent_t join2 = nullptr;
   // HBM tier: the states in one arena, the pass table, the items in round
   // order (round r: pass r of every circuit), and the tile operations and
   // values of every pass
@@ -3940,25 +3938,33 @@ int small_circuit_plan(int n, const dm_op *ops, int nops, const double *params, 
   std::vector<TileOp> tops;
   std::vector<double> vals;
   if (int rc = small_circuit_ops(n, ops, nops, params, nparams, ci, &tops, &vals)) return rc;
-  std::vector<TileOp> flat;
-  flat.reserve(tops.size() * 2);
-  for (const TileOp &op : tops) {
+  for (const TileOp &op : tops)
     if (op.kind == TOP_2Q) return DM_OK;
-    if (op.kind != TOP_ALLQ) {
-      flat.push_back(op);
-      continue;
+  const int m = n == 7 ? 7 : 6;
+  if (sizeof(T) == 8) {
+    PlainRun run;
+    for (const TileOp &op : tops) {
+      const double *v = vals.data() + op.param;
+      if (op.kind == TOP_ALLQ) run.levels.push_back({v[1], v[11], v[8], 0});
+      else push_plain(op, v, op.kind == TOP_1Q ? 12 : op.k ? 16 : 0, 0, &run);
     }
-    for (int d = 0; d < n; ++d) {
+    settle_all(n, &run);
+    reg_plan(reg_items(run.ops, run.vals, m), m, false, false, rp);
+  } else {
+    std::vector<TileOp> flat;
+    flat.reserve(tops.size() * (n + 1) / 2);
+    for (const TileOp &op : tops) {
+      if (op.kind != TOP_ALLQ) {
+        flat.push_back(op);
+        continue;
+      }
       TileOp one = op;
       one.kind = TOP_1Q;
       one.k = 1;
-      one.d[0] = d;
-      flat.push_back(one);
+      for (one.d[0] = 0; one.d[0] < n; ++one.d[0]) flat.push_back(one);
     }
+    reg_plan(reg_items_in_order(flat, vals), m, false, true, rp);
   }
-  const int m = n == 7 ? 7 : 6;
-  if (sizeof(T) == 4) reg_plan(reg_items_in_order(flat, vals), m, false, true, rp);
-  else reg_plan(reg_items(flat, vals, m), m, false, false, rp);
   *fits = true;
   return DM_OK;
 }
@@ -4044,18 +4050,16 @@ template <typename T>
 int enqueue_batch(dm_batch *b) {
   HIP_TRY(hipEventRecord(b->fork, b->master));
   HIP_TRY(hipStreamWaitEvent(b->side, b->fork, 0));
-  // whole circuits on the side streams, those of 7 qubits on one of their own:
-  // either kind rarely fills the chip
+  // whole circuits on the side stream; without an HBM tier those of 7 qubits
+  // beside them on the master stream, as either kind rarely fills the chip (a
+  // stream of their own costs a batch 0.8 ms when it is destroyed)
   constexpr bool SEQ = sizeof(T) == 4;
-  if (b->side2) {
-    HIP_TRY(hipStreamWaitEvent(b->side2, b->fork, 0));
-    if (b->nreg7) {
-      hipLaunchKernelGGL((k_circuit_reg<T, 7, SEQ>), dim3(b->nreg7), dim3(RegCircShape<7>::threads), 0, b->side2,
-                         static_cast<const RegCirc *>(b->d_rcircs) + b->nreg6,
-                         static_cast<const uint32_t *>(b->d_rrecs), static_cast<const T *>(b->d_rvals), b->d_probs,
-                         b->d_stamps + 2 * (size_t)b->nreg6);
-      if (int rc = last_launch("k_circuit_reg")) return rc;
-    }
+  hipStream_t side7 = b->nitems ? b->side : b->master;
+  if (b->nreg7) {
+    hipLaunchKernelGGL((k_circuit_reg<T, 7, SEQ>), dim3(b->nreg7), dim3(RegCircShape<7>::threads), 0, side7,
+                       static_cast<const RegCirc *>(b->d_rcircs) + b->nreg6, static_cast<const uint32_t *>(b->d_rrecs),
+                       static_cast<const T *>(b->d_rvals), b->d_probs, b->d_stamps + 2 * (size_t)b->nreg6);
+    if (int rc = last_launch("k_circuit_reg")) return rc;
   }
   if constexpr (!SEQ) {
     if (b->nreg6) {
@@ -4074,7 +4078,7 @@ int enqueue_batch(dm_batch *b) {
     return last_launch("k_circuit_lds");
   };
   if (int rc = in_lds(0, b->nlds6, b->lds6_width, b->side)) return rc;
-  if (int rc = in_lds(b->nlds6, b->nlds7, 7, b->side2)) return rc;
+  if (int rc = in_lds(b->nlds6, b->nlds7, 7, side7)) return rc;
   // HBM tier: the rounds in order on the master stream.  A round's INIT /
   // PROBS items (master), 6-digit tile items (side6) and 7-digit tile items
   // (side7, FP32) belong to distinct circuits: the three launches run side
@@ -4155,10 +4159,6 @@ int enqueue_batch(dm_batch *b) {
   }
   HIP_TRY(hipEventRecord(b->join, b->side));
   HIP_TRY(hipStreamWaitEvent(b->master, b->join, 0));
-  if (b->side2) {
-    HIP_TRY(hipEventRecord(b->join2, b->side2));
-    HIP_TRY(hipStreamWaitEvent(b->master, b->join2, 0));
-  }
   return DM_OK;
 }
 
@@ -4426,10 +4426,6 @@ static int batch_create_t(dm_batch *b, const int64_t *op_start, const dm_op *ops
   HIP_TRY(hipStreamCreateWithFlags(&b->side, hipStreamNonBlocking));
   HIP_TRY(hipEventCreateWithFlags(&b->fork, hipEventDisableTiming));
   HIP_TRY(hipEventCreateWithFlags(&b->join, hipEventDisableTiming));
-  if (b->nreg7 || b->nlds7) {
-    HIP_TRY(hipStreamCreateWithFlags(&b->side2, hipStreamNonBlocking));
-    HIP_TRY(hipEventCreateWithFlags(&b->join2, hipEventDisableTiming));
-  }
   HIP_TRY(hipStreamCreateWithFlags(&b->side6, hipStreamNonBlocking));
   HIP_TRY(hipStreamCreateWithFlags(&b->side7, hipStreamNonBlocking));
   HIP_TRY(hipEventCreateWithFlags(&b->forkr, hipEventDisableTiming));
@@ -4854,7 +4850,6 @@ int dm_batch_destroy(dm_batch *b) {
   if (!b) return DM_OK;
   if (b->master) hipStreamSynchronize(b->master);
   if (b->side) hipStreamSynchronize(b->side);
-  if (b->side2) hipStreamSynchronize(b->side2);
   if (b->side6) hipStreamSynchronize(b->side6);
   if (b->side7) hipStreamSynchronize(b->side7);
   if (b->exec) hipGraphExecDestroy(b->exec);
@@ -4862,9 +4857,9 @@ int dm_batch_destroy(dm_batch *b) {
   for (void *p : {b->d_circs, b->d_tops, b->d_vals, b->d_arena, b->d_passes, b->d_items, b->d_qtops, b->d_qvals, b->d_recs,
                   b->d_rcircs, b->d_rrecs, b->d_rvals, (void *)b->d_probs, (void *)b->d_stamps})
     if (p) hipFree(p);
-  for (hipEvent_t e : {b->fork, b->join, b->join2, b->ev0, b->ev1, b->forkr, b->join6, b->join7})
+  for (hipEvent_t e : {b->fork, b->join, b->ev0, b->ev1, b->forkr, b->join6, b->join7})
     if (e) hipEventDestroy(e);
-  for (hipStream_t st : {b->side, b->side2, b->side6, b->side7, b->master})
+  for (hipStream_t st : {b->side, b->side6, b->side7, b->master})
     if (st) hipStreamDestroy(st);
   delete b;
   return DM_OK;

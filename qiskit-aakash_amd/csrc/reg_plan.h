@@ -146,27 +146,29 @@ template <typename S>
 inline std::vector<RegItem<long double>> reg_items(const std::vector<TileOp> &ops, const std::vector<S> &vals, int m) {
   using Item = RegItem<long double>;
   std::vector<Item> out;
-  out.reserve(2 * ops.size());
+  out.reserve(ops.size());
   int pend[8];  // item index of the single-qubit map a digit's next one joins, or -1
   for (int d = 0; d < m; ++d) pend[d] = -1;
+  bool scales = false;
   for (const TileOp &op : ops) {
     const S *v = vals.data() + op.param;
     if (op.kind == TOP_1Q) {
       const int d = op.d[0];
       if (pend[d] < 0) {
-        Item it;
+        pend[d] = (int)out.size();
+        out.emplace_back();
+        Item &it = out.back();
         it.mask = 1u << d;
         it.kind = 0;
         it.scaled = it.exact = false;
         it.d0 = it.d1 = d;
         std::copy(v, v + 12, it.v);
-        pend[d] = (int)out.size();
-        out.push_back(it);
       } else {
         compose_1q(v, out[pend[d]].v);
       }
     } else {
-      Item it;
+      out.emplace_back();
+      Item &it = out.back();
       it.d0 = op.d[0];
       it.d1 = op.d[1];
       it.mask = (1u << it.d0) | (1u << it.d1);
@@ -174,10 +176,11 @@ inline std::vector<RegItem<long double>> reg_items(const std::vector<TileOp> &op
       it.scaled = op.k != 0;
       it.exact = false;
       if (op.k) std::copy(v, v + 16, it.v);
-      out.push_back(it);
+      scales = scales || it.scaled;
       pend[it.d0] = pend[it.d1] = -1;
     }
   }
+  if (!scales) return out;
   // scales
   std::vector<Item> res;
   res.reserve(out.size() + 8);
