@@ -1947,8 +1947,8 @@ __device__ __forceinline__ void queue_tiles(T *s, T *a, const BatchPass &bp, uin
 // per item of one tile, without the round kernel's loops, so the registers
 // are those of the one-tile kernel (in the grid-stride round kernel the tile
 // code sat at the 106-SGPR limit and the 7-digit form spilled to scratch).
-// Waves per SIMD: 4 in FP32 and 2 in FP64, the register-resident form's; the
-// 6-digit LDS form is left for registers of 6 qubits and dense two-qubit
+// Waves per SIMD: at least 4 in FP32 and 2 in FP64 (87 and 154 VGPRs with the
+// register-resident form: 5 and 3); the 6-digit LDS form is left for registers of 6 qubits and dense two-qubit
 // maps, the 7-digit one (two 64 KB workgroups of 8 waves per CU) for tiles
 // that do not hold the three lowest positions.
 template <typename T, int M>
@@ -3929,7 +3929,10 @@ int small_circuit_ops(int n, const dm_op *ops, int nops, const double *params, i
 // FP32: every operation on its own and in order, as the LDS kernel rounds; on
 // fewer than 7 qubits that many redistributions cost more than the LDS
 // kernel's passes (49 circuits of 6 qubits and 40-150 gates, memory noise
-// after each: 1109 us against 604; 7 qubits 1454 against 1749).
+// after each: 1109 us against 604; 7 qubits 1454 against 1749).  Planning
+// takes the host 24 us an FP64 circuit of 6 qubits and 95 gates with noise
+// after each (a run of 49: 645 -> 165 us) and 100 us an FP32 one of 7 qubits
+// and 60 gates (200 circuits of 2-7 qubits: 3.5 ms once, a run 2.07 -> 1.05).
 template <typename T>
 int small_circuit_plan(int n, const dm_op *ops, int nops, const double *params, int64_t nparams, int ci, bool *fits,
                        RegPlan *rp) {
@@ -4079,10 +4082,13 @@ int enqueue_batch(dm_batch *b) {
   };
   if (int rc = in_lds(0, b->nlds6, b->lds6_width, b->side)) return rc;
   if (int rc = in_lds(b->nlds6, b->nlds7, 7, side7)) return rc;
-  // HBM tier: the rounds in order on the master stream.  A round's INIT /
-  // PROBS items (master), 6-digit tile items (side6) and 7-digit tile items
-  // (side7, FP32) belong to distinct circuits: the three launches run side
-  // by side, forked from and joined back into master.
+  // HBM tier.  One group: its rounds in order on the master stream; a round's
+  // INIT / PROBS items (master), tile items of 6-digit records (side6) and of
+  // 7-digit ones (side7: the register-resident form, then the LDS form) belong
+  // to distinct circuits, and where a round has more than one of these they
+  // run side by side, forked from and joined back into master.  Several
+  // groups: each one's launches in order on its chain's stream (master, side6,
+  // side7), forked from master once and joined back at the end.
   const BatchPass *passes = static_cast<const BatchPass *>(b->d_passes);
   const BatchItem *items = static_cast<const BatchItem *>(b->d_items);
   const TileOp *tops = static_cast<const TileOp *>(b->d_qtops);

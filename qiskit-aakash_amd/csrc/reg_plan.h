@@ -431,7 +431,7 @@ inline void reg_plan(const std::vector<RegItem<V>> &items, int m, bool io, bool 
       else rest[nrest++] = d;
     }
     // register digits: those kept from the previous stage stay in their
-    // slots, the first such slot orders the phases
+    // slots, the last such slot orders the phases
     for (int j = 0; j < 3; ++j) y.r[j] = -1;
     y.slot = 0;
     if (k) {

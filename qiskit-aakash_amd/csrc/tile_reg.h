@@ -72,7 +72,7 @@ __device__ __forceinline__ void reg_1q(T (&v)[64], const T (&pv)[kRegVals]) {
 
 // In place (v_swap_b32): plain copies would keep a second set of registers
 // alive where the members' code paths join (FP64: 196 VGPRs, two waves per
-// SIMD, against 150 and three: 15 qubits 81.7 -> 76.9 ms, 10 qubits 366 -> 331
+// SIMD, against 154 and three: 15 qubits 81.7 -> 76.9 ms, 10 qubits 366 -> 331
 // us).
 template <typename T>
 __device__ __forceinline__ void reg_swap(T &a, T &b) {
@@ -339,7 +339,6 @@ __global__ __launch_bounds__(kRegThreads, sizeof(T) == 4 ? 5 : 3) void k_tile_re
                                                              const uint32_t *__restrict__ kinds,
                                                              const T *__restrict__ prm) {
   __shared__ __align__(16) T s[RegShape<T>::lds];
-  if (blockIdx.x >= geo.tiles) return;  // uniform over the workgroup
   // Workgroups go to the 8 XCDs in turn.  Streaming from HBM (NTM: at least
   // 4^6 tiles), an XCD takes 64 consecutive tiles, whose low digits run over
   // consecutive addresses, so that its requests fall on fewer DRAM pages:
