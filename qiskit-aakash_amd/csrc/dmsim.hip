@@ -3616,7 +3616,7 @@ int upload_image(dm_state *h, Prepared *pp, void *dev) {
   return DM_OK;
 }
 
-// The same into the handle's own buffer, in stream order from a host copy that
+// The same in stream order, from a host copy that
 // the handle keeps until the upload has ended: nothing waits for the device
 // unless the previous image is still on its way.  Passes walk their records
 // one after another, so what counts is where the image lies afterwards: a
@@ -3631,15 +3631,17 @@ int upload_image(dm_state *h, Prepared *pp, void *dev) {
 //   that runs once more than it saves; then k_image copies them from a pinned
 //   buffer (64 KB: 13.5 us against the engine's 10.5; 1 MB: 37 against 28).
 // - Above, the engine; the first few wait for the stream.
+// `pin` false: no buffer is pinned (images above kKernelImage wait).
 constexpr size_t kSmallImage = 16 << 10, kKernelImage = 256 << 10;
 constexpr int kUnpinnedImages = 3;
 
-int enqueue_image(dm_state *h, Prepared *pp) {
+int enqueue_image(dm_state *h, Prepared *pp, void *dev, bool pin) {
   const size_t bytes = pp->image_bytes();
+  if (bytes == 0) return DM_OK;
   bool pinned = bytes > kSmallImage;
-  if (pinned && h->large_images < kUnpinnedImages) {
-    ++h->large_images;
-    if (bytes > kKernelImage) return upload_image(h, pp, h->d_mat);
+  if (pinned && (!pin || h->large_images < kUnpinnedImages)) {
+    h->large_images += pin;
+    if (bytes > kKernelImage) return upload_image(h, pp, dev);
     pinned = false;
   }
   if (h->img_busy) {
@@ -3655,7 +3657,7 @@ int enqueue_image(dm_state *h, Prepared *pp) {
     if (hipHostMalloc(&h->h_img, cap, hipHostMallocDefault) != hipSuccess) {
       (void)hipGetLastError();
       h->h_img = nullptr;
-      return upload_image(h, pp, h->d_mat);
+      return upload_image(h, pp, dev);
     }
     h->img_cap = cap;
   }
@@ -3666,18 +3668,18 @@ int enqueue_image(dm_state *h, Prepared *pp) {
   if (pinned && bytes <= kKernelImage) {
     const size_t packs = (bytes + 15) / 16;  // (both buffers hold a multiple of 16)
     hipLaunchKernelGGL(k_image, dim3((unsigned)((packs + kBlock - 1) / kBlock)), dim3(kBlock), 0, h->stream,
-                       static_cast<uint4 *>(h->d_mat), reinterpret_cast<const uint4 *>(img), (uint32_t)packs);
+                       static_cast<uint4 *>(dev), reinterpret_cast<const uint4 *>(img), (uint32_t)packs);
     if (int rc = last_launch("k_image")) return rc;
   } else {
     const size_t piece = pinned ? bytes : kSmallImage;
     for (size_t at = 0; at < bytes; at += piece)
-      HIP_TRY(hipMemcpyAsync(static_cast<char *>(h->d_mat) + at, img + at, std::min(piece, bytes - at),
+      HIP_TRY(hipMemcpyAsync(static_cast<char *>(dev) + at, img + at, std::min(piece, bytes - at),
                              hipMemcpyHostToDevice, h->stream));
   }
   HIP_TRY(hipEventRecord(h->img_ev, h->stream));
   h->img_busy = true;
-  pp->d_ops = h->d_mat;
-  pp->d_mat = static_cast<const char *>(h->d_mat) + pp->vals_at;
+  pp->d_ops = dev;
+  pp->d_mat = static_cast<const char *>(dev) + pp->vals_at;
   return DM_OK;
 }
 
@@ -3689,7 +3691,7 @@ int prepare_program(dm_state *h, const dm_op *ops, int nops, const double *param
   const size_t bytes = (pp->image_bytes() + 15) & ~(size_t)15;  // (k_image copies 16 at a time)
   if (h->mat_cap < bytes) HIP_TRY(hipStreamSynchronize(h->stream));  // the old buffer may be in use
   if (int rc = ensure(&h->d_mat, &h->mat_cap, bytes)) return rc;
-  return enqueue_image(h, pp);
+  return enqueue_image(h, pp, h->d_mat, true);
 }
 
 template <typename T>
@@ -3772,8 +3774,8 @@ int scratch_address(int device, void **out) {
 
 // dm_run_program with the program image in the device's fixed scratch array
 // instead of the handle's growable buffer: stage on the host, refuse an
-// image larger than the array, copy it there after the handle's earlier work
-// has finished, enqueue the same kernels.
+// image larger than the array, copy it there behind the handle's earlier work
+// on its stream, enqueue the same kernels.
 template <typename T>
 int run_program_noalloc(dm_state *h, const dm_op *ops, int nops, const double *params, int64_t nparams) {
   Prepared pp;
@@ -3788,7 +3790,7 @@ int run_program_noalloc(dm_state *h, const dm_op *ops, int nops, const double *p
   if (!pp.tops.empty() || !pp.values.empty()) {
     void *dev = nullptr;
     if (int rc = scratch_address(h->device, &dev)) return rc;
-    if (int rc = upload_image(h, &pp, dev)) return rc;
+    if (int rc = enqueue_image(h, &pp, dev, false)) return rc;
   }
   return launch_program<T>(h, pp);
 }

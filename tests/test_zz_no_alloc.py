@@ -93,3 +93,33 @@ def test_noalloc_takes_passes_whose_register_form_exceeds_the_scratch(precision)
     st.init_product(np.array([1.0, 0.0, 0.0, 1.0] * (n - 1) + [1.0, 0.0, 0.0, -1.0]), 0.5 ** n)
     assert np.array_equal(got, st.download())
     st.close()
+
+
+@pytest.mark.parametrize('precision', ['fp64', 'fp32'])
+def test_noalloc_calls_in_a_row_on_one_handle(precision):
+    """Images of 2 KB to above 256 KB one after the other on one handle, which
+    waits for none of them, against dm_run_program: the same bit for bit."""
+    n = 9
+    progs = []
+    for passes, seed in ((2, 3), (30, 4), (900, 5), (1, 6)):
+        rng = np.random.default_rng(seed)
+        prog = Program(n)
+        for _ in range(passes):
+            q = [int(x) for x in rng.choice(n, 2, replace=False)]
+            R = ptm.depolarizing1(0.01) @ ptm.gate_ptm('u3', list(rng.uniform(0, 6, 3)))
+            prog.fused(6, q, [(native.SUB_1Q, q[:1], ptm.rows3(R)), (native.SUB_CX, q, None)])
+        progs.append(prog)
+    lib, out = native.load(), []
+    for entry in ('dm_run_program', 'dm_run_program_noalloc'):
+        st = native.DeviceState(n, precision)
+        st.init_product(np.tile([1.0, 0.3, 0.0, 0.8], n), 0.5 ** n)
+        for _ in range(4):
+            for prog in progs:
+                arr, params = prog.compile()
+                ops = (native.DmOp * len(prog)).from_buffer(arr)
+                rc = getattr(lib, entry)(st.h, ctypes.cast(ops, ctypes.c_void_p), len(prog),
+                                         params.ctypes.data_as(native.c_double_p), int(params.size))
+                native.check(rc, entry)
+        out.append(st.download())
+        st.close()
+    assert np.abs(out[0]).max() > 0 and np.array_equal(out[0], out[1])
